@@ -26,7 +26,7 @@
 //   dW                    dw_mfma_kernel / dw_batch_kernel: fp32 MFMA over the
 //                         batch with the reference's per-element rounding
 //                         (welvet_dense.metal:155-178).
-//   unaligned rows        gemv_generic_kernel / dx_generic_kernel.
+//   unaligned rows        ragged.hip (f64 products on the f64 MFMA / VALU).
 //
 // Accumulation is fp32 inside a lane/tile and f64 across split-K / segment
 // partials; outputs are fl32 of that, within the stated tolerance of the f64
@@ -747,32 +747,6 @@ __global__ void __launch_bounds__(512) gemv_loopb_kernel(GemvArgs a, int batch) 
     group(g, wb, 1);
     if (gn >= ngroups) break;
     g = gn;
-  }
-}
-
-// Element-wise fallback for shapes whose rows do not start on a chunk
-// boundary: a block per output row, f64 accumulation, any batch.
-template <int DT>
-__global__ void __launch_bounds__(256) gemv_generic_kernel(DevStore w, int batch, const float *x,
-                                                           const double *bias, int bias_len, int act,
-                                                           float *pre, float *post) {
-  __shared__ double red[4];
-  const int o = blockIdx.x;
-  for (int b = 0; b < batch; ++b) {
-    double acc = 0;
-    for (int k = threadIdx.x; k < w.cols; k += 256) {
-      const int64_t i = (int64_t)o * w.cols + k;
-      const uint64_t c = load_code<DT>(w.body, i);
-      const double wv = DT == kFloat64 ? u2d(c) : (double)dec_code<DT>(c, w.scale, w.minv);
-      acc += wv * (double)x[(int64_t)b * w.cols + k];
-    }
-    acc = wave_sum(acc);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0)
-      bias_act_store(red[0] + red[1] + red[2] + red[3], o, bias, bias_len, act, pre, post,
-                     (int64_t)b * w.rows + o);
-    __syncthreads();
   }
 }
 
@@ -2455,22 +2429,6 @@ __global__ void __launch_bounds__(256) dx_small_kernel(DxArgs a) {
       a.ws[((int64_t)seg * B + b) * a.cols + (int64_t)c * E + e] = (float)acc[b][e];
 }
 
-template <int DT>
-__global__ void __launch_bounds__(256) dx_generic_kernel(DevStore w, int batch, const float *dpre,
-                                                         float *dX) {
-  const int64_t total = (int64_t)batch * w.cols;
-  for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < total; t += (int64_t)gridDim.x * 256) {
-    const int b = (int)(t / w.cols), i = (int)(t % w.cols);
-    double acc = 0;
-    for (int o = 0; o < w.rows; ++o) {
-      const uint64_t c = load_code<DT>(w.body, (int64_t)o * w.cols + i);
-      const double wv = DT == kFloat64 ? u2d(c) : (double)dec_code<DT>(c, w.scale, w.minv);
-      acc += wv * (double)dpre[(int64_t)b * w.rows + o];
-    }
-    dX[t] = (float)acc;
-  }
-}
-
 // dW on the matrix cores with the reference's rounding.  Per output the
 // reference accumulates acc = fmaf(dpre[b][o], x[b][i], acc) over b in batch
 // order from 0 (welvet_dense.metal:155-178).  v_mfma_f32_32x32x2f32 computes
@@ -3005,21 +2963,6 @@ hipError_t gemv_dispatch(int batch, const GemvArgs &a, hipStream_t s) {
   return hipErrorInvalidValue;
 }
 
-#define WH_DT_SWITCH(dt, F)                                                                       \
-  switch (dt) {                                                                                   \
-  case kFloat64: F(kFloat64); case kFloat32: F(kFloat32); case kFloat16: F(kFloat16);             \
-  case kBFloat16: F(kBFloat16); case kFP8E4M3: F(kFP8E4M3); case kFP8E5M2: F(kFP8E5M2);           \
-  case kInt64: F(kInt64); case kInt32: F(kInt32); case kInt16: F(kInt16); case kInt8: F(kInt8);   \
-  case kUint64: F(kUint64); case kUint32: F(kUint32); case kUint16: F(kUint16);                   \
-  case kUint8: F(kUint8); case kInt4: F(kInt4); case kUint4: F(kUint4); case kFP4: F(kFP4);       \
-  case kInt2: F(kInt2); case kUint2: F(kUint2); case kTernary: F(kTernary);                       \
-  case kBinary: F(kBinary); case kInt: F(kInt); case kUint: F(kUint); case kUintptr: F(kUintptr); \
-  case kComplex64: F(kComplex64); case kComplex128: F(kComplex128); case kNF4: F(kNF4);           \
-  case kFP6: F(kFP6); case kInt6: F(kInt6); case kUint6: F(kUint6); case kInt5: F(kInt5);         \
-  case kUint5: F(kUint5); case kInt3: F(kInt3); case kUint3: F(kUint3);                           \
-  default: return hipErrorInvalidValue;                                                           \
-  }
-
 }  // namespace
 
 void set_forward_path(int path) { g_forward_path = path; }
@@ -3222,13 +3165,8 @@ hipError_t launch_forward(const DevStore &w, int batch, const float *x, const do
   const int f = kernel_fmt(w.dtype);
   if (kernel_body(w, f) == nullptr) return hipErrorInvalidValue;
   const bool batched = route == 1 && batch > 1 && gemv_batch_fits(w, batch);
-  if (route == 3 || (route == 1 && batch > 4 && !batched)) {
-#define WH_GEN(D)                                                                        \
-  gemv_generic_kernel<D><<<w.rows, 256, 0, s>>>(w, batch, x, bias, bias_len, act, pre, post); \
-  return hipGetLastError();
-    WH_DT_SWITCH(w.dtype, WH_GEN)
-#undef WH_GEN
-  }
+  if (route == 3 || (route == 1 && batch > 4 && !batched))
+    return launch_ragged_forward(w, batch, x, bias, bias_len, act, pre, post, s);
   if (route == 1) {
     GemvArgs a{kernel_body(w, f), w.lut, w.scale, w.minv, x, w.cols, w.rows, w.cols / fmt_chunk_elems(f),
                row_bytes_of(w), bias, bias_len, act, pre, post};
@@ -3503,11 +3441,11 @@ hipError_t launch_dw_batch(const DwBatch &b, hipStream_t s) {
 }
 
 // The dX kernels whose epilogue applies the lower layer's derivative: the
-// no-split gemm_regt_kernel and the reduction of the stream-K GEMMs
+// no-split gemm_regt_kernel, the ragged dX and the reduction of the stream-K GEMMs
 // (sk_reduce_kernel); not the transposed no-split bf3r epilogue.
 bool backward_dx_applies_next(const DevStore &w, int batch, int next_act) {
   if (knob(kTuneFoldDeriv) == 0 || !act_piecewise(next_act)) return false;
-  if (dx_rows(w, batch)) return true;
+  if (dx_rows(w, batch) || dx_route(w, batch) == 3) return true;
   if (dx_route(w, batch) != 2) return false;
   const int bk = dx_bf3_kind(w, batch);
   return bk < 0 || !plan_fwd_gemm(kernel_fmt(w.dtype), bk, batch, w.rows, w.cols).rows;
@@ -3535,11 +3473,8 @@ hipError_t launch_backward(const DevStore &w, int batch, const float *x, const f
   if (dX == nullptr) {
     // no input gradient wanted (the first layer of a training step)
   } else if (route == 3) {
-#define WH_DXG(D)                                                                         \
-  dx_generic_kernel<D><<<blocks_for((int64_t)batch * w.cols), 256, 0, s>>>(w, batch, dpre, dX); \
-  break;
-    WH_DT_SWITCH(w.dtype, WH_DXG)
-#undef WH_DXG
+    e = launch_ragged_dx(w, batch, dpre, dX, chain.dx_next_pre, chain.dx_next_act, s);
+    if (e != hipSuccess) return e;
   } else if (route == 1) {
     const int nseg = (w.rows + kDxSegRows - 1) / kDxSegRows;
     DxArgs a{kernel_body(w, f), w.lut, w.scale, w.minv, dpre, w.rows, w.cols, w.cols / fmt_chunk_elems(f),

@@ -94,6 +94,14 @@ size_t backward_workspace_bytes(const DevStore &w, int batch);
 hipError_t launch_forward(const DevStore &w, int batch, const float *x, const double *bias,
                           int bias_len, int act, float *pre, float *post, void *ws, size_t ws_bytes,
                           hipStream_t s);
+// ---- ragged.hip: any row alignment, any batch, f64 products and sums
+hipError_t launch_ragged_forward(const DevStore &w, int batch, const float *x, const double *bias, int bias_len,
+                                 int act, float *pre, float *post, hipStream_t s);
+// dX = dpre . W; next_pre (nullable): times act'(next_pre) of the layer below
+// (a piecewise activation) on the stored fl32.
+hipError_t launch_ragged_dx(const DevStore &w, int batch, const float *dpre, float *dX, const float *next_pre,
+                            int next_act, hipStream_t s);
+// ---- dense.hip
 // SwiGLU's Gate and Up projections at batch 1 in one launch (two stores of
 // one format and shape): g_pre = Gate x, u_pre = Up x, h = fl32(silu(g)) * u.
 // forward_pair_fits: whether the pair kernel takes the stores (FP8, NF4 /

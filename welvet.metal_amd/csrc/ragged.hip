@@ -1,0 +1,389 @@
+// ragged.hip — Dense forward and dX for rows that do not start on a chunk
+// boundary (an input width that is no multiple of the format's chunk: 4
+// elements for 32-bit formats, 8 for 16-bit, 16 for 8-bit, 32 below), any
+// format, any batch.
+//
+// A chunk of E codes may start at any bit of the packed body: a lane loads
+// the dwords that cover it (one more than a chunk has) and shifts them into
+// the aligned chunk the other kernels' decode takes.  Products and sums are
+// f64 (each f32 operand widened): on the f64 MFMA from batch 5 on, where the
+// f64 matrix rate (half of fp32's) is far above what these shapes reach, and
+// on the VALU for the batch 1-4 row products.
+#include <algorithm>
+
+#include "codec.hpp"
+#include "kernel_formats.hpp"
+#include "kernels.hpp"
+
+namespace wh {
+namespace {
+
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
+struct RaggedArgs {
+  const uint8_t *body;
+  const float *lut;
+  float scale, minv;
+  const float *A;  // x [M][K], or dpre [M][K] for dX
+  int M, K, N;     // product dims; a stored row has `cols` elements
+  int cols;
+  int nst;  // k stages
+  int gx;   // tiles along N (one-dimensional grid: tile = blockIdx.x)
+};
+
+// Chunk of E codes that starts at element `elem` of the body.  Reads at most
+// 4 bytes past the chunk: inside the store's padding for every elem < n.
+template <int F>
+__device__ inline void load_chunk_at(const uint8_t *__restrict__ body, int64_t elem, uint32_t (&w)[FI<F>::kW]) {
+  constexpr int BITS = FI<F>::kBits, W = FI<F>::kW;
+  struct __attribute__((packed, aligned(4))) Words { uint32_t v[W]; };
+  if constexpr (BITS >= 32) {
+    const Words p = *(const Words *)(body + elem * (BITS / 8));
+#pragma unroll
+    for (int i = 0; i < W; ++i) w[i] = p.v[i];
+  } else {
+    const int64_t bit = elem * BITS;
+    const uint8_t *p = body + (bit >> 5) * 4;
+    const uint32_t sh = (uint32_t)bit & 31u;
+    const Words v = *(const Words *)p;
+    const uint32_t last = *(const uint32_t *)(p + 4 * W);
+#pragma unroll
+    for (int i = 0; i < W; ++i) w[i] = __builtin_amdgcn_alignbit(i + 1 < W ? v.v[i + 1] : last, v.v[i], sh);
+  }
+}
+
+// NK (a multiple of 4, or 1 or 2) consecutive values of a row of K floats
+// from k on; `whole`: all of them lie inside the row.  Otherwise each load is
+// clamped to the row's last value (the caller zeroes what lies past it).
+template <int NK>
+__device__ inline void load_row(const float *__restrict__ row, int k, int K, bool whole, float (&v)[NK]) {
+  if (whole) {
+    if constexpr (NK % 4 == 0) {
+      struct __attribute__((packed, aligned(4))) Quad { float f[4]; };
+#pragma unroll
+      for (int q = 0; q < NK; q += 4) {
+        const Quad p = *(const Quad *)(row + k + q);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) v[q + t] = p.f[t];
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < NK; ++q) v[q] = row[k + q];
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < NK; ++q) v[q] = row[min(k + q, K - 1)];
+  }
+}
+
+// Batch 1-4 (B = 1, 2 or 4 rows of x; rows past M repeat the last one and are
+// not stored).  S waves share an output row, its chunks dealt to their lanes
+// in turn; a block holds 4 / S rows.
+template <int F, int B>
+__global__ void __launch_bounds__(256) ragged_gemv_kernel(RaggedArgs a, int S, const double *bias, int bias_len,
+                                                          int act, float *pre, float *post) {
+  using I = FI<F>;
+  constexpr int E = I::kE, W = I::kW;
+  __shared__ __align__(16) float lut_s[I::kTable];
+  __shared__ double red[4][B];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if constexpr (I::kLut) {
+    TabCopy<F> tab;
+    tab.load(a.lut, tid);
+    tab.store(lut_s, tid);
+    __syncthreads();
+  }
+  const int part = wave & (S - 1);
+  const int o = blockIdx.x * (4 / S) + wave / S;
+  const int row = min(o, a.N - 1);
+  double acc[B];
+#pragma unroll
+  for (int b = 0; b < B; ++b) acc[b] = 0.0;
+  const int nchunks = (a.K + E - 1) / E;
+  const int64_t base = (int64_t)row * a.cols;
+  for (int c = part * 64 + lane; c < nchunks; c += 64 * S) {
+    const int k = c * E;
+    uint32_t w[W];
+    load_chunk_at<F>(a.body, base + k, w);
+    const bool whole = k + E <= a.K;
+    // pieces of at most 8 elements: x of B rows in registers
+    constexpr int P = E < 8 ? E : 8;
+#pragma unroll
+    for (int p = 0; p < E; p += P) {
+      float xv[B][P];
+#pragma unroll
+      for (int b = 0; b < B; ++b)
+        load_row<P>(a.A + (int64_t)min(b, a.M - 1) * a.K, k + p, a.K, whole, xv[b]);
+#pragma unroll
+      for (int e = 0; e < P; ++e) {
+        const bool in = whole || k + p + e < a.K;
+        const double wv = in ? (double)chunk_value<F>(w, p + e, lut_s, a.scale, a.minv) : 0.0;
+#pragma unroll
+        for (int b = 0; b < B; ++b) acc[b] = fma(wv, in ? (double)xv[b][e] : 0.0, acc[b]);
+      }
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    const double s = wave_sum(acc[b]);
+    if (lane == 0) red[wave][b] = s;
+  }
+  __syncthreads();
+  // thread t: row t / B of the block, batch row t % B
+  if (tid < (4 / S) * B) {
+    const int r = tid / B, b = tid % B, oo = blockIdx.x * (4 / S) + r;
+    double s = 0.0;
+    for (int i = 0; i < S; ++i) s += red[r * S + i][b];
+    if (oo < a.N && b < a.M) bias_act_store(s, oo, bias, bias_len, act, pre, post, (int64_t)b * a.N + oo);
+  }
+}
+
+// k per lane and stage of the MFMA kernels: lane group h = lane / 16 supplies
+// k = k0 + KR h + t at step t, a run of KR consecutive elements of its row.
+template <int F>
+struct RaggedShape {
+  static constexpr int E = FI<F>::kE;
+  static constexpr int KR = E >= 8 ? 32 : 4 * E;
+  static constexpr int NCH = KR / E;
+  static constexpr int ST = 4 * KR;
+};
+
+// Sum over the block's waves (each holds the same T tiles over its own k
+// stages) in wave order, one output element per thread and turn; store(mt,
+// nt, i, j, sum) with i, j the row and column in the 16 x 16 tile.
+// v_mfma_f64_16x16x4: register r of lane (j, h) is row 4 r + h, column j.
+template <int T, int NT, typename Store>
+__device__ inline void ragged_sum(double *ex, const doublex4 (&acc)[T], int nwaves, Store store) {
+  const int tid = threadIdx.x, lane = tid & 63, g = tid >> 6;
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) ex[((g * T + t) * 4 + r) * 64 + lane] = acc[t][r];
+  __syncthreads();
+  for (int q = tid; q < T * 256; q += nwaves * 64) {
+    double s = 0.0;
+    for (int w = 0; w < nwaves; ++w) s += ex[w * T * 256 + q];
+    const int t = q >> 8, r = (q >> 6) & 3, l = q & 63;
+    store(t / NT, t % NT, 4 * r + (l >> 4), l & 15, s);
+  }
+}
+
+// Forward, batch > 4: C[m][n] = sum_k x[m][k] W[n][k] on
+// v_mfma_f64_16x16x4_f64.  A wave owns MT x NT tiles of 16 x 16 and walks k
+// stages g, g + KG, ...; the block's waves share the tiles and split the
+// stages, so K is never split across blocks (no partial tiles in memory).
+template <int F, int MT, int NT, int KG>
+__global__ void __launch_bounds__(64 * KG) ragged_gemm_kernel(RaggedArgs a, const double *bias, int bias_len,
+                                                              int act, float *pre, float *post) {
+  using I = FI<F>;
+  using S = RaggedShape<F>;
+  constexpr int E = S::E, W = I::kW, KR = S::KR, NCH = S::NCH, ST = S::ST;
+  __shared__ __align__(16) float lut_s[I::kTable];
+  __shared__ double ex[KG * MT * NT * 256];
+  const int tid = threadIdx.x, lane = tid & 63, g = tid >> 6, nw = blockDim.x >> 6;
+  const int j = lane & 15, h = lane >> 4;
+  const int n0 = blockIdx.x % a.gx * 16 * NT, m0 = blockIdx.x / a.gx * 16 * MT;
+  if constexpr (I::kLut) {
+    TabCopy<F> tab;
+    tab.load(a.lut, tid);
+    tab.store(lut_s, tid);
+    __syncthreads();
+  }
+  const float *xr[MT];
+  int64_t wr[NT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) xr[t] = a.A + (int64_t)min(m0 + 16 * t + j, a.M - 1) * a.K;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) wr[t] = (int64_t)min(n0 + 16 * t + j, a.N - 1) * a.cols;
+  doublex4 acc[MT * NT];
+#pragma unroll
+  for (int t = 0; t < MT * NT; ++t) acc[t] = doublex4{0.0, 0.0, 0.0, 0.0};
+  const int klast = (a.K - 1) / E * E;
+  for (int s = g; s < a.nst; s += nw) {
+    const int k0 = s * ST + KR * h;
+    const bool whole = (s + 1) * ST <= a.K;  // uniform over the wave
+    uint32_t w[NT][NCH][W];
+    float x[MT][KR];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) load_chunk_at<F>(a.body, wr[t] + min(k0 + c * E, klast), w[t][c]);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) load_row<KR>(xr[t], k0, a.K, whole, x[t]);
+#pragma unroll
+    for (int q = 0; q < KR; ++q) {
+      const bool in = whole || k0 + q < a.K;
+      double bv[NT], av[MT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        bv[t] = in ? (double)chunk_value<F>(w[t][q / E], q % E, lut_s, a.scale, a.minv) : 0.0;
+#pragma unroll
+      for (int t = 0; t < MT; ++t) av[t] = in ? (double)x[t][q] : 0.0;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          acc[mt * NT + nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[mt], bv[nt], acc[mt * NT + nt], 0, 0, 0);
+    }
+  }
+  ragged_sum<MT * NT, NT>(ex, acc, nw, [&](int mt, int nt, int i, int jj, double s) {
+    const int m = m0 + 16 * mt + i, n = n0 + 16 * nt + jj;
+    if (m < a.M && n < a.N) bias_act_store(s, n, bias, bias_len, act, pre, post, (int64_t)m * a.N + n);
+  });
+}
+
+// dX: C[m][i] = sum_o dpre[m][o] W[o][i], K = rows, N = cols.  A wave decodes
+// the 16-column pieces of a stage's rows into its own LDS tile (pitch 17) and
+// reads them back as B operands; otherwise as ragged_gemm_kernel.  next_pre:
+// the layer below's piecewise activation derivative is applied to the stored
+// fl32, as gemm_regt_kernel does.
+template <int F>
+struct RaggedTShape {
+  static constexpr int E = FI<F>::kE;
+  static constexpr int KR = E >= 4 ? 16 : 8;
+  static constexpr int ST = 4 * KR;
+  static constexpr int DE = E >= 16 ? 16 : E;   // elements a chunk load decodes
+  static constexpr int CPR = 16 / DE;           // chunk loads per row piece
+  static constexpr int NCH = ST * CPR / 64;     // chunk loads per lane and stage
+  static constexpr int P = 17;
+  static_assert(ST * CPR % 64 == 0, "whole chunk loads per lane");
+};
+template <int F, int MT, int KG>
+__global__ void __launch_bounds__(64 * KG) ragged_dx_kernel(RaggedArgs a, float *out, const float *next_pre,
+                                                            int next_act) {
+  using I = FI<F>;
+  using S = RaggedTShape<F>;
+  using V = typename I::Acc;
+  constexpr int E = S::E, W = I::kW, KR = S::KR, ST = S::ST, DE = S::DE, CPR = S::CPR, NCH = S::NCH, P = S::P;
+  __shared__ __align__(16) float lut_s[I::kTable];
+  __shared__ V tile[KG][ST * P];
+  __shared__ double ex[KG * MT * 256];
+  const int tid = threadIdx.x, lane = tid & 63, g = tid >> 6, nw = blockDim.x >> 6;
+  const int j = lane & 15, h = lane >> 4;
+  const int n0 = blockIdx.x % a.gx * 16, m0 = blockIdx.x / a.gx * 16 * MT;
+  if constexpr (I::kLut) {
+    TabCopy<F> tab;
+    tab.load(a.lut, tid);
+    tab.store(lut_s, tid);
+    __syncthreads();
+  }
+  const float *xr[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) xr[t] = a.A + (int64_t)min(m0 + 16 * t + j, a.M - 1) * a.K;
+  doublex4 acc[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) acc[t] = doublex4{0.0, 0.0, 0.0, 0.0};
+  V *tw = tile[g];
+  for (int s = g; s < a.nst; s += nw) {
+    const int k0 = s * ST;
+    const bool whole = k0 + ST <= a.K;
+    uint32_t w[NCH][W];
+    float x[MT][KR];
+    // load c: row q / CPR, piece q % CPR of the row's 16 columns
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      const int q = lane + 64 * c;
+      const int o = min(k0 + q / CPR, a.K - 1), col = min(n0 + (q % CPR) * DE, a.N - 1);
+      load_chunk_at<F>(a.body, (int64_t)o * a.cols + col, w[c]);
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t) load_row<KR>(xr[t], k0 + KR * h, a.K, whole, x[t]);
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      const int q = lane + 64 * c;
+      const bool in = whole || k0 + q / CPR < a.K;
+#pragma unroll
+      for (int e = 0; e < DE; ++e) {
+        const V v = chunk_value<F>(w[c], e, lut_s, a.scale, a.minv);
+        tw[(q / CPR) * P + (q % CPR) * DE + e] = in ? v : V(0);
+      }
+    }
+    // one wave's LDS operations complete in order: its tile is whole before
+    // it is read, and read before the next stage overwrites it
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int q = 0; q < KR; ++q) {
+      const bool in = whole || k0 + KR * h + q < a.K;
+      const double bv = (double)tw[(KR * h + q) * P + j];
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(in ? (double)x[t][q] : 0.0, bv, acc[t], 0, 0, 0);
+    }
+    asm volatile("" ::: "memory");
+  }
+  ragged_sum<MT, 1>(ex, acc, nw, [&](int mt, int, int i, int jj, double s) {
+    const int m = m0 + 16 * mt + i, n = n0 + jj;
+    if (m >= a.M || n >= a.N) return;
+    const int64_t idx = (int64_t)m * a.N + n;
+    float v = (float)s;
+    if (next_pre != nullptr) v = v * act_prime_piecewise(next_pre[idx], next_act);
+    out[idx] = v;
+  });
+}
+
+RaggedArgs ragged_args(const DevStore &w, const float *A, int M, int K, int N, int f) {
+  // a zero scale decodes as 1 (native_codec.cpp weight_at)
+  return RaggedArgs{kernel_body(w, f), w.lut, w.scale == 0.0f ? 1.0f : w.scale, w.minv, A, M, K, N, w.cols, 0, 0};
+}
+
+template <int F>
+hipError_t ragged_forward(RaggedArgs a, const double *bias, int bias_len, int act, float *pre, float *post,
+                          hipStream_t s) {
+  if (a.M <= 4) {
+    const int nchunks = (a.K + FI<F>::kE - 1) / FI<F>::kE;
+    const int S = nchunks > 128 ? 4 : nchunks > 64 ? 2 : 1;
+    const int blocks = (a.N + 4 / S - 1) / (4 / S);
+    if (a.M == 1) ragged_gemv_kernel<F, 1><<<blocks, 256, 0, s>>>(a, S, bias, bias_len, act, pre, post);
+    else if (a.M == 2) ragged_gemv_kernel<F, 2><<<blocks, 256, 0, s>>>(a, S, bias, bias_len, act, pre, post);
+    else ragged_gemv_kernel<F, 4><<<blocks, 256, 0, s>>>(a, S, bias, bias_len, act, pre, post);
+    return hipGetLastError();
+  }
+  a.nst = (a.K + RaggedShape<F>::ST - 1) / RaggedShape<F>::ST;
+  const int gx32 = (a.N + 31) / 32, gy32 = (a.M + 31) / 32;
+  if ((int64_t)gx32 * gy32 >= num_cus()) {
+    a.gx = gx32;
+    ragged_gemm_kernel<F, 2, 2, 4><<<gx32 * gy32, 64 * std::min(4, a.nst), 0, s>>>(a, bias, bias_len, act, pre, post);
+  } else {
+    a.gx = (a.N + 15) / 16;
+    ragged_gemm_kernel<F, 1, 1, 8><<<a.gx * ((a.M + 15) / 16), 64 * std::min(8, a.nst), 0, s>>>(a, bias, bias_len,
+                                                                                               act, pre, post);
+  }
+  return hipGetLastError();
+}
+
+template <int F>
+hipError_t ragged_dx(RaggedArgs a, float *dX, const float *next_pre, int next_act, hipStream_t s) {
+  a.nst = (a.K + RaggedTShape<F>::ST - 1) / RaggedTShape<F>::ST;
+  a.gx = (a.N + 15) / 16;
+  const int gy32 = (a.M + 31) / 32;
+  if ((int64_t)a.gx * gy32 >= 2 * num_cus())
+    ragged_dx_kernel<F, 2, 4><<<a.gx * gy32, 64 * std::min(4, a.nst), 0, s>>>(a, dX, next_pre, next_act);
+  else
+    ragged_dx_kernel<F, 1, 8><<<a.gx * ((a.M + 15) / 16), 64 * std::min(8, a.nst), 0, s>>>(a, dX, next_pre, next_act);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_ragged_forward(const DevStore &w, int batch, const float *x, const double *bias, int bias_len,
+                                 int act, float *pre, float *post, hipStream_t s) {
+  const int f = kernel_fmt(w.dtype);
+  if (kernel_body(w, f) == nullptr) return hipErrorInvalidValue;
+  const RaggedArgs a = ragged_args(w, x, batch, w.cols, w.rows, f);
+#define WH_RF(F) return ragged_forward<F>(a, bias, bias_len, act, pre, post, s);
+  WH_FMT_SWITCH(f, WH_RF)
+#undef WH_RF
+}
+
+hipError_t launch_ragged_dx(const DevStore &w, int batch, const float *dpre, float *dX, const float *next_pre,
+                            int next_act, hipStream_t s) {
+  const int f = kernel_fmt(w.dtype);
+  if (kernel_body(w, f) == nullptr) return hipErrorInvalidValue;
+  const RaggedArgs a = ragged_args(w, dpre, batch, w.rows, w.cols, f);
+#define WH_RD(F) return ragged_dx<F>(a, dX, next_pre, next_act, s);
+  WH_FMT_SWITCH(f, WH_RD)
+#undef WH_RD
+}
+
+}  // namespace wh

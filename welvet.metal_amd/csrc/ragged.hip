@@ -6,9 +6,18 @@
 // A chunk of E codes may start at any bit of the packed body: a lane loads
 // the dwords that cover it (one more than a chunk has) and shifts them into
 // the aligned chunk the other kernels' decode takes.  Products and sums are
-// f64 (each f32 operand widened): on the f64 MFMA from batch 5 on, where the
-// f64 matrix rate (half of fp32's) is far above what these shapes reach, and
-// on the VALU for the batch 1-4 row products.
+// f64 (each f32 operand widened): on the VALU for one row of x and for up to
+// four where the weights are few, else on the f64 MFMA.
+//
+// What bounds them: short rows, the launch and one load-compute-reduce chain
+// (4-6 us); large ones, the f64 matrix rate (half of fp32's) and the chunk
+// loads.  Measured against the kernels they replaced (a block per output row
+// that re-read the weights for every batch row; dX a thread per output), us:
+// Float32 1001 -> 777 b100 99 -> 11.6, Int8 393 -> 362 b20 16.1 -> 5.1, NF4
+// 4095^2 b1 15.5 -> 11.3, b20 238 -> 29.5.  x staged through LDS with
+// whole-row loads and 16-byte-aligned chunk loads with a shift were measured
+// and not kept: equal at 4095^2, 10-25% slower below (1001 -> 777 b20 Int8
+// 7.3 against 6.5, Float32 8.7 / 6.7), the staging lengthens the chain.
 #include <algorithm>
 
 #include "codec.hpp"
@@ -31,11 +40,12 @@ struct RaggedArgs {
   int gx;   // tiles along N (one-dimensional grid: tile = blockIdx.x)
 };
 
-// Chunk of E codes that starts at element `elem` of the body.  Reads at most
-// 4 bytes past the chunk: inside the store's padding for every elem < n.
-template <int F>
+// NE codes (a chunk, or its first NE) from element `elem` of the body on.
+// Reads at most 4 bytes past them: inside the store's padding for every
+// elem < n.
+template <int F, int NE = FI<F>::kE>
 __device__ inline void load_chunk_at(const uint8_t *__restrict__ body, int64_t elem, uint32_t (&w)[FI<F>::kW]) {
-  constexpr int BITS = FI<F>::kBits, W = FI<F>::kW;
+  constexpr int BITS = FI<F>::kBits, W = (NE * BITS + 31) / 32;
   struct __attribute__((packed, aligned(4))) Words { uint32_t v[W]; };
   if constexpr (BITS >= 32) {
     const Words p = *(const Words *)(body + elem * (BITS / 8));
@@ -76,14 +86,21 @@ __device__ inline void load_row(const float *__restrict__ row, int k, int K, boo
   }
 }
 
-// Batch 1-4 (B = 1, 2 or 4 rows of x; rows past M repeat the last one and are
-// not stored).  S waves share an output row, its chunks dealt to their lanes
-// in turn; a block holds 4 / S rows.
+// Row products, B = M rows of x: a block holds 4 / S output rows, S waves share one, its
+// pieces of P codes dealt to their lanes in turn.  One row: up to four codes
+// per lane (a whole chunk leaves most lanes of a short row idle).  More rows,
+// of which most start off a 16-byte boundary: one code per lane, so each
+// row's loads are whole cache lines (four dwords per lane of a 16-byte-strided
+// row take 39 cycles each: 4095^2 b2 32 us).
+template <int F, int B>
+constexpr int ragged_piece() {
+  return B > 1 ? 1 : FI<F>::kE < 4 ? FI<F>::kE : 4;
+}
 template <int F, int B>
 __global__ void __launch_bounds__(256) ragged_gemv_kernel(RaggedArgs a, int S, const double *bias, int bias_len,
                                                           int act, float *pre, float *post) {
   using I = FI<F>;
-  constexpr int E = I::kE, W = I::kW;
+  constexpr int P = ragged_piece<F, B>(), W = I::kW;
   __shared__ __align__(16) float lut_s[I::kTable];
   __shared__ double red[4][B];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -94,33 +111,34 @@ __global__ void __launch_bounds__(256) ragged_gemv_kernel(RaggedArgs a, int S, c
     __syncthreads();
   }
   const int part = wave & (S - 1);
-  const int o = blockIdx.x * (4 / S) + wave / S;
-  const int row = min(o, a.N - 1);
+  const int row = min((int)blockIdx.x * (4 / S) + wave / S, a.N - 1);
   double acc[B];
 #pragma unroll
   for (int b = 0; b < B; ++b) acc[b] = 0.0;
-  const int nchunks = (a.K + E - 1) / E;
+  const int npieces = (a.K + P - 1) / P;
   const int64_t base = (int64_t)row * a.cols;
-  for (int c = part * 64 + lane; c < nchunks; c += 64 * S) {
-    const int k = c * E;
+  for (int c = part * 64 + lane; c < npieces; c += 64 * S) {
+    const int k = c * P;
     uint32_t w[W];
-    load_chunk_at<F>(a.body, base + k, w);
-    const bool whole = k + E <= a.K;
-    // pieces of at most 8 elements: x of B rows in registers
-    constexpr int P = E < 8 ? E : 8;
+    load_chunk_at<F, P>(a.body, base + k, w);
+    const bool whole = k + P <= a.K;
+    float xv[B][P];
 #pragma unroll
-    for (int p = 0; p < E; p += P) {
-      float xv[B][P];
+    for (int b = 0; b < B; ++b) {
+      const int64_t off = (int64_t)b * a.K;
+      if (B == 1 && whole) {
+        load_x<P>(a.A + k, xv[b]);
+      } else {
 #pragma unroll
-      for (int b = 0; b < B; ++b)
-        load_row<P>(a.A + (int64_t)min(b, a.M - 1) * a.K, k + p, a.K, whole, xv[b]);
-#pragma unroll
-      for (int e = 0; e < P; ++e) {
-        const bool in = whole || k + p + e < a.K;
-        const double wv = in ? (double)chunk_value<F>(w, p + e, lut_s, a.scale, a.minv) : 0.0;
-#pragma unroll
-        for (int b = 0; b < B; ++b) acc[b] = fma(wv, in ? (double)xv[b][e] : 0.0, acc[b]);
+        for (int e = 0; e < P; ++e) xv[b][e] = a.A[off + min(k + e, a.K - 1)];
       }
+    }
+#pragma unroll
+    for (int e = 0; e < P; ++e) {
+      const bool in = whole || k + e < a.K;
+      const double wv = in ? (double)chunk_value<F>(w, e, lut_s, a.scale, a.minv) : 0.0;
+#pragma unroll
+      for (int b = 0; b < B; ++b) acc[b] = fma(wv, in ? (double)xv[b][e] : 0.0, acc[b]);
     }
   }
 #pragma unroll
@@ -129,12 +147,11 @@ __global__ void __launch_bounds__(256) ragged_gemv_kernel(RaggedArgs a, int S, c
     if (lane == 0) red[wave][b] = s;
   }
   __syncthreads();
-  // thread t: row t / B of the block, batch row t % B
-  if (tid < (4 / S) * B) {
-    const int r = tid / B, b = tid % B, oo = blockIdx.x * (4 / S) + r;
-    double s = 0.0;
-    for (int i = 0; i < S; ++i) s += red[r * S + i][b];
-    if (oo < a.N && b < a.M) bias_act_store(s, oo, bias, bias_len, act, pre, post, (int64_t)b * a.N + oo);
+  if (tid < (4 / S) * B) {  // thread t: output row t / B of the block, batch row t % B
+    const int r = tid / B, b = tid % B, o = blockIdx.x * (4 / S) + r;
+    double t = 0.0;
+    for (int i = 0; i < S; ++i) t += red[r * S + i][b];
+    if (o < a.N) bias_act_store(t, o, bias, bias_len, act, pre, post, (int64_t)b * a.N + o);
   }
 }
 
@@ -168,7 +185,7 @@ __device__ inline void ragged_sum(double *ex, const doublex4 (&acc)[T], int nwav
   }
 }
 
-// Forward, batch > 4: C[m][n] = sum_k x[m][k] W[n][k] on
+// Forward: C[m][n] = sum_k x[m][k] W[n][k] on
 // v_mfma_f64_16x16x4_f64.  A wave owns MT x NT tiles of 16 x 16 and walks k
 // stages g, g + KG, ...; the block's waves share the tiles and split the
 // stages, so K is never split across blocks (no partial tiles in memory).
@@ -330,16 +347,22 @@ RaggedArgs ragged_args(const DevStore &w, const float *A, int M, int K, int N, i
 template <int F>
 hipError_t ragged_forward(RaggedArgs a, const double *bias, int bias_len, int act, float *pre, float *post,
                           hipStream_t s) {
-  if (a.M <= 4) {
-    const int nchunks = (a.K + FI<F>::kE - 1) / FI<F>::kE;
-    const int S = nchunks > 128 ? 4 : nchunks > 64 ? 2 : 1;
+  // up to 4 rows as row products; from 8 M weights on the MFMA reads them at
+  // least as fast (4095^2 Int8 b2 / b4 17.3 / 17.5 us against 18.1 / 22.7)
+  if (a.M == 1 || (a.M <= 4 && (int64_t)a.K * a.N <= ((int64_t)8 << 20))) {
+    const int P = a.M == 1 ? ragged_piece<F, 1>() : 1;
+    const int npieces = (a.K + P - 1) / P;
+    const int S = npieces > 128 ? 4 : npieces > 64 ? 2 : 1;
     const int blocks = (a.N + 4 / S - 1) / (4 / S);
     if (a.M == 1) ragged_gemv_kernel<F, 1><<<blocks, 256, 0, s>>>(a, S, bias, bias_len, act, pre, post);
     else if (a.M == 2) ragged_gemv_kernel<F, 2><<<blocks, 256, 0, s>>>(a, S, bias, bias_len, act, pre, post);
+    else if (a.M == 3) ragged_gemv_kernel<F, 3><<<blocks, 256, 0, s>>>(a, S, bias, bias_len, act, pre, post);
     else ragged_gemv_kernel<F, 4><<<blocks, 256, 0, s>>>(a, S, bias, bias_len, act, pre, post);
     return hipGetLastError();
   }
   a.nst = (a.K + RaggedShape<F>::ST - 1) / RaggedShape<F>::ST;
+  // 32 x 32 outputs per block where that still fills the CUs (each load then
+  // feeds two tiles), else 16 x 16 on twice the waves
   const int gx32 = (a.N + 31) / 32, gy32 = (a.M + 31) / 32;
   if ((int64_t)gx32 * gy32 >= num_cus()) {
     a.gx = gx32;

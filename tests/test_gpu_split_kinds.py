@@ -1,0 +1,74 @@
+"""The split-x bf16 GEMM's kinds for batches above 16 (BFloat16, Float16,
+Float32, Int4, Uint8) against the oracle: edges of the row tiles (16, 32, 64),
+the k stage (64) and the column tiles, weights of one sign, and non-finite
+operands.  The products are exact (Float32: to 2^-23) and the sums fp32, so an
+output is within 1e-5 of the sum of magnitudes, as for the other kinds."""
+import numpy as np
+import pytest
+
+import pywelvet
+from oracle import DTYPE_NAMES
+from test_gpu_dense import check_forward, elementwise_bound, oracle_weights
+
+pytestmark = pytest.mark.gpu
+KINDS = [3, 2, 1, 14, 13]
+# (out, in, batch): K of one piece, inside a stage, 31.5 stages, whole stage
+# pairs; columns past a tile; batch at both sides of the 32- and 64-row tiles
+SHAPES = [(40, 32, 17), (129, 96, 32), (257, 2016, 33), (300, 1024, 64), (100, 512, 65), (8200, 128, 20),
+          (1000, 640, 130)]
+
+
+@pytest.fixture(scope="module", autouse=True)
+def device():
+    pywelvet.init()
+
+
+@pytest.mark.parametrize("dtype", KINDS, ids=[DTYPE_NAMES[d] for d in KINDS])
+def test_split_kinds(oracle, dtype):
+    rng = np.random.default_rng(40 + dtype)
+    for out, inn, batch in SHAPES:
+        W = rng.normal(0, 0.1, (out, inn)).astype(np.float32)
+        x = rng.normal(0, 1, (batch, inn)).astype(np.float32)
+        check_forward(oracle, dtype, W, x)
+        check_forward(oracle, dtype, W, x, act=2, bias=rng.normal(0, 0.1, out))
+    # K % 16 == 8: the half formats' rows are chunks, the x pieces are not
+    if dtype in (2, 3):
+        W = rng.normal(0, 0.1, (70, 72)).astype(np.float32)
+        check_forward(oracle, dtype, W, rng.normal(0, 1, (40, 72)).astype(np.float32))
+
+
+@pytest.mark.parametrize("lo,hi", [(0.5, 0.75), (-0.75, -0.5), (-0.05, 3.0), (0.25, 0.25)])
+def test_uint8_offsets(oracle, lo, hi):
+    """Uint8 ranges without 0, with an outlier on one side, and of no width."""
+    rng = np.random.default_rng(3)
+    W = rng.normal(0, 0.01, (96, 256)).astype(np.float32) + np.float32((lo + hi) / 2 if lo * hi > 0 else 0)
+    W = np.clip(W, lo, hi)
+    W[0, 0], W[-1, -1] = lo, hi
+    x = rng.normal(0, 1, (40, 256)).astype(np.float32)
+    pre, _ = pywelvet.forward(W, x, dtype=13)
+    Wd = oracle_weights(oracle, 13, W)
+    ref = x.astype(np.float64) @ Wd.T
+    assert np.all(np.abs(pre - ref) <= elementwise_bound(Wd, x, 1e-5))
+
+
+@pytest.mark.parametrize("dtype", [3, 2, 1, 13])
+@pytest.mark.parametrize("batch", [20, 70])
+def test_split_kinds_nonfinite(oracle, dtype, batch):
+    """Infinities and NaN in x (all kinds) and W (the float ones): the class
+    of every output is that of the whole operands' product.  K = 80 ends
+    inside a k stage, which then holds the next row's first weights."""
+    rng = np.random.default_rng(batch + dtype)
+    W = rng.choice(np.float32([-1.0, -0.5, 0.5, 1.0, 0.0]), (40, 80)).astype(np.float32)
+    W[0, 0], W[0, 1] = 1.0, -1.0
+    x = rng.choice(np.float32([-2.0, -1.0, 1.0, 0.0, 0.37]), (batch, 80)).astype(np.float32)
+    x[3, 5], x[4, 6], x[5, 7], x[6, 1], x[6, 2] = np.inf, -np.inf, np.nan, np.inf, -np.inf
+    if dtype != 13:
+        W[7, 3], W[9, 0], W[11, 79], W[13, 4] = np.inf, -np.inf, np.inf, np.nan
+    pre, _ = pywelvet.forward(W, x, dtype=dtype)
+    Wd = oracle_weights(oracle, dtype, W)
+    with np.errstate(invalid="ignore"):
+        ref = np.array([[np.sum(x[m].astype(np.float64) * Wd[n]) for n in range(40)] for m in range(batch)])
+    assert np.array_equal(np.isnan(pre), np.isnan(ref))
+    assert np.array_equal(pre[np.isinf(ref)], ref[np.isinf(ref)].astype(np.float32))
+    ok = np.isfinite(ref)
+    assert np.allclose(pre[ok], ref[ok], rtol=1e-5, atol=1e-4)

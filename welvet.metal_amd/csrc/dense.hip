@@ -12,7 +12,9 @@
 //   forward, batch 2-8    gemv_loopb_kernel where the batch's x fits in
 //                         registers; gemv_kernel for other batch <= 4 shapes.
 //   forward, batch > 4    split-x bf16 MFMA GEMM (x = three exact bf16 parts)
-//                         for FP8 / Int8 / FP4 / NF4: gemm_bf3r_kernel without
+//                         for FP8 / Int8 / FP4 / NF4, above batch 16 also for
+//                         the half formats, Float32, Int4 and Uint8:
+//                         gemm_bf3r_kernel without
 //                         a k split, else gemm_bf3{,s,k}_kernel + sk_reduce;
 //                         fp32 MFMA gemm_regr / gemm_regx (batch <= 16, no k
 //                         split), gemm_reg / gemm_sk (+ sk_reduce) for the
@@ -779,6 +781,15 @@ struct GemmArgs {
   float post = 1.0f;
 };
 
+// Split-x kinds from BK_B16 on: the kind for the reduction's recomputation of
+// NaN sums (-1: none), and for Uint8 the weights' common offset and the row
+// sums of A it multiplies (null: no such term).
+struct SplitFix {
+  int kind = -1;
+  double offset = 0.0;
+  const double *rowsum = nullptr;
+};
+
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int kBM = 64, kBN = 64, kBK = 64, kPad = 1;
@@ -1485,13 +1496,29 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // bf16 once the per-tensor scale (applied by the reduction) is factored out:
 // E4M3 and E5M2 from the decode-ready copy, Int8 and FP4 codes as they are,
 // and NF4 table values as three exact bf16 parts (hi + mid + lo, like x).
-enum Bf3Kind { BK_E4 = 0, BK_I8 = 1, BK_FP4 = 2, BK_NF4 = 3, BK_E5 = 4 };
+// The kinds from BK_B16 on serve batches above 16: BFloat16 codes as they
+// are, Float16 as two exact parts (8 + 3 significand bits), Float32 as three
+// (split like x), Int4 codes as integers (times 16: the nibbles stay in the
+// high half of a byte) and Uint8 codes as integers q - zp around the code zp
+// nearest to the value 0, the rest of the offset, min + zp * scale, times the
+// row sum of x added by the reduction (SplitFix).
+enum Bf3Kind {
+  BK_E4 = 0, BK_I8 = 1, BK_FP4 = 2, BK_NF4 = 3, BK_E5 = 4, BK_B16 = 5, BK_H16 = 6, BK_F32 = 7, BK_I4 = 8, BK_U8 = 9
+};
+
+// Uint8's centre code, the one whose value is nearest to 0 (weights of both
+// signs then keep small integers: no cancellation against the offset).
+__host__ __device__ inline float u8_centre(float scale, float minv) {
+  const float c = scale > 0.0f ? -minv / scale : 0.0f;
+  return c >= 255.0f ? 255.0f : c > 0.0f ? floorf(c + 0.5f) : 0.0f;
+}
 
 template <int BK>
 struct B3 {
-  static constexpr int kBits = (BK <= BK_I8 || BK == BK_E5) ? 8 : 4;
+  static constexpr int kBits = BK == BK_F32 ? 32 : (BK == BK_B16 || BK == BK_H16) ? 16
+                             : (BK == BK_FP4 || BK == BK_NF4 || BK == BK_I4) ? 4 : 8;
   static constexpr int kWords = kBits;  // words of a lane's 32 weights per stage
-  static constexpr int kParts = BK == BK_NF4 ? 3 : 1;
+  static constexpr int kParts = (BK == BK_NF4 || BK == BK_F32) ? 3 : BK == BK_H16 ? 2 : 1;
 };
 
 typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
@@ -1510,7 +1537,8 @@ inline __device__ bf16x8 bf16x8_of(const uint32_t (&u)[4]) {
 // 8 consecutive weights (the words of MFMA step q) as B operands: parts[0..P).
 // NF4 reads the split table t3[code] = {hi | mid << 16, lo}.
 template <int BK>
-__device__ inline void bf3_weights(const uint32_t *w, int q, const uint2 *t3, bf16x8 (&parts)[B3<BK>::kParts]) {
+__device__ inline void bf3_weights(const uint32_t *w, int q, const uint2 *t3, float zp,
+                                   bf16x8 (&parts)[B3<BK>::kParts]) {
   if constexpr (BK == BK_E4) {
     const uint32_t w0 = w[2 * q], w1 = w[2 * q + 1];
     const uint32_t u[4] = {
@@ -1545,6 +1573,51 @@ __device__ inline void bf3_weights(const uint32_t *w, int q, const uint2 *t3, bf
         __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(wd, 1.0f, 2)),
         __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(wd, 1.0f, 3))};
     parts[0] = bf16x8_of(u);
+  } else if constexpr (BK == BK_B16) {
+    const uint32_t u[4] = {w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]};
+    parts[0] = bf16x8_of(u);
+  } else if constexpr (BK == BK_H16 || BK == BK_F32) {
+    uint32_t part[3][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float v[2];
+      if constexpr (BK == BK_H16) {
+        const uint32_t wd = w[4 * q + i];
+        v[0] = (float)__builtin_bit_cast(_Float16, (uint16_t)wd);
+        v[1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(wd >> 16));
+      } else {
+        v[0] = u2f(w[8 * q + 2 * i]);
+        v[1] = u2f(w[8 * q + 2 * i + 1]);
+      }
+      uint32_t b[3][2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        b[0][e] = f2u(v[e]);
+        const float r = v[e] - u2f(f2u(v[e]) & 0xffff0000u);
+        b[1][e] = f2u(r);
+        b[2][e] = f2u(r - u2f(f2u(r) & 0xffff0000u));
+      }
+#pragma unroll
+      for (int k = 0; k < B3<BK>::kParts; ++k) part[k][i] = __builtin_amdgcn_perm(b[k][1], b[k][0], 0x07060302u);
+    }
+#pragma unroll
+    for (int k = 0; k < B3<BK>::kParts; ++k) parts[k] = bf16x8_of(part[k]);
+  } else if constexpr (BK == BK_I4) {
+    const uint32_t hi = w[q] & 0xf0f0f0f0u, lo = (w[q] & 0x0f0f0f0fu) << 4;  // elements 2j + 1, 2j: 16 times the code
+    uint32_t u[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      u[i] = __builtin_amdgcn_perm(f2u((float)(int8_t)(uint8_t)(hi >> (8 * i))),
+                                   f2u((float)(int8_t)(uint8_t)(lo >> (8 * i))), 0x07060302u);
+    parts[0] = bf16x8_of(u);
+  } else if constexpr (BK == BK_U8) {
+    uint32_t u[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t wd = w[2 * q + (i >> 1)] >> ((i & 1) * 16);
+      u[i] = __builtin_amdgcn_perm(f2u((float)((wd >> 8) & 0xffu) - zp), f2u((float)(wd & 0xffu) - zp), 0x07060302u);
+    }
+    parts[0] = bf16x8_of(u);
   } else {  // NF4
     const uint32_t wd = w[q];
     uint32_t hi[4], mid[4], lo[4];
@@ -1569,6 +1642,7 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
   constexpr int XT = kBK / XE;        // threads per x row
   __shared__ uint16_t Xs[2][3][BM][kBf3Row];
   __shared__ uint2 t3[16];
+  const float zp = BK == BK_U8 ? u8_centre(a.scale, a.minv) : 0.0f;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int j = lane & 31, h = lane >> 5;
   if constexpr (BK == BK_NF4) {
@@ -1709,7 +1783,7 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
 #pragma unroll
           for (int c = 0; c < NC; ++c) {
             bf16x8 pp[1];
-            bf3_weights<BK>(wr[d][c], q, t3, pp);
+            bf3_weights<BK>(wr[d][c], q, t3, zp, pp);
             bv[q][c][0] = pp[0];
           }
         load_w(min(u + D, last), wr[d]);
@@ -1723,7 +1797,7 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
         for (int q = 0; q < 4; ++q) {
           bf16x8 bv[NC][NP];
 #pragma unroll
-          for (int c = 0; c < NC; ++c) bf3_weights<BK>(wr[d][c], q, t3, bv[c]);
+          for (int c = 0; c < NC; ++c) bf3_weights<BK>(wr[d][c], q, t3, zp, bv[c]);
           mfma_step(acc, buf, q, bv);
         }
         load_w(min(u + D, last), wr[d]);
@@ -1770,6 +1844,7 @@ __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
   __shared__ uint16_t Xs[2][2][3][BM][kBf3Row];  // [buffer][group][part][m][k]
   static_assert(sizeof(Xs) >= (size_t)P * 16 * 256 * sizeof(float), "the exchange fits the x buffers");
   __shared__ uint2 t3[16];
+  const float zp = BK == BK_U8 ? u8_centre(a.scale, a.minv) : 0.0f;
   const int tid = threadIdx.x, grp = tid >> 8, gt = tid & 255, lane = tid & 63, wave = gt >> 6;
   const int j = lane & 31, h = lane >> 5;
   if constexpr (BK == BK_NF4) {
@@ -1908,7 +1983,7 @@ __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
 #pragma unroll
           for (int c = 0; c < NC; ++c) {
             bf16x8 pp[1];
-            bf3_weights<BK>(wr[d][c], q, t3, pp);
+            bf3_weights<BK>(wr[d][c], q, t3, zp, pp);
             bv[q][c][0] = pp[0];
           }
         load_x(min(u + D, last), xf[d], xin[d]);  // first: the early x store waits for it alone
@@ -1921,7 +1996,7 @@ __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
         for (int q = 0; q < 4; ++q) {
           bf16x8 bv[NC][NP];
 #pragma unroll
-          for (int c = 0; c < NC; ++c) bf3_weights<BK>(wr[d][c], q, t3, bv[c]);
+          for (int c = 0; c < NC; ++c) bf3_weights<BK>(wr[d][c], q, t3, zp, bv[c]);
           mfma_step(acc, buf, q, bv);
         }
         load_w(min(u + D, last), wr[d]);
@@ -1996,6 +2071,7 @@ __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
   static_assert(XE == 4 && (NW == 2 || NW == 4), "16-row split-x layout");
   __shared__ uint16_t Xs[2][3][BM][kBf3Row];
   __shared__ uint2 t3[16];
+  const float zp = BK == BK_U8 ? u8_centre(a.scale, a.minv) : 0.0f;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int j = lane & 15, g = lane >> 4;
   if constexpr (BK == BK_NF4) {
@@ -2103,7 +2179,7 @@ __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
 #pragma unroll
           for (int c = 0; c < CG; ++c) {
             bf16x8 pp[1];
-            bf3_weights<BK>(wr[d][c], q, t3, pp);
+            bf3_weights<BK>(wr[d][c], q, t3, zp, pp);
             bv[q][c][0] = pp[0];
           }
         load_x(min(u + D, last), xf[d], xin[d]);
@@ -2116,7 +2192,7 @@ __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
         for (int q = 0; q < 2; ++q) {
           bf16x8 bv[CG][NP];
 #pragma unroll
-          for (int c = 0; c < CG; ++c) bf3_weights<BK>(wr[d][c], q, t3, bv[c]);
+          for (int c = 0; c < CG; ++c) bf3_weights<BK>(wr[d][c], q, t3, zp, bv[c]);
           mfma_step(acc, buf, q, bv);
         }
         load_w(min(u + D, last), wr[d]);
@@ -2163,6 +2239,7 @@ __global__ void __launch_bounds__(64 * KG * CW) gemm_bf3r_kernel(GemmArgs a, con
   __shared__ uint16_t Xs[NB][KG][3][BM][kBf3Row];
   __shared__ float ex[KG - 1][CW][4][64];
   __shared__ uint2 t3[16];
+  const float zp = BK == BK_U8 ? u8_centre(a.scale, a.minv) : 0.0f;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int grp = wv / CW, cw = wv % CW, gt = tid & (64 * CW - 1);
   const int j = lane & 15, g = lane >> 4;
@@ -2257,7 +2334,7 @@ __global__ void __launch_bounds__(64 * KG * CW) gemm_bf3r_kernel(GemmArgs a, con
       if (r >= rounds) goto done;
       bf16x8 bv[2][NP];
 #pragma unroll
-      for (int q = 0; q < 2; ++q) bf3_weights<BK>(wr[d], q, t3, bv[q]);
+      for (int q = 0; q < 2; ++q) bf3_weights<BK>(wr[d], q, t3, zp, bv[q]);
       load_x(min(r + D, last), xf[d], xin[d]);
       load_w(min(r + D, last), wr[d]);
 #pragma unroll
@@ -2292,6 +2369,25 @@ done:
   }
 }
 
+// A NaN sum of a split product, redone on the whole operands: a part of x or
+// w that is zero times an infinite other operand is NaN, where the product of
+// the whole values is an infinity, and an infinite weight of the next row
+// inside the last k stage meets the zeros that pad x.  The walk ends at the
+// first NaN, so tensors full of them cost little.
+__device__ inline double split_nan_fix(const GemmArgs &a, int kind, int m, int n) {
+  const uint8_t *row = a.body + (int64_t)n * a.row_bytes;
+  double s = 0.0;
+  for (int k = 0; k < a.K && !isnan(s); ++k) {
+    float w;
+    if (kind == BK_B16) w = u2f((uint32_t)((const uint16_t *)row)[k] << 16);
+    else if (kind == BK_H16) w = (float)((const _Float16 *)row)[k];
+    else if (kind == BK_F32) w = ((const float *)row)[k];
+    else w = (float)row[k] * a.scale + a.minv;  // BK_U8
+    s += (double)a.A[(int64_t)m * a.K + k] * (double)w;
+  }
+  return s;
+}
+
 // Sum of a tile's stream-K partials in workgroup order (f64).  Grid: x =
 // tile, y = 1024-element slice of the tile; each thread adds four adjacent
 // outputs with float4 loads.  The forward applies bias + activation, dX
@@ -2299,10 +2395,13 @@ done:
 // a volume training step the pre of the layer below, act its piecewise
 // activation: the derivative act_deriv_kernel would apply, the same
 // expression as gemm_regt_kernel's NEXT epilogue).
-template <bool FWD>
+// FIX: the split-x kinds with a row-sum term or a NaN recomputation
+// (SplitFix); an instantiation of its own, since that code costs
+// the plain reduction 3%.
+template <bool FWD, bool FIX = false>
 __global__ void __launch_bounds__(256) sk_reduce_kernel(GemmArgs a, const double *bias, int bias_len,
                                                         int act, float *out, float *post,
-                                                        const float *next_pre) {
+                                                        const float *next_pre, SplitFix fx) {
   const int t = blockIdx.x;
   const int b0 = (int)((int64_t)t * a.nst / a.per_block);
   const int b1 = (int)(((int64_t)(t + 1) * a.nst - 1) / a.per_block);
@@ -2341,6 +2440,10 @@ __global__ void __launch_bounds__(256) sk_reduce_kernel(GemmArgs a, const double
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     if (a.post != 1.0f) sum[i] *= (double)a.post;
+    if constexpr (FIX) {
+      if (fx.rowsum != nullptr) sum[i] += fx.offset * fx.rowsum[m];
+      if (i < nv && isnan(sum[i])) sum[i] = split_nan_fix(a, fx.kind, m, n + i);
+    }
     float p = (float)sum[i];
     if constexpr (FWD) {
       if (bias != nullptr && n + i < bias_len) p = (float)((double)p + bias[n + i]);
@@ -2359,6 +2462,17 @@ __global__ void __launch_bounds__(256) sk_reduce_kernel(GemmArgs a, const double
       if constexpr (FWD) post[idx + i] = qv[i];
     }
   }
+}
+
+// out[m] = sum over k of A [m][k], f64.
+__global__ void __launch_bounds__(256) rowsum_kernel(const float *__restrict__ A, int K, double *out) {
+  __shared__ double red[4];
+  double s = 0.0;
+  for (int k = threadIdx.x; k < K; k += 256) s += (double)A[(int64_t)blockIdx.x * K + k];
+  s = wave_sum(s);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) out[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
 __global__ void __launch_bounds__(256) reduce_plain_kernel(const float *ws, int slices, int64_t total,
@@ -2755,6 +2869,26 @@ int bf3_kind(const DevStore &w) {
   return -1;
 }
 
+// The forward's kind at a batch: above 16 rows (whose x pieces of 16 values
+// need K % 16 == 0) also the half formats, Float32, Int4 and Uint8.
+int bf3_fwd_kind(const DevStore &w, int batch) {
+  const int bk = bf3_kind(w);
+  if (bk >= 0 || knob(kTuneBf3) == 0 || batch <= 16 || w.cols % 16 != 0) return bk;
+  const int64_t units = (int64_t)((batch + 31) / 32) * ((w.rows + 127) / 128) * ((w.cols + kBK - 1) / kBK);
+  switch (w.dtype) {
+  case kBFloat16: return BK_B16;
+  case kFloat16: return BK_H16;
+  // six products: fewer outputs than 512 lose to the fp32 MFMA's narrower
+  // tiles (768 -> 300 b256 12.8 us against 11.1, 512^2 10.1 against 10.3)
+  case kFloat32: return w.rows >= 512 ? BK_F32 : -1;
+  case kInt4: return BK_I4;
+  // its row sums are a launch of their own (1024^2 b100, 512 units: 14.8 us
+  // against 14.0 on the fp32 MFMA; 2048^2 b48, 1024 units: 17.5 / 19.3)
+  case kUint8: return units >= 1024 ? BK_U8 : -1;
+  }
+  return -1;
+}
+
 inline int blocks_for(int64_t n) {
   int64_t b = (n + 255) / 256;
   return (int)(b < 1 ? 1 : (b > 65536 ? 65536 : b));
@@ -2792,7 +2926,11 @@ SkPlan plan_sk(int M, int K, int N, int bm = kBM, int bn = kBN, int occ = 2, int
   p.nst = (K + kBK - 1) / kBK / kg;
   const int64_t T = (int64_t)p.gx * p.gy * p.nst;
   const int64_t G = (int64_t)occ * num_cus();
-  p.per_block = (int)((T + G - 1) / G);
+  // at most 16 partial tiles per tile: past that the reduction's serial sum
+  // costs more than the shorter shares save (FP8 32 x 128 tiles, 4096 -> 512
+  // b48 19.2 -> 11.7 us, 8192 -> 300 b24 28.0 -> 15.0, 1024^2 b100 11.9 ->
+  // 9.5; 8 and 4 lose at K >= 4096, 24 and 32 at K <= 4096)
+  p.per_block = std::max((int)((T + G - 1) / G), (p.nst + 15) / 16);
   p.blocks = (int)((T + p.per_block - 1) / p.per_block);
   p.maxspan = (p.per_block + p.nst - 1) / p.nst + 1;
   p.ws_bytes = (size_t)p.blocks * p.maxspan * bm * bn * sizeof(float);
@@ -2806,22 +2944,42 @@ dim3 sk_reduce_grid(const SkPlan &p) {
 bool reg_gemm_ok(int f) { return f >= 0 && fmt_chunk_elems(f) >= 8; }  // formats of <= 16 bits
 
 
+// Row sums of x for Uint8 on the split-x GEMM, at the end of the workspace.
+size_t rowsum_bytes(int M) { return ((size_t)M * sizeof(double) + 15) / 16 * 16; }
+
 // Forward GEMM plan: the split-x bf16 kernel for the formats it takes, the
 // register-B kernel for other <= 16-bit formats, else the LDS-staged kernel.
 SkPlan plan_fwd_gemm(int f, int bk, int M, int K, int N) {
   if (bk >= 0) {
     const int occ = 2;
-    const int bm = M <= 16 ? 16 : M <= 32 ? 32 : 64;
-    // tile width: 128 output columns where outputs are few (N <= 8192) for
-    // the 16-row tile and for the one-byte kinds' 32-row tile (their
-    // stream-K partial tiles then weigh as much as the weights: 4096^2 FP8
-    // b16 12.9 against 16.3 us, b32 15.2 against 18.1, NF4 b16 14.3 against
-    // 17.2; 11008 -> 4096 FP8 b16 21.4 against 22.9), else 256 (4096 ->
-    // 11008 b8 FP8 19.6 against 20.1; the 4-bit kinds' 32-row tile keeps
-    // the two-group workgroups, which need 256)
-    const bool narrow = N <= 8192 && (bm == 16 || (bm == 32 && bk != BK_NF4 && bk != BK_FP4));
-    const int bn = narrow ? 128 : 256;
     const int stages = (K + kBK - 1) / kBK;
+    // Above 16 rows: 32-row tiles while the problem is small, else 64-row
+    // ones.  units: 32 x 128 tiles times k stages.  Measured over K 512-11008,
+    // N 300-11008, batch 24-512: FP8 1024^2 b256 12.6 us on 32 x 128 tiles
+    // against 14.8 on 64 x 256 ones, 512^2 b64 7.4 / 10.9; the two-group
+    // 32 x 256 tiles up to 8192 units for the kinds of one product per weight
+    // part (4096^2 FP8 b64 15.6 / 19.1, 2048 -> 8192 b128 23.8 / 25.1, 4096 ->
+    // 11008 b128 50.6 / 47.3) and up to 4096 for NF4 (2048 -> 8192 b64 22.5 /
+    // 23.5, b256 60.8 / 56.5).  The 16-bit kinds gain nothing from the groups
+    // there (twice the weight registers): 32 x 128 up to 4096 units (4096^2
+    // b64 18.3 / 21.9, b100 27.0 / 24.6), Float32 64 x 128 tiles beyond 1024
+    // (4096^2 b64 26.5 us, 32 x 128 28.7, 64 x 256 29.7; 4096 -> 11008 b512
+    // 329 / - / 339).
+    const int64_t units = (int64_t)((M + 31) / 32) * ((N + 127) / 128) * stages;
+    const bool wide_codes = bk == BK_B16 || bk == BK_H16 || bk == BK_F32;
+    const bool small = units <= (bk == BK_F32 ? 1024 : wide_codes ? 4096 : 2048);
+    const bool mid = !wide_codes && stages % 2 == 0 && units <= (bk == BK_NF4 ? 4096 : 8192);
+    const int bm = M <= 16 ? 16 : (M <= 32 || small || mid) ? 32 : 64;
+    // tile width: 128 output columns where outputs are few (N <= 8192) for
+    // the 16-row tile and for the one-byte kinds' 32-row tile at batch <= 32
+    // (their stream-K partial tiles then weigh as much as the weights: 4096^2
+    // FP8 b16 12.9 against 16.3 us, b32 15.2 against 18.1, NF4 b16 14.3
+    // against 17.2; 11008 -> 4096 FP8 b16 21.4 against 22.9), else 256 (4096
+    // -> 11008 b8 FP8 19.6 against 20.1; the 4-bit kinds' 32-row tile keeps
+    // the two-group workgroups, which need 256)
+    const bool four_bit = bk == BK_NF4 || bk == BK_FP4 || bk == BK_I4;
+    const bool narrow = bk == BK_F32 || (M <= 16 ? N <= 8192 : M <= 32 ? N <= 8192 && !four_bit : small);
+    const int bn = narrow ? 128 : 256;
     // no k split for K <= 2048 (measured at batch 5-16: 1024^2 6.6 against
     // 10.3 us, 2048 -> 4096 9.4 against 14.3; at K = 4096 about even, at
     // K = 11008 1.6x slower: too few workgroups for the serial K walk)
@@ -2840,13 +2998,14 @@ SkPlan plan_fwd_gemm(int f, int bk, int M, int K, int N) {
       p.ws_bytes = 0;
       return p;
     }
-    // two-group workgroups: every 64-row tile; 32-row tiles only for the
-    // 4-bit kinds (FP8 / Int8 measured slower there)
-    const bool groups = bn == 256 && stages % 2 == 0 &&
-                        (bm == 64 || (bm == 32 && (bk == BK_NF4 || bk == BK_FP4)));
+    // two-group workgroups: every 64 x 256 tile, the 32 x 256 tiles above
+    // batch 32 and, up to it, those of the 4-bit kinds (FP8 / Int8 measured
+    // slower there)
+    const bool groups = bn == 256 && stages % 2 == 0 && (bm == 64 || (bm == 32 && (M > 32 || four_bit)));
     SkPlan p = groups ? plan_sk(M, K, N, bm, bn, 1, 2)
                       : plan_sk(M, K, N, bm, bn, occ);
     p.bf3 = true;
+    if (bk == BK_U8) p.ws_bytes += rowsum_bytes(M);
     return p;
   }
   // batch <= 16 without a k split (gemm_regr_kernel): K <= 2048 as for the
@@ -2976,7 +3135,7 @@ int tuning(int key) { return key < 0 || key >= kNumTune || !tune_key_kept(key) ?
 
 size_t forward_workspace_bytes(const DevStore &w, int batch) {
   if (fwd_route(w, batch) != 2) return 0;
-  return plan_fwd_gemm(kernel_fmt(w.dtype), bf3_kind(w), batch, w.cols, w.rows).ws_bytes;
+  return plan_fwd_gemm(kernel_fmt(w.dtype), bf3_fwd_kind(w, batch), batch, w.cols, w.rows).ws_bytes;
 }
 
 // gemm_bf3r_kernel for plan p (p.rows): the forward (bias, activation, pre
@@ -3034,6 +3193,10 @@ hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
   if (p.bm == 32) gemm_bf3k_kernel<BK, 1, 2, 2><<<p.blocks, 512, 0, s>>>(a);                  \
   else gemm_bf3k_kernel<BK, 2, 2, 2><<<p.blocks, 512, 0, s>>>(a);
     switch (bk) {
+    case BK_B16: WH_GK(BK_B16) break;
+    case BK_H16: WH_GK(BK_H16) break;
+    case BK_I4: WH_GK(BK_I4) break;
+    case BK_U8: WH_GK(BK_U8) break;
     case BK_E4: WH_GK(BK_E4) break;
     case BK_I8: WH_GK(BK_I8) break;
     case BK_FP4: WH_GK(BK_FP4) break;
@@ -3044,7 +3207,24 @@ hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
 #undef WH_GK
     return hipGetLastError();
   }
+#define WH_GB32(BK)  /* batches above 16 only */                                      \
+  if (p.bm == 32) {                                                                   \
+    if (p.bn == 128) gemm_bf3_kernel<BK, 1, 1, 1><<<p.blocks, 256, 0, s>>>(a);         \
+    else gemm_bf3_kernel<BK, 1, 1, 2><<<p.blocks, 256, 0, s>>>(a);                     \
+  } else {                                                                            \
+    if (p.bn == 128) gemm_bf3_kernel<BK, 2, 1, 1><<<p.blocks, 256, 0, s>>>(a);         \
+    else gemm_bf3_kernel<BK, 2, 1, 2><<<p.blocks, 256, 0, s>>>(a);                     \
+  }
   switch (bk) {
+  case BK_B16: WH_GB32(BK_B16) break;
+  case BK_H16: WH_GB32(BK_H16) break;
+  case BK_F32:  // 128-column tiles only (plan_fwd_gemm)
+    if (p.bn != 128) return hipErrorInvalidValue;
+    if (p.bm == 32) gemm_bf3_kernel<BK_F32, 1, 1, 1><<<p.blocks, 256, 0, s>>>(a);
+    else gemm_bf3_kernel<BK_F32, 2, 1, 1><<<p.blocks, 256, 0, s>>>(a);
+    break;
+  case BK_I4: WH_GB32(BK_I4) break;
+  case BK_U8: WH_GB32(BK_U8) break;
   case BK_E4: WH_GB(BK_E4) break;
   case BK_I8: WH_GB(BK_I8) break;
   case BK_FP4: WH_GB(BK_FP4) break;
@@ -3053,6 +3233,7 @@ hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
   default: return hipErrorInvalidValue;
   }
 #undef WH_GB
+#undef WH_GB32
   return hipGetLastError();
 }
 
@@ -3279,14 +3460,22 @@ hipError_t launch_forward(const DevStore &w, int batch, const float *x, const do
     WH_FMT_SWITCH(f, WH_GV)
 #undef WH_GV
   }
-  const int bk = bf3_kind(w);
+  const int bk = bf3_fwd_kind(w, batch);
   const SkPlan p = plan_fwd_gemm(f, bk, batch, w.cols, w.rows);
   if (ws_bytes < p.ws_bytes) return hipErrorInvalidValue;
   GemmArgs a{kernel_body(w, f), w.lut, w.scale, w.minv, x, batch, w.cols, w.rows, row_bytes_of(w),
              p.gx, p.gy, p.nst, p.per_block, p.maxspan, (float *)ws, p.bm, p.bn};
+  SplitFix fx;
   if (p.bf3) {
-    a.post = (bk == BK_I8 || bk == BK_NF4) ? w.scale : 1.0f;
+    a.post = (bk == BK_I8 || bk == BK_NF4 || bk == BK_U8) ? w.scale : bk == BK_I4 ? w.scale * 0.0625f : 1.0f;
     if (bk == BK_E4 || bk == BK_E5) a.body = w.kbody;
+    if (bk == BK_B16 || bk == BK_H16 || bk == BK_F32 || bk == BK_U8) fx.kind = bk;
+    if (bk == BK_U8) {
+      fx.offset = (double)w.minv + (double)u8_centre(w.scale, w.minv) * (double)w.scale;
+      double *rs = (double *)((char *)ws + p.ws_bytes - rowsum_bytes(batch));
+      rowsum_kernel<<<batch, 256, 0, s>>>(x, w.cols, rs);
+      fx.rowsum = rs;
+    }
     if (p.rows) return launch_bf3r<true>(p, bk, a, bias, bias_len, act, pre, post, s);
     const hipError_t e = launch_bf3(p, bk, a, s);
     if (e != hipSuccess) return e;
@@ -3317,7 +3506,10 @@ hipError_t launch_forward(const DevStore &w, int batch, const float *x, const do
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  sk_reduce_kernel<true><<<sk_reduce_grid(p), 256, 0, s>>>(a, bias, bias_len, act, pre, post, nullptr);
+  if (fx.kind >= 0)
+    sk_reduce_kernel<true, true><<<sk_reduce_grid(p), 256, 0, s>>>(a, bias, bias_len, act, pre, post, nullptr, fx);
+  else
+    sk_reduce_kernel<true><<<sk_reduce_grid(p), 256, 0, s>>>(a, bias, bias_len, act, pre, post, nullptr, fx);
   return hipGetLastError();
 }
 
@@ -3504,7 +3696,7 @@ hipError_t launch_backward(const DevStore &w, int batch, const float *x, const f
       e = launch_bf3(p, bk, a, s);
       if (e != hipSuccess) return e;
       sk_reduce_kernel<false><<<sk_reduce_grid(p), 256, 0, s>>>(a, nullptr, 0, chain.dx_next_act, dX, nullptr,
-                                                                chain.dx_next_pre);
+                                                                chain.dx_next_pre, SplitFix{});
     }
   } else if (dx_rows(w, batch)) {
     const int st = dx_rows_stage(f);
@@ -3536,7 +3728,7 @@ hipError_t launch_backward(const DevStore &w, int batch, const float *x, const f
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     sk_reduce_kernel<false><<<sk_reduce_grid(p), 256, 0, s>>>(a, nullptr, 0, chain.dx_next_act, dX, nullptr,
-                                                              chain.dx_next_pre);
+                                                              chain.dx_next_pre, SplitFix{});
   }
   e = hipGetLastError();
   if (e != hipSuccess) return e;

@@ -125,6 +125,10 @@ welvet_status store_prepare_backward(Store *w, int batch, hipStream_t s) {
   return ok();
 }
 
+// Bytes of a body's allocation: a GEMM's last 64-element k stage may read
+// past the last row's end (at most 63 elements of 4 bytes).
+static size_t body_alloc(size_t body_bytes) { return (body_bytes + 256 + 255) / 256 * 256; }
+
 // Device scratch reused by encode: Meta + Stats.
 struct EncodeScratch {
   Meta meta;
@@ -141,8 +145,7 @@ welvet_status store_make(Store *w, int dtype, int rows, int cols, const float *d
   const int64_t n = w->n();
   const int bits = dtype_bits(dtype);
   w->body_bytes = (size_t)((n * bits + 7) / 8);
-  // padding: a full 16-byte chunk past the last element stays in the allocation
-  const size_t alloc = ((w->body_bytes + 64 + 255) / 256) * 256;
+  const size_t alloc = body_alloc(w->body_bytes);
   WH_HIP(hipMalloc(&w->body, alloc));
   WH_HIP(hipMemsetAsync(w->body, 0, alloc, s));
   if (dtype == kFP8E4M3 || dtype == kFP8E5M2) {
@@ -204,7 +207,7 @@ welvet_status store_from_native(Store *w, int dtype, int rows, int cols, float s
   w->rows = rows;
   w->cols = cols;
   w->body_bytes = (size_t)((n * dtype_bits(dtype) + 7) / 8);
-  const size_t alloc = ((w->body_bytes + 64 + 255) / 256) * 256;
+  const size_t alloc = body_alloc(w->body_bytes);
   WH_HIP(hipMalloc(&w->body, alloc));
   WH_HIP(hipMemsetAsync(w->body, 0, alloc, s));
   if (is_f32) {  // WeightStore::f32; the scale of a Float32 store is 1 (encode_format_none)

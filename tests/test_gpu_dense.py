@@ -631,3 +631,19 @@ def test_read_probe():
         st.close()
         buf.free()
         sink.free()
+
+
+@pytest.mark.parametrize("out,inn", [(1, 1), (31, 33), (33, 31), (63, 65), (65, 63), (129, 127), (10, 300), (2100, 2050)])
+@pytest.mark.parametrize("batch", [1, 2, 23, 24, 25, 49])
+def test_dw_ragged_tiles(oracle, out, inn, batch):
+    """dW of sizes that are no multiple of 128, on 64 x 64 blocks (small
+    layers) and 128 x 128 ones, batches around its groups of 24 and 12 rows:
+    the reference's sequential FMA bit for bit."""
+    rng = np.random.default_rng(out * 7 + inn + batch)
+    W = rng.normal(0, 0.1, (out, inn)).astype(np.float32)
+    x = rng.normal(0, 1, (batch, inn)).astype(np.float32)
+    gy = rng.normal(0, 1, (batch, out)).astype(np.float32)
+    with pywelvet.Session(W, batch=batch, act=-1, dtype=1) as s:
+        _, dW = s.backward(x, gy, gy)
+    _, _, rdW = oracle.backward(W.astype(np.float64), x, gy, gy, -1)
+    assert_bit_equal(dW, rdW, "dW")

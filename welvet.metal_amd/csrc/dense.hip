@@ -2551,63 +2551,66 @@ __global__ void __launch_bounds__(256) dx_small_kernel(DxArgs a) {
 // bit patterns, denormals, infinities, NaNs and signed zeros), so a chain of
 // them over k = batch rows reproduces the reference exactly.  An odd batch
 // ends with a -0 product, which leaves every accumulator (-0 included) as it
-// is.  Block: 128 (o) x 128 (i) outputs, four waves of 64 x 64 (2 x 2 tiles of
-// 32 x 32); lane (j, h) supplies batch row b + h of operand column j: the
+// is.  Block: 64 T (o) x 64 T (i) outputs, four waves of T x T tiles of 32 x
+// 32 (T = 2, or 1 where 128 x 128 blocks would leave CUs idle: the chain over
+// the batch cannot be split, so a small layer is bound by one block's chain
+// and a wave with one tile has a quarter of the MFMAs in it); lane (j, h) supplies batch row b + h of operand column j: the
 // A operand dpre[b][o0 + j], the B operand x[b][i0 + j] (coalesced 128-byte
 // rows).  Out-of-range rows and columns read a clamped valid element and are
 // never stored.
+template <int T>
 __global__ void __launch_bounds__(256) dw_mfma_kernel(const float *__restrict__ dpre,
                                                       const float *__restrict__ x, int B, int rows,
                                                       int cols, float *__restrict__ dW, int *flag) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int j = lane & 31, h = lane >> 5;
-  const int o0 = blockIdx.y * 128 + (wave >> 1) * 64, i0 = blockIdx.x * 128 + (wave & 1) * 64;
-  const float *pa[2], *pb[2];
+  const int o0 = blockIdx.y * 64 * T + (wave >> 1) * 32 * T, i0 = blockIdx.x * 64 * T + (wave & 1) * 32 * T;
+  const float *pa[T], *pb[T];
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
+  for (int t = 0; t < T; ++t) {
     pa[t] = dpre + min(o0 + 32 * t + j, rows - 1);
     pb[t] = x + min(i0 + 32 * t + j, cols - 1);
   }
-  floatx16 acc[2][2];
+  floatx16 acc[T][T];
 #pragma unroll
-  for (int mt = 0; mt < 2; ++mt)
+  for (int mt = 0; mt < T; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
+    for (int nt = 0; nt < T; ++nt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0.0f;
   // groups of kU k steps (2 kU batch rows); group g + 1's loads are in flight
   // while group g's MFMAs run (two register sets).  Loads past the batch read
   // row 0; the -0 / 0 padding replaces them where they are used (a select
   // right after a load would make the compiler wait for that load at once).
-  constexpr int kU = 6;  // 24 loads per group: two groups fit the 63 loads a wave can have in flight
+  constexpr int kU = T == 2 ? 6 : 12;  // 24 loads per group: two groups fit the 63 loads a wave can have in flight
   const int ng = (B + 2 * kU - 1) / (2 * kU);
-  auto load = [&](int g, float (&av)[kU][2], float (&bv)[kU][2]) {
+  auto load = [&](int g, float (&av)[kU][T], float (&bv)[kU][T]) {
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
       const int b = g * 2 * kU + 2 * u + h;
       const int64_t bc = b < B ? b : 0;
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
+      for (int t = 0; t < T; ++t) {
         av[u][t] = pa[t][bc * rows];
         bv[u][t] = pb[t][bc * cols];
       }
     }
   };
-  auto mfmas = [&](int g, const float (&av)[kU][2], const float (&bv)[kU][2]) {
+  auto mfmas = [&](int g, const float (&av)[kU][T], const float (&bv)[kU][T]) {
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
       const int b = g * 2 * kU + 2 * u;
       if (b >= B) break;
       const bool in = b + h < B;
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
+      for (int mt = 0; mt < T; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
+        for (int nt = 0; nt < T; ++nt)
           acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? av[u][mt] : -0.0f, in ? bv[u][nt] : 0.0f,
                                                              acc[mt][nt], 0, 0, 0);
     }
   };
-  float a0[kU][2], b0v[kU][2], a1[kU][2], b1v[kU][2];
+  float a0[kU][T], b0v[kU][T], a1[kU][T], b1v[kU][T];
   load(0, a0, b0v);
   for (int g = 0; g < ng; g += 2) {
     load(g + 1, a1, b1v);
@@ -2619,9 +2622,9 @@ __global__ void __launch_bounds__(256) dw_mfma_kernel(const float *__restrict__ 
   // D[m][n]: lane (j, h) holds column j, rows 8 (r / 4) + 4 h + r % 4
   int bad = 0;
 #pragma unroll
-  for (int mt = 0; mt < 2; ++mt)
+  for (int mt = 0; mt < T; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
+    for (int nt = 0; nt < T; ++nt) {
       const int i = i0 + 32 * nt + j;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -3741,8 +3744,11 @@ hipError_t launch_backward(const DevStore &w, int batch, const float *x, const f
     dim3 g2(w.cols / 128, w.rows / 128);
     dw_mfma_lds_kernel<<<g2, 256, 0, s>>>(dpre, x, batch, w.rows, w.cols, dW, flag);
   } else {
-    dim3 g2((w.cols + 127) / 128, (w.rows + 127) / 128);
-    dw_mfma_kernel<<<g2, 256, 0, s>>>(dpre, x, batch, w.rows, w.cols, dW, flag);
+    const dim3 g2((w.cols + 127) / 128, (w.rows + 127) / 128), g1((w.cols + 63) / 64, (w.rows + 63) / 64);
+    if ((int64_t)g2.x * g2.y < num_cus())
+      dw_mfma_kernel<1><<<g1, 256, 0, s>>>(dpre, x, batch, w.rows, w.cols, dW, flag);
+    else
+      dw_mfma_kernel<2><<<g2, 256, 0, s>>>(dpre, x, batch, w.rows, w.cols, dW, flag);
   }
   return hipGetLastError();
 }

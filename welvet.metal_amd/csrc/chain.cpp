@@ -123,10 +123,10 @@ welvet_status run_forward(bool residual, int32_t batch, int32_t seq, int32_t dim
   welvet_status st = make(&L, residual, rows, dim, depth, act, dtype, packed);
   if (st.code) return st;
   const int64_t n = (int64_t)rows * dim;
-  WH_HIP(hipMemcpyAsync(L.x, x, n * sizeof(float), hipMemcpyHostToDevice, L.stream));
+  WH_HIP(copy_to_device(L.x, x, n * sizeof(float), L.stream));
   if ((st = forward(&L)).code) return st;
-  WH_HIP(hipMemcpyAsync(pre, L.pre[depth - 1], n * sizeof(float), hipMemcpyDeviceToHost, L.stream));
-  WH_HIP(hipMemcpyAsync(post, L.y, n * sizeof(float), hipMemcpyDeviceToHost, L.stream));
+  WH_HIP(copy_to_host(pre, L.pre[depth - 1], n * sizeof(float), L.stream));
+  WH_HIP(copy_to_host(post, L.y, n * sizeof(float), L.stream));
   WH_HIP(hipStreamSynchronize(L.stream));
   return ok();
 }
@@ -141,7 +141,7 @@ welvet_status run_normalbp(bool residual, int32_t batch, int32_t seq, int32_t di
   if (st.code) return st;
   const hipStream_t s = L.stream;
   const int64_t n = (int64_t)rows * dim, cn = (int64_t)dim * dim;
-  WH_HIP(hipMemcpyAsync(L.x, x, n * sizeof(float), hipMemcpyHostToDevice, s));
+  WH_HIP(copy_to_device(L.x, x, n * sizeof(float), s));
   if ((st = forward(&L)).code) return st;
   float *gy = nullptr, *g[2] = {nullptr, nullptr}, *gin = nullptr, *dpre = nullptr, *dw = nullptr;
   float *w_after = nullptr;
@@ -155,11 +155,11 @@ welvet_status run_normalbp(bool residual, int32_t batch, int32_t seq, int32_t di
   if (use_target) {
     float *d_t = nullptr;
     if ((st = L.alloc(&d_t, n)).code) return st;
-    WH_HIP(hipMemcpyAsync(d_t, grad_or_target, n * sizeof(float), hipMemcpyHostToDevice, s));
+    WH_HIP(copy_to_device(d_t, grad_or_target, n * sizeof(float), s));
     WH_HIP(launch_mse(L.y, d_t, n, d_loss, gy, L.ws, L.ws_bytes, s));
     WH_HIP(hipMemcpyAsync(&h_loss, d_loss, sizeof(double), hipMemcpyDeviceToHost, s));
   } else {
-    WH_HIP(hipMemcpyAsync(gy, grad_or_target, n * sizeof(float), hipMemcpyHostToDevice, s));
+    WH_HIP(copy_to_device(gy, grad_or_target, n * sizeof(float), s));
   }
   // the children in reverse; each one's dX is the gradient of the one before
   const float *gcur = gy;
@@ -179,11 +179,11 @@ welvet_status run_normalbp(bool residual, int32_t batch, int32_t seq, int32_t di
       if ((st = store_sgd(&L.child[i], dw + i * cn, lr, L.flag, s)).code) return st;
   for (int i = 0; i < depth; ++i)
     if ((st = store_export(L.child[i], w_after + i * cn, s)).code) return st;
-  WH_HIP(hipMemcpyAsync(W_after, w_after, depth * cn * sizeof(float), hipMemcpyDeviceToHost, s));
-  WH_HIP(hipMemcpyAsync(pre, L.pre[depth - 1], n * sizeof(float), hipMemcpyDeviceToHost, s));
-  WH_HIP(hipMemcpyAsync(post, L.y, n * sizeof(float), hipMemcpyDeviceToHost, s));
-  WH_HIP(hipMemcpyAsync(dX, gin, n * sizeof(float), hipMemcpyDeviceToHost, s));
-  WH_HIP(hipMemcpyAsync(dW, dw, depth * cn * sizeof(float), hipMemcpyDeviceToHost, s));
+  WH_HIP(copy_to_host(W_after, w_after, depth * cn * sizeof(float), s));
+  WH_HIP(copy_to_host(pre, L.pre[depth - 1], n * sizeof(float), s));
+  WH_HIP(copy_to_host(post, L.y, n * sizeof(float), s));
+  WH_HIP(copy_to_host(dX, gin, n * sizeof(float), s));
+  WH_HIP(copy_to_host(dW, dw, depth * cn * sizeof(float), s));
   WH_HIP(hipStreamSynchronize(s));
   *loss = h_loss;
   return ok();

@@ -28,7 +28,7 @@
 //   dW                    dw_mfma_kernel / dw_batch_kernel: fp32 MFMA over the
 //                         batch with the reference's per-element rounding
 //                         (welvet_dense.metal:155-178).
-//   unaligned rows        ragged.hip (f64 products on the f64 MFMA / VALU).
+//   unaligned rows        ragged.hpp (f64 products on the f64 MFMA / VALU).
 //
 // Accumulation is fp32 inside a lane/tile and f64 across split-K / segment
 // partials; outputs are fl32 of that, within the stated tolerance of the f64
@@ -40,6 +40,7 @@
 #include "codec.hpp"
 #include "kernel_formats.hpp"
 #include "kernels.hpp"
+#include "ragged.hpp"
 
 namespace wh {
 namespace {
@@ -3141,6 +3142,12 @@ size_t forward_workspace_bytes(const DevStore &w, int batch) {
   return plan_fwd_gemm(kernel_fmt(w.dtype), bf3_fwd_kind(w, batch), batch, w.cols, w.rows).ws_bytes;
 }
 
+size_t forward_workspace_min_bytes(const DevStore &w, int batch) {
+  const size_t b = forward_workspace_bytes(w, batch);
+  if (fwd_route(w, batch) != 2 || bf3_fwd_kind(w, batch) < BK_B16) return b;
+  return std::min(b, plan_fwd_gemm(kernel_fmt(w.dtype), -1, batch, w.cols, w.rows).ws_bytes);
+}
+
 // gemm_bf3r_kernel for plan p (p.rows): the forward (bias, activation, pre
 // and post) or dX (out only, FWD false).
 template <bool FWD>
@@ -3463,8 +3470,12 @@ hipError_t launch_forward(const DevStore &w, int batch, const float *x, const do
     WH_FMT_SWITCH(f, WH_GV)
 #undef WH_GV
   }
-  const int bk = bf3_fwd_kind(w, batch);
-  const SkPlan p = plan_fwd_gemm(f, bk, batch, w.cols, w.rows);
+  int bk = bf3_fwd_kind(w, batch);
+  SkPlan p = plan_fwd_gemm(f, bk, batch, w.cols, w.rows);
+  if (bk >= BK_B16 && ws_bytes < p.ws_bytes) {  // a fixed workspace that only the fp32 MFMA's plan fits
+    bk = -1;
+    p = plan_fwd_gemm(f, bk, batch, w.cols, w.rows);
+  }
   if (ws_bytes < p.ws_bytes) return hipErrorInvalidValue;
   GemmArgs a{kernel_body(w, f), w.lut, w.scale, w.minv, x, batch, w.cols, w.rows, row_bytes_of(w),
              p.gx, p.gy, p.nst, p.per_block, p.maxspan, (float *)ws, p.bm, p.bn};

@@ -1,6 +1,6 @@
 // kernel_formats.hpp — the storage formats as the product kernels read them:
 // kernel formats, the chunks lanes load, their decode, and the small device
-// helpers the kernels of dense.hip and ragged.hip share.
+// helpers the kernels of dense.hip and ragged.hpp share.
 #pragma once
 
 #include <hip/hip_runtime.h>

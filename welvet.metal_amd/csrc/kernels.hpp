@@ -89,12 +89,15 @@ hipError_t launch_e5m2_nonfinite(const uint8_t *codes, int64_t n, int *flag, hip
 // Bytes of workspace the forward / backward launches below need.
 size_t forward_workspace_bytes(const DevStore &w, int batch);
 size_t backward_workspace_bytes(const DevStore &w, int batch);
+// The least workspace launch_forward can run with: where the preferred plan
+// needs more than it is given, a format with an fp32 MFMA plan takes that.
+size_t forward_workspace_min_bytes(const DevStore &w, int batch);
 
 // pre/post [batch][rows] = act(x[batch][cols] . W^T (+ bias)).
 hipError_t launch_forward(const DevStore &w, int batch, const float *x, const double *bias,
                           int bias_len, int act, float *pre, float *post, void *ws, size_t ws_bytes,
                           hipStream_t s);
-// ---- ragged.hip: any row alignment, any batch, f64 products and sums
+// ---- ragged.hpp: any row alignment, any batch, f64 products and sums
 hipError_t launch_ragged_forward(const DevStore &w, int batch, const float *x, const double *bias, int bias_len,
                                  int act, float *pre, float *post, hipStream_t s);
 // dX = dpre . W; next_pre (nullable): times act'(next_pre) of the layer below

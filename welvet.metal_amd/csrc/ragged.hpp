@@ -1,4 +1,4 @@
-// ragged.hip — Dense forward and dX for rows that do not start on a chunk
+// ragged.hpp (part of dense.hip) — Dense forward and dX for rows that do not start on a chunk
 // boundary (an input width that is no multiple of the format's chunk: 4
 // elements for 32-bit formats, 8 for 16-bit, 16 for 8-bit, 32 below), any
 // format, any batch.
@@ -18,6 +18,8 @@
 // whole-row loads and 16-byte-aligned chunk loads with a shift were measured
 // and not kept: equal at 4095^2, 10-25% slower below (1001 -> 777 b20 Int8
 // 7.3 against 6.5, Float32 8.7 / 6.7), the staging lengthens the chain.
+#pragma once
+
 #include <algorithm>
 
 #include "codec.hpp"

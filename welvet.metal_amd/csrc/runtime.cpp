@@ -22,6 +22,7 @@
 
 #include "../../include/welvet_c.h"
 #include "codec.hpp"
+#include "hostio.hpp"
 #include "runtime.hpp"
 
 using namespace wh;
@@ -96,14 +97,20 @@ const char *device_identity() {
 }
 
 // ------------------------------------------------------- resident store
+template <typename T>
+static hipError_t store_alloc(const Store &w, T **p, size_t bytes) {
+  return w.pooled ? dev_alloc((void **)p, bytes) : hipMalloc((void **)p, bytes);
+}
+static void store_free(const Store &w, void *p) {
+  if (w.pooled) dev_free(p);
+  else (void)hipFree(p);
+}
+
 void free_store(Store *w) {
-  if (w->body) (void)hipFree(w->body);
-  if (w->kbody) (void)hipFree(w->kbody);
-  if (w->tbody) (void)hipFree(w->tbody);
+  for (void *p : {(void *)w->body, (void *)w->kbody, (void *)w->tbody, (void *)w->lut, (void *)w->bias})
+    if (p) store_free(*w, p);
   w->tbody = nullptr;
   w->tbody_ok = false;
-  if (w->lut) (void)hipFree(w->lut);
-  if (w->bias) (void)hipFree(w->bias);
   w->body = nullptr;
   w->kbody = nullptr;
   w->lut = nullptr;
@@ -116,7 +123,7 @@ welvet_status store_prepare_backward(Store *w, int batch, hipStream_t s) {
   if (w->tbody == nullptr) {
     // padding: the GEMM's last 64-column stage may read past the last row
     const size_t alloc = ((bytes + 64 + 255) / 256) * 256;
-    WH_HIP(hipMalloc(&w->tbody, alloc));
+    WH_HIP(store_alloc(*w, &w->tbody, alloc));
     WH_HIP(hipMemsetAsync(w->tbody, 0, alloc, s));
   }
   const uint8_t *src = (w->dtype == kFP8E4M3 || w->dtype == kFP8E5M2) ? w->kbody : w->body;
@@ -146,10 +153,10 @@ welvet_status store_make(Store *w, int dtype, int rows, int cols, const float *d
   const int bits = dtype_bits(dtype);
   w->body_bytes = (size_t)((n * bits + 7) / 8);
   const size_t alloc = body_alloc(w->body_bytes);
-  WH_HIP(hipMalloc(&w->body, alloc));
+  WH_HIP(store_alloc(*w, &w->body, alloc));
   WH_HIP(hipMemsetAsync(w->body, 0, alloc, s));
   if (dtype == kFP8E4M3 || dtype == kFP8E5M2) {
-    WH_HIP(hipMalloc(&w->kbody, alloc));
+    WH_HIP(store_alloc(*w, &w->kbody, alloc));
     WH_HIP(hipMemsetAsync(w->kbody, 0, alloc, s));
   }
   return store_encode(w, d_w, false, s);
@@ -169,8 +176,9 @@ welvet_status store_encode(Store *w, const float *d_w, bool repack, hipStream_t 
     w->minv = 0.0f;
     return ok();
   }
-  EncodeScratch *scratch = nullptr;
-  WH_HIP(hipMalloc(&scratch, sizeof(EncodeScratch)));
+  DevBuf buf(s);
+  WH_HIP(buf.alloc(sizeof(EncodeScratch)));
+  EncodeScratch *scratch = buf.as<EncodeScratch>();
   hipError_t e = launch_encode(dtype, d_w, n, w->body, w->kbody, &scratch->meta, &scratch->stats, s, repack);
   Meta m{};
   int nonfinite = 0;
@@ -181,13 +189,12 @@ welvet_status store_encode(Store *w, const float *d_w, bool repack, hipStream_t 
   }
   if (e == hipSuccess) e = hipMemcpyAsync(&m, &scratch->meta, sizeof(Meta), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  (void)hipFree(scratch);
   WH_HIP(e);
   w->scale = m.scale;
   w->minv = m.minv;
   w->finite = nonfinite == 0;
   if (dtype_lut(dtype)) {
-    if (w->lut == nullptr) WH_HIP(hipMalloc(&w->lut, kLutFloats * sizeof(float)));
+    if (w->lut == nullptr) WH_HIP(store_alloc(*w, &w->lut, kLutFloats * sizeof(float)));
     WH_HIP(launch_lut(dtype, w->scale, w->minv, w->lut, s));
     WH_HIP(hipStreamSynchronize(s));
   }
@@ -208,10 +215,10 @@ welvet_status store_from_native(Store *w, int dtype, int rows, int cols, float s
   w->cols = cols;
   w->body_bytes = (size_t)((n * dtype_bits(dtype) + 7) / 8);
   const size_t alloc = body_alloc(w->body_bytes);
-  WH_HIP(hipMalloc(&w->body, alloc));
+  WH_HIP(store_alloc(*w, &w->body, alloc));
   WH_HIP(hipMemsetAsync(w->body, 0, alloc, s));
   if (is_f32) {  // WeightStore::f32; the scale of a Float32 store is 1 (encode_format_none)
-    WH_HIP(hipMemcpyAsync(w->body, f32, (size_t)n * 4, hipMemcpyHostToDevice, s));
+    WH_HIP(copy_to_device(w->body, f32, (size_t)n * 4, s));
     w->scale = 1.0f;
     w->minv = 0.0f;
     WH_HIP(hipStreamSynchronize(s));
@@ -221,7 +228,7 @@ welvet_status store_from_native(Store *w, int dtype, int rows, int cols, float s
   w->scale = scale;
   w->minv = 0.0f;
   if (hdr) std::memcpy(&w->minv, raw, 4);
-  WH_HIP(hipMemcpyAsync(w->body, raw + hdr, w->body_bytes, hipMemcpyHostToDevice, s));
+  WH_HIP(copy_to_device(w->body, raw + hdr, w->body_bytes, s));
   std::vector<uint8_t> k;
   if (dtype == kFP8E4M3 || dtype == kFP8E5M2) {  // the decode-ready copy, made on the host
     k.resize(w->body_bytes);
@@ -236,12 +243,12 @@ welvet_status store_from_native(Store *w, int dtype, int rows, int cols, float s
       }
     }
     w->finite = finite;
-    WH_HIP(hipMalloc(&w->kbody, alloc));
+    WH_HIP(store_alloc(*w, &w->kbody, alloc));
     WH_HIP(hipMemsetAsync(w->kbody, 0, alloc, s));
-    WH_HIP(hipMemcpyAsync(w->kbody, k.data(), k.size(), hipMemcpyHostToDevice, s));
+    WH_HIP(copy_to_device(w->kbody, k.data(), k.size(), s));
   }
   if (dtype_lut(dtype)) {
-    WH_HIP(hipMalloc(&w->lut, kLutFloats * sizeof(float)));
+    WH_HIP(store_alloc(*w, &w->lut, kLutFloats * sizeof(float)));
     WH_HIP(launch_lut(dtype, w->scale, w->minv, w->lut, s));
   }
   WH_HIP(hipStreamSynchronize(s));  // k and the caller's buffers outlive the copies
@@ -249,23 +256,20 @@ welvet_status store_from_native(Store *w, int dtype, int rows, int cols, float s
 }
 
 welvet_status store_repack_host(Store *w, const float *values, hipStream_t s) {
-  float *d = nullptr;
+  DevBuf d(s);
   const size_t bytes = (size_t)w->n() * sizeof(float);
-  WH_HIP(hipMalloc(&d, bytes));
-  hipError_t e = hipMemcpyAsync(d, values, bytes, hipMemcpyHostToDevice, s);
-  welvet_status st = e == hipSuccess ? store_encode(w, d, true, s)
-                                     : make_status(kInternal, "hip: %s", hipGetErrorString(e));
-  e = hipStreamSynchronize(s);
-  (void)hipFree(d);
+  WH_HIP(d.alloc(bytes));
+  WH_HIP(copy_to_device(d.p, values, bytes, s));
+  const welvet_status st = store_encode(w, d.as<float>(), true, s);
   if (st.code) return st;
-  WH_HIP(e);
+  WH_HIP(hipStreamSynchronize(s));
   return ok();
 }
 
 welvet_status store_set_bias(Store *w, const double *bias, size_t bias_len, hipStream_t s) {
   if (bias == nullptr || bias_len == 0) return ok();
   if (bias_len > (size_t)INT32_MAX) return make_status(kInvalid, "bias too long");
-  WH_HIP(hipMalloc(&w->bias, bias_len * sizeof(double)));
+  WH_HIP(store_alloc(*w, &w->bias, bias_len * sizeof(double)));
   WH_HIP(hipMemcpyAsync(w->bias, bias, bias_len * sizeof(double), hipMemcpyHostToDevice, s));
   w->bias_len = (int)bias_len;
   return ok();
@@ -274,15 +278,11 @@ welvet_status store_set_bias(Store *w, const double *bias, size_t bias_len, hipS
 // Upload f32 weights and build the store.
 welvet_status store_from_host(Store *w, int dtype, int rows, int cols, const float *W_init,
                               hipStream_t s) {
-  float *d_w = nullptr;
+  DevBuf d(s);
   const size_t bytes = (size_t)rows * cols * sizeof(float);
-  WH_HIP(hipMalloc(&d_w, bytes));
-  hipError_t e = hipMemcpyAsync(d_w, W_init, bytes, hipMemcpyHostToDevice, s);
-  welvet_status st = e == hipSuccess ? store_make(w, dtype, rows, cols, d_w, s)
-                                     : make_status(kInternal, "hip: %s", hipGetErrorString(e));
-  (void)hipStreamSynchronize(s);
-  (void)hipFree(d_w);
-  return st;
+  WH_HIP(d.alloc(bytes));
+  WH_HIP(copy_to_device(d.p, W_init, bytes, s));
+  return store_make(w, dtype, rows, cols, d.as<float>(), s);
 }
 
 // WeightStore::apply_sgd (native_codec.cpp:909-945) on a device gradient,
@@ -324,7 +324,7 @@ welvet_status store_native(const Store &w, uint8_t *out, size_t cap, size_t *len
   if (len) *len = need;
   if (out == nullptr || cap < need) return make_status(kInvalid, "native: buffer too small (%zu)", need);
   if (hdr) std::memcpy(out, &w.minv, 4);
-  WH_HIP(hipMemcpyAsync(out + hdr, w.body, w.body_bytes, hipMemcpyDeviceToHost, s));
+  WH_HIP(copy_to_host(out + hdr, w.body, w.body_bytes, s));
   WH_HIP(hipStreamSynchronize(s));
   return ok();
 }
@@ -351,19 +351,25 @@ struct welvet_dense_session {
   void *ws = nullptr;
   size_t ws_bytes = 0;
   int *d_flag = nullptr;
+  bool pooled = false;  // the session of one host-buffer call: its memory is dev_alloc's
 };
 
 namespace {
+
+template <typename T>
+hipError_t session_alloc(welvet_dense_session *s, T **p, size_t bytes) {
+  return s->pooled ? dev_alloc((void **)p, bytes) : hipMalloc((void **)p, bytes);
+}
 
 void session_free(welvet_dense_session *s) {
   if (!s) return;
   if (s->stream) (void)hipStreamSynchronize(s->stream);
   free_store(&s->W);
-  if (s->d_x) (void)hipFree(s->d_x);
-  if (s->d_pre) (void)hipFree(s->d_pre);
-  if (s->d_post) (void)hipFree(s->d_post);
-  if (s->ws) (void)hipFree(s->ws);
-  if (s->d_flag) (void)hipFree(s->d_flag);
+  for (void *p : {(void *)s->d_x, (void *)s->d_pre, (void *)s->d_post, s->ws, (void *)s->d_flag}) {
+    if (p == nullptr) continue;
+    if (s->pooled) dev_free(p);
+    else (void)hipFree(p);
+  }
   if (s->stream) (void)hipStreamDestroy(s->stream);
   delete s;
 }
@@ -371,24 +377,29 @@ void session_free(welvet_dense_session *s) {
 welvet_status session_alloc_io(welvet_dense_session *s) {
   const size_t xb = (size_t)s->batch * s->W.cols * sizeof(float);
   const size_t yb = (size_t)s->batch * s->W.rows * sizeof(float);
-  WH_HIP(hipMalloc(&s->d_x, xb));
-  WH_HIP(hipMalloc(&s->d_pre, yb));
-  WH_HIP(hipMalloc(&s->d_post, yb));
-  WH_HIP(hipMalloc(&s->d_flag, 256));
+  WH_HIP(session_alloc(s, &s->d_x, xb));
+  WH_HIP(session_alloc(s, &s->d_pre, yb));
+  WH_HIP(session_alloc(s, &s->d_post, yb));
+  WH_HIP(session_alloc(s, &s->d_flag, 256));
   s->ws_bytes = forward_workspace_bytes(s->W.dev(), s->batch);
   const size_t mb = mse_workspace_bytes(0);
   if (s->ws_bytes < mb) s->ws_bytes = mb;
-  WH_HIP(hipMalloc(&s->ws, s->ws_bytes));
+  WH_HIP(session_alloc(s, &s->ws, s->ws_bytes));
   return ok();
 }
 
 welvet_status ensure_ws(welvet_dense_session *s, size_t bytes) {
   if (bytes <= s->ws_bytes) return ok();
-  // the old workspace may be in use on a caller's stream: drain the device
-  WH_HIP(hipDeviceSynchronize());
-  if (s->ws) WH_HIP(hipFree(s->ws));
+  if (s->pooled) {  // one call's own stream
+    WH_HIP(hipStreamSynchronize(s->stream));
+    dev_free(s->ws);
+  } else {
+    // the old workspace may be in use on a caller's stream: drain the device
+    WH_HIP(hipDeviceSynchronize());
+    if (s->ws) WH_HIP(hipFree(s->ws));
+  }
   s->ws = nullptr;
-  WH_HIP(hipMalloc(&s->ws, bytes));
+  WH_HIP(session_alloc(s, &s->ws, bytes));
   s->ws_bytes = bytes;
   return ok();
 }
@@ -452,7 +463,7 @@ struct WeightSource {
 // session_mount session.cpp:37-84 (dtype -> 2, dims/batch -> 1)
 welvet_status mount(int32_t batch, int32_t in, int32_t out, int32_t act, int32_t dtype,
                     const WeightSource &src, const double *bias, size_t bias_len,
-                    welvet_dense_session **sess) {
+                    welvet_dense_session **sess, bool pooled = false) {
   if (!sess || (src.kind == WeightSource::kNative ? !src.raw : !src.f32))
     return make_status(kInvalid, "invalid argument");
   if (dtype < 0 || dtype >= kNumDTypes)
@@ -464,6 +475,7 @@ welvet_status mount(int32_t batch, int32_t in, int32_t out, int32_t act, int32_t
   auto *s = new welvet_dense_session();
   s->batch = batch;
   s->act = act;
+  s->pooled = s->W.pooled = pooled;
   if (hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) != hipSuccess) {
     delete s;
     return make_status(kInternal, "hipStreamCreate failed");
@@ -497,31 +509,35 @@ welvet_status execute(welvet_dense_session *s, const float *x, float *pre, float
   const size_t xb = (size_t)s->batch * s->W.cols * sizeof(float);
   const size_t yb = (size_t)s->batch * s->W.rows * sizeof(float);
   WH_HIP(hipSetDevice(g_dev.id));
-  WH_HIP(hipMemcpyAsync(s->d_x, x, xb, hipMemcpyHostToDevice, s->stream));
+  WH_HIP(copy_to_device(s->d_x, x, xb, s->stream));
   welvet_status st = forward_device(s, s->d_x, s->d_pre, s->d_post, s->stream);
   if (st.code) return st;
-  WH_HIP(hipMemcpyAsync(pre, s->d_pre, yb, hipMemcpyDeviceToHost, s->stream));
-  WH_HIP(hipMemcpyAsync(post, s->d_post, yb, hipMemcpyDeviceToHost, s->stream));
+  WH_HIP(copy_to_host(pre, s->d_pre, yb, s->stream));
+  WH_HIP(copy_to_host(post, s->d_post, yb, s->stream));
   WH_HIP(hipStreamSynchronize(s->stream));
   return ok();
 }
 
-// Device buffers of one NormalBP / backward call.
+// Device buffers of one NormalBP / backward call on a session's stream.
 struct Bwd {
   float *gy = nullptr, *dpre = nullptr, *dX = nullptr, *dW = nullptr, *pre = nullptr;
   double *loss = nullptr;
+  hipStream_t stream;
+  explicit Bwd(hipStream_t s) : stream(s) {}
   ~Bwd() {
-    for (void *p : {(void *)gy, (void *)dpre, (void *)dX, (void *)dW, (void *)pre, (void *)loss})
-      if (p) (void)hipFree(p);
+    (void)hipStreamSynchronize(stream);
+    for (void *p : {(void *)gy, (void *)dpre, (void *)dX, (void *)dW, (void *)pre, (void *)loss}) dev_free(p);
   }
+  template <typename T>
+  hipError_t alloc(T **p, size_t bytes) { return dev_alloc((void **)p, bytes); }
 };
 
 welvet_status backward_device(welvet_dense_session *s, const float *d_x, const float *d_pre,
                               const float *d_gy, Bwd *b) {
   const int64_t ny = (int64_t)s->batch * s->W.rows, nx = (int64_t)s->batch * s->W.cols;
-  WH_HIP(hipMalloc(&b->dpre, ny * sizeof(float)));
-  WH_HIP(hipMalloc(&b->dX, nx * sizeof(float)));
-  WH_HIP(hipMalloc(&b->dW, s->W.n() * sizeof(float)));
+  WH_HIP(b->alloc(&b->dpre, ny * sizeof(float)));
+  WH_HIP(b->alloc(&b->dX, nx * sizeof(float)));
+  WH_HIP(b->alloc(&b->dW, s->W.n() * sizeof(float)));
   welvet_status st = ensure_ws(s, backward_workspace_bytes(s->W.dev(), s->batch));
   if (st.code == 0) st = store_prepare_backward(&s->W, s->batch, s->stream);
   if (st.code) return st;
@@ -611,7 +627,7 @@ welvet_status welvet_dense_forward_f32(int32_t batch, int32_t in, int32_t out, i
   welvet_dense_session *s = nullptr;
   WeightSource src;
   src.f32 = W_init;
-  welvet_status st = mount(batch, in, out, act, dtype, src, bias, bias_len, &s);
+  welvet_status st = mount(batch, in, out, act, dtype, src, bias, bias_len, &s, true);
   if (st.code) return st;
   st = execute(s, x, pre, post);
   session_free(s);
@@ -631,30 +647,27 @@ welvet_status welvet_dense_normalbp_f32(int32_t batch, int32_t in, int32_t out, 
   welvet_dense_session *s = nullptr;
   WeightSource src;
   src.f32 = W_init;
-  welvet_status st = mount(batch, in, out, act, dtype, src, bias, bias_len, &s);
+  welvet_status st = mount(batch, in, out, act, dtype, src, bias, bias_len, &s, true);
   if (st.code) return st;
   const int64_t ny = (int64_t)batch * out, nx = (int64_t)batch * in, nw = (int64_t)out * in;
   hipStream_t strm = s->stream;
-  Bwd b;
   auto run = [&]() -> welvet_status {
-    WH_HIP(hipMemcpyAsync(s->d_x, x, nx * sizeof(float), hipMemcpyHostToDevice, strm));
+    Bwd b(strm);
+    WH_HIP(copy_to_device(s->d_x, x, nx * sizeof(float), strm));
     st = forward_device(s, s->d_x, s->d_pre, s->d_post, strm);
     if (st.code) return st;
-    WH_HIP(hipMalloc(&b.gy, ny * sizeof(float)));
-    WH_HIP(hipMalloc(&b.loss, sizeof(double)));
+    WH_HIP(b.alloc(&b.gy, ny * sizeof(float)));
+    WH_HIP(b.alloc(&b.loss, sizeof(double)));
     double h_loss = 0.0;
     if (use_target) {
-      float *d_t = nullptr;
-      WH_HIP(hipMalloc(&d_t, ny * sizeof(float)));
-      hipError_t e = hipMemcpyAsync(d_t, grad_or_target, ny * sizeof(float), hipMemcpyHostToDevice, strm);
-      if (e == hipSuccess)
-        e = launch_mse(s->d_post, d_t, ny, b.loss, b.gy, s->ws, s->ws_bytes, strm);
-      if (e == hipSuccess) e = hipMemcpyAsync(&h_loss, b.loss, sizeof(double), hipMemcpyDeviceToHost, strm);
-      if (e == hipSuccess) e = hipStreamSynchronize(strm);
-      (void)hipFree(d_t);
-      WH_HIP(e);
+      DevBuf t(strm);
+      WH_HIP(t.alloc(ny * sizeof(float)));
+      WH_HIP(copy_to_device(t.p, grad_or_target, ny * sizeof(float), strm));
+      WH_HIP(launch_mse(s->d_post, t.as<float>(), ny, b.loss, b.gy, s->ws, s->ws_bytes, strm));
+      WH_HIP(hipMemcpyAsync(&h_loss, b.loss, sizeof(double), hipMemcpyDeviceToHost, strm));
+      WH_HIP(hipStreamSynchronize(strm));
     } else {
-      WH_HIP(hipMemcpyAsync(b.gy, grad_or_target, ny * sizeof(float), hipMemcpyHostToDevice, strm));
+      WH_HIP(copy_to_device(b.gy, grad_or_target, ny * sizeof(float), strm));
     }
     st = backward_device(s, s->d_x, s->d_pre, b.gy, &b);
     if (st.code) return st;
@@ -662,19 +675,15 @@ welvet_status welvet_dense_normalbp_f32(int32_t batch, int32_t in, int32_t out, 
       st = store_sgd(&s->W, b.dW, lr, s->d_flag, strm);
       if (st.code) return st;
     }
-    float *d_after = nullptr;
-    WH_HIP(hipMalloc(&d_after, nw * sizeof(float)));
-    st = store_export(s->W, d_after, strm);
-    hipError_t e = st.code ? hipSuccess
-                           : hipMemcpyAsync(W_after, d_after, nw * sizeof(float), hipMemcpyDeviceToHost, strm);
-    if (e == hipSuccess) e = hipStreamSynchronize(strm);
-    (void)hipFree(d_after);
+    DevBuf after(strm);
+    WH_HIP(after.alloc(nw * sizeof(float)));
+    st = store_export(s->W, after.as<float>(), strm);
     if (st.code) return st;
-    WH_HIP(e);
-    WH_HIP(hipMemcpyAsync(pre, s->d_pre, ny * sizeof(float), hipMemcpyDeviceToHost, strm));
-    WH_HIP(hipMemcpyAsync(post, s->d_post, ny * sizeof(float), hipMemcpyDeviceToHost, strm));
-    WH_HIP(hipMemcpyAsync(dX, b.dX, nx * sizeof(float), hipMemcpyDeviceToHost, strm));
-    WH_HIP(hipMemcpyAsync(dW, b.dW, nw * sizeof(float), hipMemcpyDeviceToHost, strm));
+    WH_HIP(copy_to_host(W_after, after.p, nw * sizeof(float), strm));
+    WH_HIP(copy_to_host(pre, s->d_pre, ny * sizeof(float), strm));
+    WH_HIP(copy_to_host(post, s->d_post, ny * sizeof(float), strm));
+    WH_HIP(copy_to_host(dX, b.dX, nx * sizeof(float), strm));
+    WH_HIP(copy_to_host(dW, b.dW, nw * sizeof(float), strm));
     WH_HIP(hipStreamSynchronize(strm));
     *loss = h_loss;
     return ok();
@@ -701,7 +710,7 @@ welvet_status welvet_hip_dense_forward_noalloc(welvet_dense_session *s, int32_t 
   if (((uintptr_t)d_x | (uintptr_t)d_pre | (uintptr_t)d_post) & 15)
     return make_status(kInvalid, "device pointers must be 16-byte aligned");
   if (batch <= 0) return make_status(kInvalid, "bad batch %d", batch);
-  const size_t need = forward_workspace_bytes(s->W.dev(), batch);
+  const size_t need = forward_workspace_min_bytes(s->W.dev(), batch);
   if (need > kScratchBytes)
     return make_status(kInvalid, "no-allocation forward: batch %d needs %zu bytes of scratch (limit %zu)",
                        batch, need, kScratchBytes);
@@ -740,14 +749,12 @@ welvet_status welvet_hip_dense_export_f32(welvet_dense_session *s, float *W_out)
   if (!s || !W_out) return make_status(kInvalid, "weights: nil dst");
   std::lock_guard<std::mutex> lock(s->mu);
   const size_t bytes = (size_t)s->W.n() * sizeof(float);
-  float *d = nullptr;
-  WH_HIP(hipMalloc(&d, bytes));
-  welvet_status st = store_export(s->W, d, s->stream);
-  hipError_t e = st.code ? hipSuccess : hipMemcpyAsync(W_out, d, bytes, hipMemcpyDeviceToHost, s->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-  (void)hipFree(d);
+  DevBuf d(s->stream);
+  WH_HIP(d.alloc(bytes));
+  const welvet_status st = store_export(s->W, d.as<float>(), s->stream);
   if (st.code) return st;
-  WH_HIP(e);
+  WH_HIP(copy_to_host(W_out, d.p, bytes, s->stream));
+  WH_HIP(hipStreamSynchronize(s->stream));
   return ok();
 }
 
@@ -756,16 +763,16 @@ welvet_status welvet_hip_dense_backward(welvet_dense_session *s, const float *x,
   if (!s || !x || !pre || !gy || !dX || !dW) return make_status(kInvalid, "null resident backward");
   std::lock_guard<std::mutex> lock(s->mu);
   const int64_t ny = (int64_t)s->batch * s->W.rows, nx = (int64_t)s->batch * s->W.cols;
-  Bwd b;
-  WH_HIP(hipMalloc(&b.gy, ny * sizeof(float)));
-  WH_HIP(hipMalloc(&b.pre, ny * sizeof(float)));
-  WH_HIP(hipMemcpyAsync(s->d_x, x, nx * sizeof(float), hipMemcpyHostToDevice, s->stream));
-  WH_HIP(hipMemcpyAsync(b.pre, pre, ny * sizeof(float), hipMemcpyHostToDevice, s->stream));
-  WH_HIP(hipMemcpyAsync(b.gy, gy, ny * sizeof(float), hipMemcpyHostToDevice, s->stream));
+  Bwd b(s->stream);
+  WH_HIP(b.alloc(&b.gy, ny * sizeof(float)));
+  WH_HIP(b.alloc(&b.pre, ny * sizeof(float)));
+  WH_HIP(copy_to_device(s->d_x, x, nx * sizeof(float), s->stream));
+  WH_HIP(copy_to_device(b.pre, pre, ny * sizeof(float), s->stream));
+  WH_HIP(copy_to_device(b.gy, gy, ny * sizeof(float), s->stream));
   welvet_status st = backward_device(s, s->d_x, b.pre, b.gy, &b);
   if (st.code) return st;
-  WH_HIP(hipMemcpyAsync(dX, b.dX, nx * sizeof(float), hipMemcpyDeviceToHost, s->stream));
-  WH_HIP(hipMemcpyAsync(dW, b.dW, s->W.n() * sizeof(float), hipMemcpyDeviceToHost, s->stream));
+  WH_HIP(copy_to_host(dX, b.dX, nx * sizeof(float), s->stream));
+  WH_HIP(copy_to_host(dW, b.dW, s->W.n() * sizeof(float), s->stream));
   WH_HIP(hipStreamSynchronize(s->stream));
   return ok();
 }
@@ -773,14 +780,12 @@ welvet_status welvet_hip_dense_backward(welvet_dense_session *s, const float *x,
 welvet_status welvet_hip_dense_sgd(welvet_dense_session *s, const float *dW, double lr) {
   if (!s || !dW) return make_status(kInvalid, "weights: bad SGD arguments");
   std::lock_guard<std::mutex> lock(s->mu);
-  float *d = nullptr;
+  DevBuf d(s->stream);
   const size_t bytes = (size_t)s->W.n() * sizeof(float);
-  WH_HIP(hipMalloc(&d, bytes));
-  hipError_t e = hipMemcpyAsync(d, dW, bytes, hipMemcpyHostToDevice, s->stream);
-  welvet_status st = e == hipSuccess ? store_sgd(&s->W, d, lr, s->d_flag, s->stream)
-                                     : make_status(kInternal, "hip: %s", hipGetErrorString(e));
+  WH_HIP(d.alloc(bytes));
+  WH_HIP(copy_to_device(d.p, dW, bytes, s->stream));
+  const welvet_status st = store_sgd(&s->W, d.as<float>(), lr, s->d_flag, s->stream);
   (void)hipStreamSynchronize(s->stream);
-  (void)hipFree(d);
   return st;
 }
 

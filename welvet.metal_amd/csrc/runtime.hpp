@@ -29,6 +29,30 @@ void device_init();
 bool device_ready();
 const char *device_identity();
 
+// ------------------------------------------------ host buffers (hostio.hpp)
+// hipMemcpyAsync between the device and host memory, pageable memory of 1 MB
+// and more through pinned slots on several threads (complete on return).  As
+// with hipMemcpyAsync, a host destination holds the data once `s` is synchronised.
+hipError_t copy_to_device(void *dst, const void *src, size_t bytes, hipStream_t s);
+hipError_t copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t s);
+// Device memory for one call's buffers, from a bounded pool of freed blocks.
+// dev_free: no work on the block may be in flight.
+hipError_t dev_alloc(void **p, size_t bytes);
+void dev_free(void *p);
+void dev_trim();  // gives every idle block back
+// A call's buffer, freed when `stream` has drained.
+struct DevBuf {
+  void *p = nullptr;
+  hipStream_t stream;
+  explicit DevBuf(hipStream_t s) : stream(s) {}
+  ~DevBuf();
+  DevBuf(const DevBuf &) = delete;
+  DevBuf &operator=(const DevBuf &) = delete;
+  hipError_t alloc(size_t bytes) { return dev_alloc(&p, bytes); }
+  template <typename T>
+  T *as() const { return (T *)p; }
+};
+
 // ------------------------------------------------------- resident store
 struct Store {
   int dtype = kFloat32, rows = 0, cols = 0;
@@ -43,6 +67,9 @@ struct Store {
   // no code decodes to Inf / NaN: found at encode (FP8 E5M2 can hold them),
   // cleared by an SGD step of a format that can produce them
   bool finite = true;
+  // the allocations come from dev_alloc (a store of one call, whose stream
+  // drains before free_store), else from hipMalloc
+  bool pooled = false;
   // transposed codes for dX on the split-x GEMM (tbody_ok: current with body)
   uint8_t *tbody = nullptr;
   bool tbody_ok = false;

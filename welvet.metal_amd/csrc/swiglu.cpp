@@ -143,10 +143,10 @@ welvet_status welvet_swiglu_forward_f32(int32_t batch, int32_t seq, int32_t inpu
   welvet_status st = make(&L, bs, input_dim, intermediate_dim, dtype, Gate, Up, Down);
   if (st.code) return st;
   const int64_t nh = (int64_t)bs * intermediate_dim, nx = (int64_t)bs * input_dim;
-  WH_HIP(hipMemcpyAsync(L.x, x, nx * sizeof(float), hipMemcpyHostToDevice, L.stream));
+  WH_HIP(copy_to_device(L.x, x, nx * sizeof(float), L.stream));
   if ((st = forward(&L)).code) return st;
-  WH_HIP(hipMemcpyAsync(pre, L.h, nh * sizeof(float), hipMemcpyDeviceToHost, L.stream));
-  WH_HIP(hipMemcpyAsync(post, L.d_post, nx * sizeof(float), hipMemcpyDeviceToHost, L.stream));
+  WH_HIP(copy_to_host(pre, L.h, nh * sizeof(float), L.stream));
+  WH_HIP(copy_to_host(post, L.d_post, nx * sizeof(float), L.stream));
   WH_HIP(hipStreamSynchronize(L.stream));
   return ok();
 }
@@ -167,7 +167,7 @@ welvet_status welvet_swiglu_normalbp_f32(int32_t batch, int32_t seq, int32_t inp
   if (st.code) return st;
   const hipStream_t s = L.stream;
   const int64_t nh = (int64_t)bs * inter, nx = (int64_t)bs * in, nw = (int64_t)inter * in;
-  WH_HIP(hipMemcpyAsync(L.x, x, nx * sizeof(float), hipMemcpyHostToDevice, s));
+  WH_HIP(copy_to_device(L.x, x, nx * sizeof(float), s));
   if ((st = forward(&L)).code) return st;
 
   // output gradient: the caller's, or the MSE gradient against the target
@@ -184,11 +184,11 @@ welvet_status welvet_swiglu_normalbp_f32(int32_t batch, int32_t seq, int32_t inp
   if (use_target) {
     float *d_t = nullptr;
     if ((st = L.alloc(&d_t, nx)).code) return st;
-    WH_HIP(hipMemcpyAsync(d_t, grad_or_target, nx * sizeof(float), hipMemcpyHostToDevice, s));
+    WH_HIP(copy_to_device(d_t, grad_or_target, nx * sizeof(float), s));
     WH_HIP(launch_mse(L.d_post, d_t, nx, d_loss, gy, L.ws, L.ws_bytes, s));
     WH_HIP(hipMemcpyAsync(&h_loss, d_loss, sizeof(double), hipMemcpyDeviceToHost, s));
   } else {
-    WH_HIP(hipMemcpyAsync(gy, grad_or_target, nx * sizeof(float), hipMemcpyHostToDevice, s));
+    WH_HIP(copy_to_device(gy, grad_or_target, nx * sizeof(float), s));
   }
 
   // swiglu::backward_f32: Down on h, op_swiglu, Gate and Up on x
@@ -214,11 +214,11 @@ welvet_status welvet_swiglu_normalbp_f32(int32_t batch, int32_t seq, int32_t inp
   if ((st = store_export(L.gate, w_after, s)).code) return st;
   if ((st = store_export(L.up, w_after + nw, s)).code) return st;
   if ((st = store_export(L.down, w_after + 2 * nw, s)).code) return st;
-  WH_HIP(hipMemcpyAsync(W_after, w_after, 3 * nw * sizeof(float), hipMemcpyDeviceToHost, s));
-  WH_HIP(hipMemcpyAsync(pre, L.h, nh * sizeof(float), hipMemcpyDeviceToHost, s));
-  WH_HIP(hipMemcpyAsync(post, L.d_post, nx * sizeof(float), hipMemcpyDeviceToHost, s));
-  WH_HIP(hipMemcpyAsync(dX, gx, nx * sizeof(float), hipMemcpyDeviceToHost, s));
-  WH_HIP(hipMemcpyAsync(dW, dw, 3 * nw * sizeof(float), hipMemcpyDeviceToHost, s));
+  WH_HIP(copy_to_host(W_after, w_after, 3 * nw * sizeof(float), s));
+  WH_HIP(copy_to_host(pre, L.h, nh * sizeof(float), s));
+  WH_HIP(copy_to_host(post, L.d_post, nx * sizeof(float), s));
+  WH_HIP(copy_to_host(dX, gx, nx * sizeof(float), s));
+  WH_HIP(copy_to_host(dW, dw, 3 * nw * sizeof(float), s));
   WH_HIP(hipStreamSynchronize(s));
   *loss = h_loss;
   return ok();

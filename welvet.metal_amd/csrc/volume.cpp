@@ -691,8 +691,7 @@ welvet_status welvet_hip_grid_export_f32(welvet_hip_grid *g, int32_t z, int32_t 
   WH_HIP(hipMalloc(&d, (size_t)c->W.n() * sizeof(float)));
   st = store_export(c->W, d, g->stream);
   hipError_t e = hipSuccess;
-  if (st.code == 0) e = hipMemcpyAsync(W_out, d, (size_t)c->W.n() * sizeof(float),
-                                       hipMemcpyDeviceToHost, g->stream);
+  if (st.code == 0) e = copy_to_host(W_out, d, (size_t)c->W.n() * sizeof(float), g->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(g->stream);
   (void)hipFree(d);
   if (st.code) return st;

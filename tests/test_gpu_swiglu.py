@@ -211,3 +211,32 @@ def test_resident_session_matches_one_shot():
             hip.hipFree(p)
     np.testing.assert_array_equal(h, pre)
     np.testing.assert_array_equal(y, post)
+
+
+@pytest.mark.parametrize("dtype", [4, 5, 9, 14, 16, 26], ids=[pywelvet.DTYPE_NAMES[d] for d in (4, 5, 9, 14, 16, 26)])
+@pytest.mark.parametrize("rows,inn,inter", [(5, 4096, 300), (16, 2112, 257), (17, 96, 1000), (40, 640, 384), (70, 512, 1030)])
+def test_gate_and_up_in_one_launch(oracle, dtype, rows, inn, inter):
+    """Gate and Up as one split-x GEMM launch with one reduction (16-, 32- and
+    64-row tiles, ragged outputs): h and post against the f64 products of the
+    decoded weights.  g and u carry a product's 1e-5; h = silu(g) u at most
+    their sum (|silu'| <= 1.1), post one product more."""
+    rng = np.random.default_rng(rows + inn + dtype)
+    scale = 2.0 if dtype == 16 else 0.5 / np.sqrt(inn)
+    G, U = (rng.normal(0, scale, (inter, inn)).astype(np.float32) for _ in range(2))
+    D = rng.normal(0, scale, (inn, inter)).astype(np.float32)
+    x = rng.normal(0, 0.05 if dtype == 16 else 1.0, (rows, inn)).astype(np.float32)
+    pre, post = pywelvet.swiglu_forward(G, U, D, x, dtype=dtype)
+
+    def decoded(W):
+        raw, s = oracle.pack(dtype, W)
+        return oracle.decode_f64(dtype, raw, s, W.size).reshape(W.shape)
+
+    Gd, Ud, Dd = decoded(G), decoded(U), decoded(D)
+    xd = x.astype(np.float64)
+    g, u = xd @ Gd.T, xd @ Ud.T
+    sg = g / (1 + np.exp(-g))
+    ref = sg * u
+    tol_g, tol_u = (1e-5 * (np.abs(xd) @ np.abs(W).T) for W in (Gd, Ud))
+    tol_h = 1.2 * tol_g * (np.abs(u) + tol_u) + np.abs(sg) * tol_u + 1e-6 * np.abs(ref) + 1e-30
+    assert np.all(np.abs(pre - ref) <= tol_h)
+    assert np.all(np.abs(post - ref @ Dd.T) <= tol_h @ np.abs(Dd).T + 1e-5 * (np.abs(ref) @ np.abs(Dd).T) + 1e-30)

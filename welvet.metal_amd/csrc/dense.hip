@@ -780,6 +780,10 @@ struct GemmArgs {
   // the reduction multiplies sums by post (a per-tensor scale the split-x
   // GEMM factors out of the weights)
   float post = 1.0f;
+  // a second store's product with the same x in the same launch (grid y = 1):
+  // its body, and its partial tiles this many floats into ws
+  const uint8_t *body2 = nullptr;
+  int64_t ws2 = 0;
 };
 
 // Split-x kinds from BK_B16 on: the kind for the reduction's recomputation of
@@ -1635,8 +1639,17 @@ __device__ inline void bf3_weights(const uint32_t *w, int q, const uint2 *t3, fl
   }
 }
 
+// Blocks of grid row 1 work on the second store.
+__device__ inline void take_pair(GemmArgs &a) {
+  if (blockIdx.y != 0) {
+    a.body = a.body2;
+    a.ws += a.ws2;
+  }
+}
+
 template <int BK, int MT, int D, int NC>
 __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
+  take_pair(a);
   using K3 = B3<BK>;
   constexpr int BM = 32 * MT, BN = 128 * NC, NW = K3::kWords, NP = K3::kParts;
   constexpr int XE = BM * kBK / 256;  // x values per thread per stage (8 or 16)
@@ -1836,6 +1849,7 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
 // writes half the partial tiles.  GemmArgs::nst counts stage pairs here.
 template <int BK, int MT, int D, int NC>
 __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
+  take_pair(a);
   using K3 = B3<BK>;
   constexpr int BM = 32 * MT, BN = 128 * NC, NW = K3::kWords, NP = K3::kParts;
   constexpr int XE = BM * kBK / 256;  // x values per thread per stage (8 or 16)
@@ -2064,6 +2078,7 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // 4 g .. 4 g + 3.
 template <int BK, int D, int NC>
 __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
+  take_pair(a);
   using K3 = B3<BK>;
   constexpr int BM = 16, BN = 128 * NC, NW = K3::kWords / 2, NP = K3::kParts;
   constexpr int CG = 2 * NC;          // 16-column groups per wave
@@ -2465,6 +2480,65 @@ __global__ void __launch_bounds__(256) sk_reduce_kernel(GemmArgs a, const double
   }
 }
 
+// The reduction of a pair launch: g and u are the two stores' products (each
+// as sk_reduce_kernel sums one), h = fl32(silu(g)) * u, op_swiglu's product.
+__global__ void __launch_bounds__(256) sk_reduce_pair_kernel(GemmArgs a, float post2, float *g_pre, float *u_pre,
+                                                             float *h) {
+  const int t = blockIdx.x;
+  const int b0 = (int)((int64_t)t * a.nst / a.per_block);
+  const int b1 = (int)(((int64_t)(t + 1) * a.nst - 1) / a.per_block);
+  const int tile = a.bm * a.bn;
+  const int off = (blockIdx.y * 256 + threadIdx.x) * 4;
+  if (off >= tile) return;
+  const int m = (t / a.gx) * a.bm + off / a.bn, n = (t % a.gx) * a.bn + off % a.bn;
+  if (m >= a.M) return;
+  double sum[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+  for (int g = b0; g <= b1; g += 4) {
+    float4 v[2][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int b = g + i;
+      if (b <= b1) {
+        const int slot = t - (int)((int64_t)b * a.per_block / a.nst);
+        const float *src = a.ws + ((int64_t)b * a.maxspan + slot) * tile + off;
+        v[0][i] = *(const float4 *)src;
+        v[1][i] = *(const float4 *)(src + a.ws2);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (g + i <= b1) {
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          sum[w][0] += (double)v[w][i].x;
+          sum[w][1] += (double)v[w][i].y;
+          sum[w][2] += (double)v[w][i].z;
+          sum[w][3] += (double)v[w][i].w;
+        }
+      }
+  }
+  float gv[4], uv[4], hv[4];
+  const int nv = min(4, a.N - n);
+  const int64_t idx = (int64_t)m * a.N + n;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    gv[i] = (float)(sum[0][i] * (double)a.post);
+    uv[i] = (float)(sum[1][i] * (double)post2);
+    hv[i] = i < nv ? act_value(gv[i], kSilu) * uv[i] : 0.0f;
+  }
+  if (nv == 4 && (a.N & 3) == 0) {
+    *(float4 *)(g_pre + idx) = make_float4(gv[0], gv[1], gv[2], gv[3]);
+    *(float4 *)(u_pre + idx) = make_float4(uv[0], uv[1], uv[2], uv[3]);
+    *(float4 *)(h + idx) = make_float4(hv[0], hv[1], hv[2], hv[3]);
+  } else {
+    for (int i = 0; i < nv; ++i) {
+      g_pre[idx + i] = gv[i];
+      u_pre[idx + i] = uv[i];
+      h[idx + i] = hv[i];
+    }
+  }
+}
+
 // out[m] = sum over k of A [m][k], f64.
 __global__ void __launch_bounds__(256) rowsum_kernel(const float *__restrict__ A, int K, double *out) {
   __shared__ double red[4];
@@ -2777,8 +2851,11 @@ __global__ void __launch_bounds__(256) dw_mfma_lds_kernel(const float *__restric
 }
 
 // The dW of up to kDwBatch layers in one launch (blockIdx.z = layer; the
-// grid covers the largest layer, blocks past a smaller one's tiles exit).
-__global__ void __launch_bounds__(256) dw_batch_kernel(DwBatch b) {
+// grid covers the largest layer, blocks past a smaller one's tiles exit).  Four
+// blocks per CU (128 registers) instead of three: 16 layers of 1024^2 at batch
+// 16, bound by the 67 MB of stores, 17.3 -> 16.0 us; a large layer's long MFMA
+// chains (2048 x 8192, b256) lose by it (81 -> 84) and keep three.
+__global__ void __launch_bounds__(256, 4) dw_batch_kernel(DwBatch b) {
   const int l = blockIdx.z;
   if (l >= b.count) return;
   const DwJob &t = b.job[l];
@@ -2918,9 +2995,10 @@ struct SkPlan {
 };
 
 // Stream-K split of an M x N x K product over bm x bn tiles into equal
-// shares, `occ` workgroups per CU; units of `kg` consecutive k stages (the
+// shares, `occ` workgroups per CU (of 1 / `share` of the CUs, where as many
+// products share a launch); units of `kg` consecutive k stages (the
 // caller makes the stage count a multiple of kg).
-SkPlan plan_sk(int M, int K, int N, int bm = kBM, int bn = kBN, int occ = 2, int kg = 1) {
+SkPlan plan_sk(int M, int K, int N, int bm = kBM, int bn = kBN, int occ = 2, int kg = 1, int share = 1) {
   SkPlan p;
   p.bm = bm;
   p.bn = bn;
@@ -2929,7 +3007,7 @@ SkPlan plan_sk(int M, int K, int N, int bm = kBM, int bn = kBN, int occ = 2, int
   p.gy = (M + bm - 1) / bm;
   p.nst = (K + kBK - 1) / kBK / kg;
   const int64_t T = (int64_t)p.gx * p.gy * p.nst;
-  const int64_t G = (int64_t)occ * num_cus();
+  const int64_t G = std::max<int64_t>(1, (int64_t)occ * num_cus() / share);
   // at most 16 partial tiles per tile: past that the reduction's serial sum
   // costs more than the shorter shares save (FP8 32 x 128 tiles, 4096 -> 512
   // b48 19.2 -> 11.7 us, 8192 -> 300 b24 28.0 -> 15.0, 1024^2 b100 11.9 ->
@@ -2948,12 +3026,17 @@ dim3 sk_reduce_grid(const SkPlan &p) {
 bool reg_gemm_ok(int f) { return f >= 0 && fmt_chunk_elems(f) >= 8; }  // formats of <= 16 bits
 
 
+// The factor the reduction applies for a kind whose codes carry no scale.
+float bf3_post(const DevStore &w, int bk) {
+  return (bk == BK_I8 || bk == BK_NF4 || bk == BK_U8) ? w.scale : bk == BK_I4 ? w.scale * 0.0625f : 1.0f;
+}
+
 // Row sums of x for Uint8 on the split-x GEMM, at the end of the workspace.
 size_t rowsum_bytes(int M) { return ((size_t)M * sizeof(double) + 15) / 16 * 16; }
 
 // Forward GEMM plan: the split-x bf16 kernel for the formats it takes, the
 // register-B kernel for other <= 16-bit formats, else the LDS-staged kernel.
-SkPlan plan_fwd_gemm(int f, int bk, int M, int K, int N) {
+SkPlan plan_fwd_gemm(int f, int bk, int M, int K, int N, int share = 1) {
   if (bk >= 0) {
     const int occ = 2;
     const int stages = (K + kBK - 1) / kBK;
@@ -3006,8 +3089,8 @@ SkPlan plan_fwd_gemm(int f, int bk, int M, int K, int N) {
     // batch 32 and, up to it, those of the 4-bit kinds (FP8 / Int8 measured
     // slower there)
     const bool groups = bn == 256 && stages % 2 == 0 && (bm == 64 || (bm == 32 && (M > 32 || four_bit)));
-    SkPlan p = groups ? plan_sk(M, K, N, bm, bn, 1, 2)
-                      : plan_sk(M, K, N, bm, bn, occ);
+    SkPlan p = groups ? plan_sk(M, K, N, bm, bn, 1, 2, share)
+                      : plan_sk(M, K, N, bm, bn, occ, 1, share);
     p.bf3 = true;
     if (bk == BK_U8) p.ws_bytes += rowsum_bytes(M);
     return p;
@@ -3186,22 +3269,23 @@ hipError_t launch_bf3r(const SkPlan &p, int bk, const GemmArgs &a, const double 
 
 // The split-x GEMM of plan p for weight kind bk (a.body, a.post set).
 hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
+  const dim3 grid(p.blocks, a.body2 != nullptr ? 2 : 1);
 #define WH_GB(BK)                                                                     \
   if (p.bm == 16) {                                                                   \
-    if (p.bn == 128) gemm_bf3s_kernel<BK, 1, 1><<<p.blocks, 256, 0, s>>>(a);           \
-    else gemm_bf3s_kernel<BK, 1, 2><<<p.blocks, 256, 0, s>>>(a);                       \
+    if (p.bn == 128) gemm_bf3s_kernel<BK, 1, 1><<<grid, 256, 0, s>>>(a);           \
+    else gemm_bf3s_kernel<BK, 1, 2><<<grid, 256, 0, s>>>(a);                       \
   } else if (p.bm == 32) {                                                            \
-    if (p.bn == 128) gemm_bf3_kernel<BK, 1, 1, 1><<<p.blocks, 256, 0, s>>>(a);         \
-    else gemm_bf3_kernel<BK, 1, 1, 2><<<p.blocks, 256, 0, s>>>(a);                     \
+    if (p.bn == 128) gemm_bf3_kernel<BK, 1, 1, 1><<<grid, 256, 0, s>>>(a);         \
+    else gemm_bf3_kernel<BK, 1, 1, 2><<<grid, 256, 0, s>>>(a);                     \
   } else {                                                                            \
-    if (p.bn == 128) gemm_bf3_kernel<BK, 2, 1, 1><<<p.blocks, 256, 0, s>>>(a);         \
-    else gemm_bf3_kernel<BK, 2, 1, 2><<<p.blocks, 256, 0, s>>>(a);                     \
+    if (p.bn == 128) gemm_bf3_kernel<BK, 2, 1, 1><<<grid, 256, 0, s>>>(a);         \
+    else gemm_bf3_kernel<BK, 2, 1, 2><<<grid, 256, 0, s>>>(a);                     \
   }
   if (p.rows) return hipErrorInvalidValue;  // launched with its epilogue by the caller
   if (p.kg == 2) {  // two wave groups, a ring two units deep
 #define WH_GK(BK)                                                                             \
-  if (p.bm == 32) gemm_bf3k_kernel<BK, 1, 2, 2><<<p.blocks, 512, 0, s>>>(a);                  \
-  else gemm_bf3k_kernel<BK, 2, 2, 2><<<p.blocks, 512, 0, s>>>(a);
+  if (p.bm == 32) gemm_bf3k_kernel<BK, 1, 2, 2><<<grid, 512, 0, s>>>(a);                  \
+  else gemm_bf3k_kernel<BK, 2, 2, 2><<<grid, 512, 0, s>>>(a);
     switch (bk) {
     case BK_B16: WH_GK(BK_B16) break;
     case BK_H16: WH_GK(BK_H16) break;
@@ -3219,19 +3303,19 @@ hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
   }
 #define WH_GB32(BK)  /* batches above 16 only */                                      \
   if (p.bm == 32) {                                                                   \
-    if (p.bn == 128) gemm_bf3_kernel<BK, 1, 1, 1><<<p.blocks, 256, 0, s>>>(a);         \
-    else gemm_bf3_kernel<BK, 1, 1, 2><<<p.blocks, 256, 0, s>>>(a);                     \
+    if (p.bn == 128) gemm_bf3_kernel<BK, 1, 1, 1><<<grid, 256, 0, s>>>(a);         \
+    else gemm_bf3_kernel<BK, 1, 1, 2><<<grid, 256, 0, s>>>(a);                     \
   } else {                                                                            \
-    if (p.bn == 128) gemm_bf3_kernel<BK, 2, 1, 1><<<p.blocks, 256, 0, s>>>(a);         \
-    else gemm_bf3_kernel<BK, 2, 1, 2><<<p.blocks, 256, 0, s>>>(a);                     \
+    if (p.bn == 128) gemm_bf3_kernel<BK, 2, 1, 1><<<grid, 256, 0, s>>>(a);         \
+    else gemm_bf3_kernel<BK, 2, 1, 2><<<grid, 256, 0, s>>>(a);                     \
   }
   switch (bk) {
   case BK_B16: WH_GB32(BK_B16) break;
   case BK_H16: WH_GB32(BK_H16) break;
   case BK_F32:  // 128-column tiles only (plan_fwd_gemm)
     if (p.bn != 128) return hipErrorInvalidValue;
-    if (p.bm == 32) gemm_bf3_kernel<BK_F32, 1, 1, 1><<<p.blocks, 256, 0, s>>>(a);
-    else gemm_bf3_kernel<BK_F32, 2, 1, 1><<<p.blocks, 256, 0, s>>>(a);
+    if (p.bm == 32) gemm_bf3_kernel<BK_F32, 1, 1, 1><<<grid, 256, 0, s>>>(a);
+    else gemm_bf3_kernel<BK_F32, 2, 1, 1><<<grid, 256, 0, s>>>(a);
     break;
   case BK_I4: WH_GB32(BK_I4) break;
   case BK_U8: WH_GB32(BK_U8) break;
@@ -3481,7 +3565,7 @@ hipError_t launch_forward(const DevStore &w, int batch, const float *x, const do
              p.gx, p.gy, p.nst, p.per_block, p.maxspan, (float *)ws, p.bm, p.bn};
   SplitFix fx;
   if (p.bf3) {
-    a.post = (bk == BK_I8 || bk == BK_NF4 || bk == BK_U8) ? w.scale : bk == BK_I4 ? w.scale * 0.0625f : 1.0f;
+    a.post = bf3_post(w, bk);
     if (bk == BK_E4 || bk == BK_E5) a.body = w.kbody;
     if (bk == BK_B16 || bk == BK_H16 || bk == BK_F32 || bk == BK_U8) fx.kind = bk;
     if (bk == BK_U8) {
@@ -3524,6 +3608,43 @@ hipError_t launch_forward(const DevStore &w, int batch, const float *x, const do
     sk_reduce_kernel<true, true><<<sk_reduce_grid(p), 256, 0, s>>>(a, bias, bias_len, act, pre, post, nullptr, fx);
   else
     sk_reduce_kernel<true><<<sk_reduce_grid(p), 256, 0, s>>>(a, bias, bias_len, act, pre, post, nullptr, fx);
+  return hipGetLastError();
+}
+
+namespace {
+// The plan of a pair launch on the split-x GEMM, each store on half the CUs
+// (half the partial tiles of a launch of its own); false where the batch
+// takes another route or the kind's reduction does more than add.
+bool pair_gemm_plan(const DevStore &g, const DevStore &u, int batch, int &bk, SkPlan &p) {
+  if (g.dtype != u.dtype || g.rows != u.rows || g.cols != u.cols || fwd_route(g, batch) != 2) return false;
+  bk = bf3_fwd_kind(g, batch);
+  if (bk < 0 || bk != bf3_fwd_kind(u, batch) || (bk >= BK_B16 && bk != BK_I4)) return false;
+  p = plan_fwd_gemm(kernel_fmt(g.dtype), bk, batch, g.cols, g.rows, 2);
+  return p.bf3 && !p.rows;
+}
+}  // namespace
+
+size_t forward_pair_gemm_bytes(const DevStore &g, const DevStore &u, int batch) {
+  int bk;
+  SkPlan p;
+  return pair_gemm_plan(g, u, batch, bk, p) ? 2 * p.ws_bytes : 0;
+}
+
+hipError_t launch_forward_pair_gemm(const DevStore &g, const DevStore &u, int batch, const float *x, float *g_pre,
+                                    float *u_pre, float *h, void *ws, size_t ws_bytes, hipStream_t s) {
+  int bk;
+  SkPlan p;
+  if (!pair_gemm_plan(g, u, batch, bk, p) || ws_bytes < 2 * p.ws_bytes) return hipErrorInvalidValue;
+  const bool ready = bk == BK_E4 || bk == BK_E5;
+  GemmArgs a{ready ? g.kbody : g.body, g.lut, g.scale, g.minv, x, batch, g.cols, g.rows, row_bytes_of(g),
+             p.gx, p.gy, p.nst, p.per_block, p.maxspan, (float *)ws, p.bm, p.bn};
+  a.post = bf3_post(g, bk);
+  a.body2 = ready ? u.kbody : u.body;
+  a.ws2 = (int64_t)(p.ws_bytes / sizeof(float));
+  if (a.body == nullptr || a.body2 == nullptr) return hipErrorInvalidValue;
+  const hipError_t e = launch_bf3(p, bk, a, s);
+  if (e != hipSuccess) return e;
+  sk_reduce_pair_kernel<<<sk_reduce_grid(p), 256, 0, s>>>(a, bf3_post(u, bk), g_pre, u_pre, h);
   return hipGetLastError();
 }
 

@@ -112,6 +112,12 @@ hipError_t launch_ragged_dx(const DevStore &w, int batch, const float *dpre, flo
 bool forward_pair_fits(const DevStore &g, const DevStore &u, int batch);
 hipError_t launch_forward_pair(const DevStore &g, const DevStore &u, const float *x, float *g_pre,
                                float *u_pre, float *h, hipStream_t s);
+// The same at a batch that the split-x GEMM takes: both products in one launch
+// (grid y = store) and one reduction that writes g, u and h.  The workspace it
+// needs, 0 where it does not apply.
+size_t forward_pair_gemm_bytes(const DevStore &g, const DevStore &u, int batch);
+hipError_t launch_forward_pair_gemm(const DevStore &g, const DevStore &u, int batch, const float *x, float *g_pre,
+                                    float *u_pre, float *h, void *ws, size_t ws_bytes, hipStream_t s);
 // out[c][r] = in[r][c] for a rows x cols byte matrix.
 hipError_t launch_transpose_u8(const uint8_t *in, int rows, int cols, uint8_t *out, hipStream_t s);
 // True when launch_backward's dX would use the store's transposed codes

@@ -100,6 +100,7 @@ welvet_status make(Swiglu *L, int bs, int in, int inter, int dtype, const float 
   for (const Store *w : {&L->gate, &L->up, &L->down})
     need = std::max({need, forward_workspace_bytes(w->dev(), bs), backward_workspace_bytes(w->dev(), bs),
                      mse_workspace_bytes(nx)});
+  need = std::max(need, forward_pair_gemm_bytes(L->gate.dev(), L->up.dev(), bs));
   return L->grow_ws(need);
 }
 
@@ -109,10 +110,15 @@ welvet_status make(Swiglu *L, int bs, int in, int inter, int dtype, const float 
 // element into fl32(silu(g)) * u, op_swiglu's product, and keeps u in u_pre
 // (Linear: post = pre); then Down on h.
 // At batch 1 both projections run as one launch (x read once per block, the
-// product in its epilogue).
+// product in its epilogue); on the split-x GEMM also one launch and one
+// reduction, which writes g, u and h.
 welvet_status forward(Swiglu *L, const float *x, float *h, float *post, hipStream_t s) {
   if (forward_pair_fits(L->gate.dev(), L->up.dev(), L->bs)) {
     WH_HIP(launch_forward_pair(L->gate.dev(), L->up.dev(), x, L->g_pre, L->u_pre, h, s));
+  } else if (const size_t pair = forward_pair_gemm_bytes(L->gate.dev(), L->up.dev(), L->bs);
+             pair > 0 && pair <= L->ws_bytes) {
+    WH_HIP(launch_forward_pair_gemm(L->gate.dev(), L->up.dev(), L->bs, x, L->g_pre, L->u_pre, h, L->ws, L->ws_bytes,
+                                    s));
   } else {
     WH_HIP(launch_forward(L->gate.dev(), L->bs, x, nullptr, 0, kLinear, L->g_pre, h, L->ws, L->ws_bytes, s));
     WH_HIP(launch_forward(L->up.dev(), L->bs, x, nullptr, 0, kSwiGated, L->u_pre, h, L->ws, L->ws_bytes, s));

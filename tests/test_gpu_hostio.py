@@ -18,7 +18,7 @@ def device():
     pywelvet.init()
 
 
-@pytest.mark.parametrize("n", [1, MB - 1, MB, MB + 1, 2 * MB + 3, 5 * MB + 1023, 17 * MB + 1])
+@pytest.mark.parametrize("n", [1, MB - 1, MB, MB + 1, 2 * MB + 3, 5 * MB + 1023, 8 * MB, 17 * MB + 1, 33 * MB + 5])
 def test_copies_are_whole(n):
     """A Float32 store takes its values and gives them back bit for bit."""
     rng = np.random.default_rng(n)

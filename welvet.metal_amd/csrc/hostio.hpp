@@ -26,8 +26,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
+#include <new>
 #include <thread>
 #include <unordered_map>
 #include <vector>
@@ -92,7 +93,9 @@ void give_slot(Slot s) {
   free_slot(s);
 }
 
-// Pieces of a staged copy, taken in turn by every thread that works on it.
+// Pieces of a staged copy, taken in turn by every thread that works on it.  A
+// thread that gets no slot takes none: what no thread took (`next`) is left to
+// the caller.
 struct Staged {
   char *host;
   char *dev;
@@ -106,9 +109,12 @@ struct Staged {
   void work() {
     hipError_t e = hipSetDevice(device);
     Slot s;
-    if (e == hipSuccess) e = take_slot(&s);
     if (e != hipSuccess) {
       error = e;
+      return;
+    }
+    if (take_slot(&s) != hipSuccess) {
+      (void)hipGetLastError();  // no pinned memory must not read as a failed launch
       return;
     }
     for (size_t at = next.fetch_add(piece); at < bytes && error == hipSuccess; at = next.fetch_add(piece)) {
@@ -124,6 +130,7 @@ struct Staged {
       }
       if (!up) std::memcpy(host + at, s.mem, n);
     }
+    if (error != hipSuccess) (void)hipStreamSynchronize(stream);  // a slot goes back with no copy on it
     give_slot(s);
   }
 };
@@ -157,11 +164,15 @@ hipError_t staged_copy(void *host, void *dev, size_t bytes, bool up, hipStream_t
   int started = 0;
   try {
     for (; started < threads - 1; ++started) team[started] = std::thread([&c] { c.work(); });
-  } catch (const std::system_error &) {  // no more threads: those there are do it
+  } catch (const std::exception &) {  // no more threads (or memory for one): those there are do it
   }
   c.work();
   for (int i = 0; i < started; ++i) team[i].join();
-  return (hipError_t)c.error.load();
+  if (c.error != hipSuccess) return (hipError_t)c.error.load();
+  const size_t at = c.next;
+  if (at >= bytes) return hipSuccess;
+  return up ? hipMemcpyAsync(c.dev + at, c.host + at, bytes - at, hipMemcpyHostToDevice, s)
+            : hipMemcpyAsync(c.host + at, c.dev + at, bytes - at, hipMemcpyDeviceToHost, s);
 }
 
 }  // namespace
@@ -184,11 +195,12 @@ constexpr size_t kPoolBytes = size_t(256) << 20;
 struct Block {
   void *p;
   size_t bytes;
+  int device;
 };
 struct DevPool {
   std::mutex mu;
   std::vector<Block> idle;
-  std::unordered_map<void *, size_t> out;  // blocks handed out
+  std::unordered_map<void *, Block> out;  // blocks handed out
   size_t kept = 0;
 };
 DevPool &pool() {
@@ -202,16 +214,19 @@ hipError_t dev_alloc(void **p, size_t bytes) try {
   DevPool &d = pool();
   bytes = (std::max<size_t>(bytes, 1) + 4095) / 4096 * 4096;
   *p = nullptr;
+  int device = 0;
+  hipError_t e = hipGetDevice(&device);
+  if (e != hipSuccess) return e;
   {
     std::lock_guard<std::mutex> lk(d.mu);
     size_t best = d.idle.size();  // the smallest block that fits without wasting half of itself
     for (size_t i = 0; i < d.idle.size(); ++i)
-      if (d.idle[i].bytes >= bytes && d.idle[i].bytes <= 2 * bytes &&
+      if (d.idle[i].device == device && d.idle[i].bytes >= bytes && d.idle[i].bytes <= 2 * bytes &&
           (best == d.idle.size() || d.idle[i].bytes < d.idle[best].bytes))
         best = i;
     if (best < d.idle.size()) {
       const Block b = d.idle[best];
-      d.out[b.p] = b.bytes;
+      d.out[b.p] = b;
       d.idle[best] = d.idle.back();
       d.idle.pop_back();
       d.kept -= b.bytes;
@@ -219,7 +234,7 @@ hipError_t dev_alloc(void **p, size_t bytes) try {
       return hipSuccess;
     }
   }
-  hipError_t e = hipMalloc(p, bytes);
+  e = hipMalloc(p, bytes);
   if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
     dev_trim();
@@ -228,7 +243,7 @@ hipError_t dev_alloc(void **p, size_t bytes) try {
   if (e != hipSuccess) return e;
   try {
     std::lock_guard<std::mutex> lk(d.mu);
-    d.out[*p] = bytes;
+    d.out[*p] = Block{*p, bytes, device};
   } catch (const std::bad_alloc &) {
     (void)hipFree(*p);
     *p = nullptr;
@@ -245,12 +260,14 @@ void dev_free(void *p) {
   try {
     std::lock_guard<std::mutex> lk(d.mu);
     const auto it = d.out.find(p);
-    const size_t bytes = it == d.out.end() ? 0 : it->second;
-    if (it != d.out.end()) d.out.erase(it);
-    if (bytes > 0 && d.kept + bytes <= kPoolBytes) {
-      d.idle.push_back(Block{p, bytes});
-      d.kept += bytes;
-      return;
+    if (it != d.out.end()) {
+      const Block b = it->second;
+      d.out.erase(it);
+      if (d.kept + b.bytes <= kPoolBytes) {
+        d.idle.push_back(b);
+        d.kept += b.bytes;
+        return;
+      }
     }
   } catch (const std::bad_alloc &) {
   }

@@ -30,8 +30,8 @@ bool device_ready();
 const char *device_identity();
 
 // ------------------------------------------------ host buffers (hostio.hpp)
-// hipMemcpyAsync between the device and host memory, pageable memory of 1 MB
-// and more through pinned slots on several threads (complete on return).  As
+// hipMemcpyAsync between the device and host memory, large pageable copies
+// (32 MB up, 8 MB down) through pinned slots on several threads.  As
 // with hipMemcpyAsync, a host destination holds the data once `s` is synchronised.
 hipError_t copy_to_device(void *dst, const void *src, size_t bytes, hipStream_t s);
 hipError_t copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t s);

@@ -1639,6 +1639,18 @@ __device__ inline void bf3_weights(const uint32_t *w, int q, const uint2 *t3, fl
   }
 }
 
+// Accumulators of a row of tiles: cleared, and added to others.
+template <typename V, int N>
+__device__ inline void zero_row(V (&v)[N]) {
+#pragma unroll
+  for (int c = 0; c < N; ++c) v[c] = V{};
+}
+template <typename V, int N>
+__device__ inline void add_row(V (&to)[N], const V (&v)[N]) {
+#pragma unroll
+  for (int c = 0; c < N; ++c) to[c] += v[c];
+}
+
 // Blocks of grid row 1 work on the second store.
 __device__ inline void take_pair(GemmArgs &a) {
   if (blockIdx.y != 0) {
@@ -1647,7 +1659,16 @@ __device__ inline void take_pair(GemmArgs &a) {
   }
 }
 
-template <int BK, int MT, int D, int NC>
+// SUMS (pair launches of one row of tiles): a stage's products go into
+// accumulators of their own, added to the tile's once per stage.  A pair's
+// shares are twice as long as a single launch's; one fp32 rounding per stage in
+// place of 12 or 24 keeps the error below a single launch's (SwiGLU 4096 x
+// 11008 against 64 bits: NF4 b8 6.4e-7 as two launches, 7.5e-7 as a pair
+// without, 5.2e-7 with; Int8 b24 3.9e-7 / - / 3.2e-7) at 1% of its time (56.4
+// -> 57.3 us; two launches 68.6).  It costs a single launch 1% (NF4 4096 -> 11008 b8 21.6 -> 21.9 us), and with two rows of tiles
+// 7-12% (the accumulators take the registers of the loads in flight: FP4 b100
+// 41.5 -> 44.3, NF4 b64 41.5 -> 47.2), so neither has it.
+template <int BK, int MT, int D, int NC, bool SUMS = false>
 __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
   take_pair(a);
   using K3 = B3<BK>;
@@ -1763,7 +1784,8 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
   // decoded (its x went to LDS one unit earlier).  A tile's partial sum is
   // written after its last unit here.  Rows past N read row N - 1 (finite
   // codes) and their columns are never stored.
-  floatx16 acc[MT][NC];
+  static_assert(!SUMS || MT == 1, "one row of stage accumulators");
+  floatx16 acc[MT][NC], part[MT][NC];
   int buf = 0;
   // loads past the share re-read its last unit (valid addresses, unused
   // data): unconditional loads keep the wait counts static
@@ -1789,6 +1811,7 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[mt][c][i] = 0.0f;
       }
+      if constexpr (SUMS) zero_row(part[0]);
       if constexpr (NP == 1) {
         // decode the unit's weights, refill the slot, then the MFMAs
         bf16x8 bv[4][NC][1];
@@ -1803,7 +1826,7 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
         load_w(min(u + D, last), wr[d]);
         load_x(min(u + D, last), xf[d], xin[d]);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) mfma_step(acc, buf, q, bv[q]);
+        for (int q = 0; q < 4; ++q) mfma_step(SUMS ? part : acc, buf, q, bv[q]);
       } else {
         // three weight parts: decode step by step, refill the slot afterwards
         load_x(min(u + D, last), xf[d], xin[d]);
@@ -1812,10 +1835,11 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
           bf16x8 bv[NC][NP];
 #pragma unroll
           for (int c = 0; c < NC; ++c) bf3_weights<BK>(wr[d][c], q, t3, zp, bv[c]);
-          mfma_step(acc, buf, q, bv);
+          mfma_step(SUMS ? part : acc, buf, q, bv);
         }
         load_w(min(u + D, last), wr[d]);
       }
+      if constexpr (SUMS) add_row(acc[0], part[0]);
       store_x(buf ^ 1, xf[(d + 1) % D], xin[(d + 1) % D]);
       __syncthreads();
       buf ^= 1;
@@ -1847,7 +1871,7 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
 // and each writes half of the one partial tile.  One workgroup per CU keeps
 // two waves per SIMD, like two 4-wave workgroups per CU, while a launch
 // writes half the partial tiles.  GemmArgs::nst counts stage pairs here.
-template <int BK, int MT, int D, int NC>
+template <int BK, int MT, int D, int NC, bool SUMS = false>
 __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
   take_pair(a);
   using K3 = B3<BK>;
@@ -1951,7 +1975,8 @@ __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
       }
     }
   };
-  floatx16 acc[MT][NC];
+  static_assert(!SUMS || MT == 1, "one row of stage accumulators");
+  floatx16 acc[MT][NC], part[MT][NC];
   int buf = 0;
   const int last = max(it, it_end - 1);
   // the first unit's loads go out alone: every workgroup asks at once, and
@@ -1991,6 +2016,7 @@ __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[mt][c][i] = 0.0f;
       }
+      if constexpr (SUMS) zero_row(part[0]);
       if constexpr (NP == 1) {
         bf16x8 bv[4][NC][1];
 #pragma unroll
@@ -2004,7 +2030,7 @@ __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
         load_x(min(u + D, last), xf[d], xin[d]);  // first: the early x store waits for it alone
         load_w(min(u + D, last), wr[d]);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) mfma_step(acc, buf, q, bv[q]);
+        for (int q = 0; q < 4; ++q) mfma_step(SUMS ? part : acc, buf, q, bv[q]);
       } else {
         load_x(min(u + D, last), xf[d], xin[d]);
 #pragma unroll
@@ -2012,10 +2038,11 @@ __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
           bf16x8 bv[NC][NP];
 #pragma unroll
           for (int c = 0; c < NC; ++c) bf3_weights<BK>(wr[d][c], q, t3, zp, bv[c]);
-          mfma_step(acc, buf, q, bv);
+          mfma_step(SUMS ? part : acc, buf, q, bv);
         }
         load_w(min(u + D, last), wr[d]);
       }
+      if constexpr (SUMS) add_row(acc[0], part[0]);
       if (tile_end) {
         // piece pc = mt * NC + c: group 0 keeps pieces 0 .. P/2 - 1, group 1
         // the rest; each group leaves the other's pieces in region grp of the
@@ -2076,7 +2103,7 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // k = 16 g + 8 q + i (i < 8) from both operands: a permutation of the stage's
 // k order, the same on both sides.  D lane (j, g) holds column j, rows
 // 4 g .. 4 g + 3.
-template <int BK, int D, int NC>
+template <int BK, int D, int NC, bool SUMS = false>
 __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
   take_pair(a);
   using K3 = B3<BK>;
@@ -2164,7 +2191,7 @@ __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
           if (p + wp <= 2) acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv[c][wp], acc[c], 0, 0, 0);
     }
   };
-  floatx4 acc[CG];
+  floatx4 acc[CG], part[CG];
   int buf = 0;
   const int last = max(it, it_end - 1);
 #pragma unroll
@@ -2188,6 +2215,7 @@ __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) acc[c][i] = 0.0f;
       }
+      if constexpr (SUMS) zero_row(part);
       if constexpr (NP == 1) {
         bf16x8 bv[2][CG][1];
 #pragma unroll
@@ -2201,7 +2229,7 @@ __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
         load_x(min(u + D, last), xf[d], xin[d]);
         load_w(min(u + D, last), wr[d]);
 #pragma unroll
-        for (int q = 0; q < 2; ++q) mfma_step(acc, buf, q, bv[q]);
+        for (int q = 0; q < 2; ++q) mfma_step(SUMS ? part : acc, buf, q, bv[q]);
       } else {
         load_x(min(u + D, last), xf[d], xin[d]);
 #pragma unroll
@@ -2209,10 +2237,11 @@ __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
           bf16x8 bv[CG][NP];
 #pragma unroll
           for (int c = 0; c < CG; ++c) bf3_weights<BK>(wr[d][c], q, t3, zp, bv[c]);
-          mfma_step(acc, buf, q, bv);
+          mfma_step(SUMS ? part : acc, buf, q, bv);
         }
         load_w(min(u + D, last), wr[d]);
       }
+      if constexpr (SUMS) add_row(acc, part);
       store_x(buf ^ 1, xf[(d + 1) % D], xin[(d + 1) % D]);
       lds_barrier();  // the next units' loads stay in flight
       buf ^= 1;
@@ -3270,6 +3299,29 @@ hipError_t launch_bf3r(const SkPlan &p, int bk, const GemmArgs &a, const double 
 // The split-x GEMM of plan p for weight kind bk (a.body, a.post set).
 hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
   const dim3 grid(p.blocks, a.body2 != nullptr ? 2 : 1);
+  if (a.body2 != nullptr && p.bm <= 32) {
+#define WH_GP(BK)                                                                             \
+  if (p.bm == 16) {                                                                           \
+    if (p.bn == 128) gemm_bf3s_kernel<BK, 1, 1, true><<<grid, 256, 0, s>>>(a);             \
+    else gemm_bf3s_kernel<BK, 1, 2, true><<<grid, 256, 0, s>>>(a);                         \
+  } else WH_GP32(BK)
+#define WH_GP32(BK)                                                                           \
+  if (p.kg == 2) gemm_bf3k_kernel<BK, 1, 2, 2, true><<<grid, 512, 0, s>>>(a);              \
+  else if (p.bn == 128) gemm_bf3_kernel<BK, 1, 1, 1, true><<<grid, 256, 0, s>>>(a);        \
+  else gemm_bf3_kernel<BK, 1, 1, 2, true><<<grid, 256, 0, s>>>(a);
+    switch (bk) {
+    case BK_I4: WH_GP32(BK_I4) break;  // batches above 16 only
+    case BK_E4: WH_GP(BK_E4) break;
+    case BK_I8: WH_GP(BK_I8) break;
+    case BK_FP4: WH_GP(BK_FP4) break;
+    case BK_NF4: WH_GP(BK_NF4) break;
+    case BK_E5: WH_GP(BK_E5) break;
+    default: return hipErrorInvalidValue;
+    }
+#undef WH_GP
+#undef WH_GP32
+    return hipGetLastError();
+  }
 #define WH_GB(BK)                                                                     \
   if (p.bm == 16) {                                                                   \
     if (p.bn == 128) gemm_bf3s_kernel<BK, 1, 1><<<grid, 256, 0, s>>>(a);           \
@@ -3612,14 +3664,19 @@ hipError_t launch_forward(const DevStore &w, int batch, const float *x, const do
 }
 
 namespace {
-// The plan of a pair launch on the split-x GEMM, each store on half the CUs
-// (half the partial tiles of a launch of its own); false where the batch
-// takes another route or the kind's reduction does more than add.
+// The plan of a pair launch on the split-x GEMM; false where the batch takes
+// another route or the kind's reduction does more than add.  Up to 32-row
+// tiles each store has half the CUs (half the partial tiles of a launch of its
+// own), with stage sums (gemm_bf3_kernel).  64-row tiles have no registers for
+// those and keep a single launch's shares and so its bits: 4096 x 11008 FP8
+// b64 93.1 -> 85.7 us, NF4 b64 123.8 -> 118.7, FP4 b512 396.5 -> 386.4 (half
+// the CUs each: FP8 85.4, FP4 387.0, with 4-17% more error).
 bool pair_gemm_plan(const DevStore &g, const DevStore &u, int batch, int &bk, SkPlan &p) {
   if (g.dtype != u.dtype || g.rows != u.rows || g.cols != u.cols || fwd_route(g, batch) != 2) return false;
   bk = bf3_fwd_kind(g, batch);
   if (bk < 0 || bk != bf3_fwd_kind(u, batch) || (bk >= BK_B16 && bk != BK_I4)) return false;
   p = plan_fwd_gemm(kernel_fmt(g.dtype), bk, batch, g.cols, g.rows, 2);
+  if (p.bf3 && p.bm == 64) p = plan_fwd_gemm(kernel_fmt(g.dtype), bk, batch, g.cols, g.rows);
   return p.bf3 && !p.rows;
 }
 }  // namespace

@@ -176,7 +176,7 @@ welvet_status store_encode(Store *w, const float *d_w, bool repack, hipStream_t 
     w->minv = 0.0f;
     return ok();
   }
-  DevBuf buf(s);
+  DevBuf buf(s, w->pooled || repack);
   WH_HIP(buf.alloc(sizeof(EncodeScratch)));
   EncodeScratch *scratch = buf.as<EncodeScratch>();
   hipError_t e = launch_encode(dtype, d_w, n, w->body, w->kbody, &scratch->meta, &scratch->stats, s, repack);
@@ -278,7 +278,7 @@ welvet_status store_set_bias(Store *w, const double *bias, size_t bias_len, hipS
 // Upload f32 weights and build the store.
 welvet_status store_from_host(Store *w, int dtype, int rows, int cols, const float *W_init,
                               hipStream_t s) {
-  DevBuf d(s);
+  DevBuf d(s, w->pooled);
   const size_t bytes = (size_t)rows * cols * sizeof(float);
   WH_HIP(d.alloc(bytes));
   WH_HIP(copy_to_device(d.p, W_init, bytes, s));

@@ -40,15 +40,17 @@ hipError_t copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t s)
 hipError_t dev_alloc(void **p, size_t bytes);
 void dev_free(void *p);
 void dev_trim();  // gives every idle block back
-// A call's buffer, freed when `stream` has drained.
+// A call's buffer, freed when `stream` has drained; pooled: from dev_alloc,
+// else from hipMalloc.
 struct DevBuf {
   void *p = nullptr;
   hipStream_t stream;
-  explicit DevBuf(hipStream_t s) : stream(s) {}
+  bool pooled;
+  explicit DevBuf(hipStream_t s, bool from_pool = true) : stream(s), pooled(from_pool) {}
   ~DevBuf();
   DevBuf(const DevBuf &) = delete;
   DevBuf &operator=(const DevBuf &) = delete;
-  hipError_t alloc(size_t bytes) { return dev_alloc(&p, bytes); }
+  hipError_t alloc(size_t bytes) { return pooled ? dev_alloc(&p, bytes) : hipMalloc(&p, bytes); }
   template <typename T>
   T *as() const { return (T *)p; }
 };

@@ -1659,7 +1659,7 @@ __device__ inline void take_pair(GemmArgs &a) {
   }
 }
 
-// SUMS (pair launches of one row of tiles): a stage's products go into
+// SUMS (pair launches and longer shares, one row of tiles): a stage's products go into
 // accumulators of their own, added to the tile's once per stage.  A pair's
 // shares are twice as long as a single launch's; one fp32 rounding per stage in
 // place of 12 or 24 keeps the error below a single launch's (SwiGLU 4096 x
@@ -3021,6 +3021,7 @@ struct SkPlan {
   bool bf3 = false;  // split-x GEMM plan (bn = 128 or 256)
   int kg = 1;        // k stages per unit: 2 = the two-group split-x GEMM
   bool rows = false;  // gemm_bf3r_kernel: whole K per workgroup, no partials
+  bool longer = false;  // shares of more units than an equal split over the CUs
 };
 
 // Stream-K split of an M x N x K product over bm x bn tiles into equal
@@ -3041,7 +3042,9 @@ SkPlan plan_sk(int M, int K, int N, int bm = kBM, int bn = kBN, int occ = 2, int
   // costs more than the shorter shares save (FP8 32 x 128 tiles, 4096 -> 512
   // b48 19.2 -> 11.7 us, 8192 -> 300 b24 28.0 -> 15.0, 1024^2 b100 11.9 ->
   // 9.5; 8 and 4 lose at K >= 4096, 24 and 32 at K <= 4096)
+  // (such longer shares with stage sums, see launch_bf3)
   p.per_block = std::max((int)((T + G - 1) / G), (p.nst + 15) / 16);
+  p.longer = p.per_block > (T + G - 1) / G;
   p.blocks = (int)((T + p.per_block - 1) / p.per_block);
   p.maxspan = (p.per_block + p.nst - 1) / p.nst + 1;
   p.ws_bytes = (size_t)p.blocks * p.maxspan * bm * bn * sizeof(float);
@@ -3299,7 +3302,10 @@ hipError_t launch_bf3r(const SkPlan &p, int bk, const GemmArgs &a, const double 
 // The split-x GEMM of plan p for weight kind bk (a.body, a.post set).
 hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
   const dim3 grid(p.blocks, a.body2 != nullptr ? 2 : 1);
-  if (a.body2 != nullptr && p.bm <= 32) {
+  // stage sums where the shares are longer than an equal split's: the error
+  // stays that of the shorter ones (FP4 3136 -> 1368 b13 1.3e-7 from 64 bits at
+  // shares of two stages, 1.7e-7 at four without)
+  if ((a.body2 != nullptr || p.longer) && p.bm <= 32 && !p.rows && (bk < BK_B16 || bk == BK_I4)) {
 #define WH_GP(BK)                                                                             \
   if (p.bm == 16) {                                                                           \
     if (p.bn == 128) gemm_bf3s_kernel<BK, 1, 1, true><<<grid, 256, 0, s>>>(a);             \

@@ -342,8 +342,7 @@ __global__ void __launch_bounds__(64 * KG) ragged_dx_kernel(RaggedArgs a, float 
 }
 
 RaggedArgs ragged_args(const DevStore &w, const float *A, int M, int K, int N, int f) {
-  // a zero scale decodes as 1 (native_codec.cpp weight_at)
-  return RaggedArgs{kernel_body(w, f), w.lut, w.scale == 0.0f ? 1.0f : w.scale, w.minv, A, M, K, N, w.cols, 0, 0};
+  return RaggedArgs{kernel_body(w, f), w.lut, w.scale, w.minv, A, M, K, N, w.cols, 0, 0};
 }
 
 template <int F>

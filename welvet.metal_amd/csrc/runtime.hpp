@@ -76,8 +76,11 @@ struct Store {
   uint8_t *tbody = nullptr;
   bool tbody_ok = false;
 
+  // the store as the product kernels take it: a zero scale decodes as 1
+  // (native_codec.cpp weight_at)
   DevStore dev() const {
-    return DevStore{dtype, rows, cols, scale, minv, body, kbody, lut, finite, tbody_ok ? tbody : nullptr};
+    return DevStore{dtype, rows, cols, scale == 0.0f ? 1.0f : scale, minv, body, kbody, lut, finite,
+                    tbody_ok ? tbody : nullptr};
   }
   int64_t n() const { return (int64_t)rows * cols; }
 };

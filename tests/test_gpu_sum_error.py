@@ -1,0 +1,45 @@
+"""How far sums over a long K are from 64 bits (2-norm of the difference over
+2-norm of the result), which the element-wise tolerances do not see.  A GEMM's
+fp32 chains end at its shares of K (they are added in f64): c products of
+random sign in one chain of fp32 additions, each rounded to 2^-24 / 2 at most
+of a partial sum that grows as the root of its length, end within 2^-24
+sqrt(c / 2) of the result (a mean over the outputs; about a third of it is
+measured)."""
+import numpy as np
+import pytest
+
+import pywelvet
+from test_gpu_dense import oracle_weights
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def device():
+    pywelvet.init()
+
+
+def chain_bound(products):
+    return 2.0 ** -24 * np.sqrt(products / 2)
+
+
+def error(got, ref):
+    return np.linalg.norm(got - ref) / np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("dtype,batch", [(1, 17), (1, 64), (2, 13), (2, 33), (3, 13), (3, 33), (8, 33), (13, 33),
+                                         (15, 33), (27, 64)])
+def test_long_k_few_outputs(oracle, dtype, batch):
+    """128 outputs over K = 11008: one k stage of 64 per share in the kernels
+    without stage sums, forward and (K = rows) dX."""
+    rng = np.random.default_rng(dtype * 100 + batch)
+    W = rng.normal(0, 0.1, (128, 11008)).astype(np.float32)
+    x = rng.normal(0, 1, (batch, 11008)).astype(np.float32)
+    pre, _ = pywelvet.forward(W, x, dtype=dtype)
+    Wd = oracle_weights(oracle, dtype, W)
+    assert error(pre, x.astype(np.float64) @ Wd.T) <= chain_bound(64)
+    V = np.ascontiguousarray(W.T)
+    with pywelvet.Session(V, batch=batch, dtype=dtype) as s:
+        dX, _ = s.backward(np.zeros((batch, 128), np.float32), x, x)
+    Vd = oracle_weights(oracle, dtype, V)
+    assert error(dX, x.astype(np.float64) @ Vd) <= chain_bound(64)

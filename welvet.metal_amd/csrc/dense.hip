@@ -3021,14 +3021,16 @@ struct SkPlan {
   bool bf3 = false;  // split-x GEMM plan (bn = 128 or 256)
   int kg = 1;        // k stages per unit: 2 = the two-group split-x GEMM
   bool rows = false;  // gemm_bf3r_kernel: whole K per workgroup, no partials
-  bool longer = false;  // shares of more units than an equal split over the CUs
+  bool sums = false;  // split-x GEMM with stage sums (gemm_bf3_kernel's SUMS)
 };
 
 // Stream-K split of an M x N x K product over bm x bn tiles into equal
 // shares, `occ` workgroups per CU (of 1 / `share` of the CUs, where as many
 // products share a launch); units of `kg` consecutive k stages (the
-// caller makes the stage count a multiple of kg).
-SkPlan plan_sk(int M, int K, int N, int bm = kBM, int bn = kBN, int occ = 2, int kg = 1, int share = 1) {
+// caller makes the stage count a multiple of kg); shares of at least `least`
+// units, with stage sums where that makes them longer than equal ones.
+SkPlan plan_sk(int M, int K, int N, int bm = kBM, int bn = kBN, int occ = 2, int kg = 1, int share = 1,
+               int least = 1) {
   SkPlan p;
   p.bm = bm;
   p.bn = bn;
@@ -3038,13 +3040,8 @@ SkPlan plan_sk(int M, int K, int N, int bm = kBM, int bn = kBN, int occ = 2, int
   p.nst = (K + kBK - 1) / kBK / kg;
   const int64_t T = (int64_t)p.gx * p.gy * p.nst;
   const int64_t G = std::max<int64_t>(1, (int64_t)occ * num_cus() / share);
-  // at most 16 partial tiles per tile: past that the reduction's serial sum
-  // costs more than the shorter shares save (FP8 32 x 128 tiles, 4096 -> 512
-  // b48 19.2 -> 11.7 us, 8192 -> 300 b24 28.0 -> 15.0, 1024^2 b100 11.9 ->
-  // 9.5; 8 and 4 lose at K >= 4096, 24 and 32 at K <= 4096)
-  // (such longer shares with stage sums, see launch_bf3)
-  p.per_block = std::max((int)((T + G - 1) / G), (p.nst + 15) / 16);
-  p.longer = p.per_block > (T + G - 1) / G;
+  p.per_block = std::max((int)((T + G - 1) / G), least);
+  p.sums = p.per_block > (T + G - 1) / G;
   p.blocks = (int)((T + p.per_block - 1) / p.per_block);
   p.maxspan = (p.per_block + p.nst - 1) / p.nst + 1;
   p.ws_bytes = (size_t)p.blocks * p.maxspan * bm * bn * sizeof(float);
@@ -3121,9 +3118,23 @@ SkPlan plan_fwd_gemm(int f, int bk, int M, int K, int N, int share = 1) {
     // batch 32 and, up to it, those of the 4-bit kinds (FP8 / Int8 measured
     // slower there)
     const bool groups = bn == 256 && stages % 2 == 0 && (bm == 64 || (bm == 32 && (M > 32 || four_bit)));
-    SkPlan p = groups ? plan_sk(M, K, N, bm, bn, 1, 2, share)
-                      : plan_sk(M, K, N, bm, bn, occ, 1, share);
+    // Shares of at least a sixteenth of K (a tile then has at most 17 partial
+    // tiles): past that the reduction's serial sum costs more than the shorter
+    // shares save (FP8 32 x 128 tiles, 4096 -> 512 b48 19.2 -> 11.7 us, 8192 ->
+    // 300 b24 28.0 -> 15.0, 1024^2 b100 11.9 -> 9.5; 16 x 128 tiles 4096 -> 512
+    // b13 17.0 -> 10.3; an eighth and a quarter lose at K >= 4096, shorter
+    // shares at K <= 4096).  Only with stage sums, which keep the longer
+    // shares' error: without them it triples (Float32 11008 -> 128 b17 1.5e-7
+    // -> 5.0e-7 from 64 bits, on the fp32 MFMA, where it is also slower:
+    // Int16 11008 -> 1024 b64 35.1 -> 45.0).  Not for NF4's two-group tiles,
+    // whose units take longest (11008 -> 1024 b17 19.7 -> 24.4).
+    const bool can_sum = bm <= 32 && (bk < BK_B16 || bk == BK_I4);
+    const int units_k = groups ? stages / 2 : stages;
+    const int least = can_sum && !(groups && bk == BK_NF4) ? (units_k + 15) / 16 : 1;
+    SkPlan p = groups ? plan_sk(M, K, N, bm, bn, 1, 2, share, least)
+                      : plan_sk(M, K, N, bm, bn, occ, 1, share, least);
     p.bf3 = true;
+    if (can_sum && share > 1) p.sums = true;  // a pair's shares are longer too
     if (bk == BK_U8) p.ws_bytes += rowsum_bytes(M);
     return p;
   }
@@ -3302,10 +3313,7 @@ hipError_t launch_bf3r(const SkPlan &p, int bk, const GemmArgs &a, const double 
 // The split-x GEMM of plan p for weight kind bk (a.body, a.post set).
 hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
   const dim3 grid(p.blocks, a.body2 != nullptr ? 2 : 1);
-  // stage sums where the shares are longer than an equal split's: the error
-  // stays that of the shorter ones (FP4 3136 -> 1368 b13 1.3e-7 from 64 bits at
-  // shares of two stages, 1.7e-7 at four without)
-  if ((a.body2 != nullptr || p.longer) && p.bm <= 32 && !p.rows && (bk < BK_B16 || bk == BK_I4)) {
+  if (p.sums) {
 #define WH_GP(BK)                                                                             \
   if (p.bm == 16) {                                                                           \
     if (p.bn == 128) gemm_bf3s_kernel<BK, 1, 1, true><<<grid, 256, 0, s>>>(a);             \

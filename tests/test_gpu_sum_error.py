@@ -43,3 +43,19 @@ def test_long_k_few_outputs(oracle, dtype, batch):
         dX, _ = s.backward(np.zeros((batch, 128), np.float32), x, x)
     Vd = oracle_weights(oracle, dtype, V)
     assert error(dX, x.astype(np.float64) @ Vd) <= chain_bound(64)
+
+
+@pytest.mark.parametrize("dtype", [4, 5, 9, 16, 26, 2])
+@pytest.mark.parametrize("inn,out,batch", [(1024, 1024, 512), (4096, 512, 250), (2048, 4096, 120), (1024, 3000, 100)])
+def test_stage_sums(oracle, dtype, inn, out, batch):
+    """32-row tiles above batch 32 (K = 4 to 8 stages a share): a stage rounds
+    its sum four times (16 products a step; the products of x's and w's lower
+    parts weigh 2^-8) and the tile's sum once, n stages a share and the
+    output's own rounding on top."""
+    rng = np.random.default_rng(dtype * 100 + batch)
+    W = rng.normal(0, 2.0 if dtype == 16 else 0.1, (out, inn)).astype(np.float32)
+    x = rng.normal(0, 1, (batch, inn)).astype(np.float32)
+    pre, _ = pywelvet.forward(W, x, dtype=dtype)
+    Wd = oracle_weights(oracle, dtype, W)
+    stages = -(-(-(-batch // 32) * -(-out // 128) * (inn // 64)) // 512)  # a share of 512 blocks' equal ones
+    assert error(pre, x.astype(np.float64) @ Wd.T) <= 2.0 ** -24 * np.sqrt((4 + stages + 1) / 2)

@@ -1659,15 +1659,12 @@ __device__ inline void take_pair(GemmArgs &a) {
   }
 }
 
-// SUMS (pair launches and longer shares, one row of tiles): a stage's products go into
-// accumulators of their own, added to the tile's once per stage.  A pair's
-// shares are twice as long as a single launch's; one fp32 rounding per stage in
-// place of 12 or 24 keeps the error below a single launch's (SwiGLU 4096 x
-// 11008 against 64 bits: NF4 b8 6.4e-7 as two launches, 7.5e-7 as a pair
-// without, 5.2e-7 with; Int8 b24 3.9e-7 / - / 3.2e-7) at 1% of its time (56.4
-// -> 57.3 us; two launches 68.6).  It costs a single launch 1% (NF4 4096 -> 11008 b8 21.6 -> 21.9 us), and with two rows of tiles
-// 7-12% (the accumulators take the registers of the loads in flight: FP4 b100
-// 41.5 -> 44.3, NF4 b64 41.5 -> 47.2), so neither has it.
+// SUMS (one row of tiles; plan_fwd_gemm says where): a stage's products go
+// into accumulators of their own (`part`), added to the tile's once per stage,
+// and of them the small ones, those of the lower parts of x or w, first, or
+// where a weight has parts into a third set (`low`, added at the tile's end):
+// they are 2^-8 of the others, so a stage rounds its sum four times and not 12
+// to 24.
 template <int BK, int MT, int D, int NC, bool SUMS = false>
 __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
   take_pair(a);
@@ -1763,19 +1760,19 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
   };
   // One MFMA step: products of x part p with weight part wp for p + wp <= 2
   // (the dropped NF4 terms are below 2^-23 of each product).
-  auto mfma_step = [&](floatx16 (&acc)[MT][NC], int buf, int q, const bf16x8 (&bv)[NC][NP]) {
+  auto mfma_part = [&](floatx16 (&acc)[MT][NC], floatx16 (&low)[MT][NC], int buf, int q, int p,
+                       const bf16x8 (&bv)[NC][NP]) {
 #pragma unroll
-    for (int p = 0; p < 3; ++p) {
+    for (int mt = 0; mt < MT; ++mt) {
+      const bf16x8 av = __builtin_bit_cast(bf16x8, *(const shortx8 *)&Xs[buf][p][mt * 32 + j][32 * h + 8 * q]);
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const bf16x8 av = __builtin_bit_cast(bf16x8, *(const shortx8 *)&Xs[buf][p][mt * 32 + j][32 * h + 8 * q]);
+      for (int c = 0; c < NC; ++c)
 #pragma unroll
-        for (int c = 0; c < NC; ++c)
-#pragma unroll
-          for (int wp = 0; wp < NP; ++wp)
-            if (p + wp <= 2)
-              acc[mt][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv[c][wp], acc[mt][c], 0, 0, 0);
-      }
+        for (int wp = 0; wp < NP; ++wp) {
+          if (p + wp > 2) continue;
+          floatx16 &to = p + wp == 0 ? acc[mt][c] : low[mt][c];
+          to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv[c][wp], to, 0, 0, 0);
+        }
     }
   };
   // The block's units run as one stream across tile boundaries: unit u
@@ -1785,7 +1782,7 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
   // written after its last unit here.  Rows past N read row N - 1 (finite
   // codes) and their columns are never stored.
   static_assert(!SUMS || MT == 1, "one row of stage accumulators");
-  floatx16 acc[MT][NC], part[MT][NC];
+  floatx16 acc[MT][NC], part[MT][NC], low[MT][NC];
   int buf = 0;
   // loads past the share re-read its last unit (valid addresses, unused
   // data): unconditional loads keep the wait counts static
@@ -1810,6 +1807,7 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
           for (int c = 0; c < NC; ++c)
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[mt][c][i] = 0.0f;
+        if constexpr (SUMS && NP > 1) zero_row(low[0]);
       }
       if constexpr (SUMS) zero_row(part[0]);
       if constexpr (NP == 1) {
@@ -1825,8 +1823,17 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
           }
         load_w(min(u + D, last), wr[d]);
         load_x(min(u + D, last), xf[d], xin[d]);
+        if constexpr (SUMS) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) mfma_step(SUMS ? part : acc, buf, q, bv[q]);
+          for (int p = 2; p >= 0; --p)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) mfma_part(part, part, buf, q, p, bv[q]);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int p = 0; p < 3; ++p) mfma_part(acc, acc, buf, q, p, bv[q]);
+        }
       } else {
         // three weight parts: decode step by step, refill the slot afterwards
         load_x(min(u + D, last), xf[d], xin[d]);
@@ -1835,7 +1842,8 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
           bf16x8 bv[NC][NP];
 #pragma unroll
           for (int c = 0; c < NC; ++c) bf3_weights<BK>(wr[d][c], q, t3, zp, bv[c]);
-          mfma_step(SUMS ? part : acc, buf, q, bv);
+#pragma unroll
+          for (int p = 0; p < 3; ++p) mfma_part(SUMS ? part : acc, SUMS ? low : acc, buf, q, p, bv);
         }
         load_w(min(u + D, last), wr[d]);
       }
@@ -1844,6 +1852,7 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
       __syncthreads();
       buf ^= 1;
       if (st == a.nst - 1 || u + 1 == it_end) {
+        if constexpr (SUMS && NP > 1) add_row(acc[0], low[0]);
         // D[m][n]: lane (j, h) holds column j, rows 8*(r/4) + 4*h + r%4.
         // Groups of 8 rows wholly past M are never read by the reduction:
         // not stored (a wave-uniform test)
@@ -1959,24 +1968,24 @@ __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
         *(uint4 *)&Xs[buf][grp][p][xm][xk + 8 * q] =
             make_uint4(wp[p][4 * q], wp[p][4 * q + 1], wp[p][4 * q + 2], wp[p][4 * q + 3]);
   };
-  auto mfma_step = [&](floatx16 (&acc)[MT][NC], int buf, int q, const bf16x8 (&bv)[NC][NP]) {
+  auto mfma_part = [&](floatx16 (&acc)[MT][NC], floatx16 (&low)[MT][NC], int buf, int q, int p,
+                       const bf16x8 (&bv)[NC][NP]) {
 #pragma unroll
-    for (int p = 0; p < 3; ++p) {
+    for (int mt = 0; mt < MT; ++mt) {
+      const bf16x8 av =
+          __builtin_bit_cast(bf16x8, *(const shortx8 *)&Xs[buf][grp][p][mt * 32 + j][32 * h + 8 * q]);
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const bf16x8 av =
-            __builtin_bit_cast(bf16x8, *(const shortx8 *)&Xs[buf][grp][p][mt * 32 + j][32 * h + 8 * q]);
+      for (int c = 0; c < NC; ++c)
 #pragma unroll
-        for (int c = 0; c < NC; ++c)
-#pragma unroll
-          for (int wp = 0; wp < NP; ++wp)
-            if (p + wp <= 2)
-              acc[mt][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv[c][wp], acc[mt][c], 0, 0, 0);
-      }
+        for (int wp = 0; wp < NP; ++wp) {
+          if (p + wp > 2) continue;
+          floatx16 &to = p + wp == 0 ? acc[mt][c] : low[mt][c];
+          to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv[c][wp], to, 0, 0, 0);
+        }
     }
   };
   static_assert(!SUMS || MT == 1, "one row of stage accumulators");
-  floatx16 acc[MT][NC], part[MT][NC];
+  floatx16 acc[MT][NC], part[MT][NC], low[MT][NC];
   int buf = 0;
   const int last = max(it, it_end - 1);
   // the first unit's loads go out alone: every workgroup asks at once, and
@@ -2015,6 +2024,7 @@ __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
           for (int c = 0; c < NC; ++c)
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[mt][c][i] = 0.0f;
+        if constexpr (SUMS && NP > 1) zero_row(low[0]);
       }
       if constexpr (SUMS) zero_row(part[0]);
       if constexpr (NP == 1) {
@@ -2029,8 +2039,17 @@ __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
           }
         load_x(min(u + D, last), xf[d], xin[d]);  // first: the early x store waits for it alone
         load_w(min(u + D, last), wr[d]);
+        if constexpr (SUMS) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) mfma_step(SUMS ? part : acc, buf, q, bv[q]);
+          for (int p = 2; p >= 0; --p)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) mfma_part(part, part, buf, q, p, bv[q]);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int p = 0; p < 3; ++p) mfma_part(acc, acc, buf, q, p, bv[q]);
+        }
       } else {
         load_x(min(u + D, last), xf[d], xin[d]);
 #pragma unroll
@@ -2038,12 +2057,14 @@ __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
           bf16x8 bv[NC][NP];
 #pragma unroll
           for (int c = 0; c < NC; ++c) bf3_weights<BK>(wr[d][c], q, t3, zp, bv[c]);
-          mfma_step(SUMS ? part : acc, buf, q, bv);
+#pragma unroll
+          for (int p = 0; p < 3; ++p) mfma_part(SUMS ? part : acc, SUMS ? low : acc, buf, q, p, bv);
         }
         load_w(min(u + D, last), wr[d]);
       }
       if constexpr (SUMS) add_row(acc[0], part[0]);
       if (tile_end) {
+        if constexpr (SUMS && NP > 1) add_row(acc[0], low[0]);
         // piece pc = mt * NC + c: group 0 keeps pieces 0 .. P/2 - 1, group 1
         // the rest; each group leaves the other's pieces in region grp of the
         // exchange, lane-major (same wave index and lane = same outputs)
@@ -2180,18 +2201,18 @@ __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
 #pragma unroll
     for (int p = 0; p < 3; ++p) *(uint2 *)&Xs[buf][p][xm][xk] = make_uint2(wp[p][0], wp[p][1]);
   };
-  auto mfma_step = [&](floatx4 (&acc)[CG], int buf, int q, const bf16x8 (&bv)[CG][NP]) {
+  auto mfma_part = [&](floatx4 (&acc)[CG], floatx4 (&low)[CG], int buf, int q, int p, const bf16x8 (&bv)[CG][NP]) {
+    const bf16x8 av = __builtin_bit_cast(bf16x8, *(const shortx8 *)&Xs[buf][p][j][16 * g + 8 * q]);
 #pragma unroll
-    for (int p = 0; p < 3; ++p) {
-      const bf16x8 av = __builtin_bit_cast(bf16x8, *(const shortx8 *)&Xs[buf][p][j][16 * g + 8 * q]);
+    for (int c = 0; c < CG; ++c)
 #pragma unroll
-      for (int c = 0; c < CG; ++c)
-#pragma unroll
-        for (int wp = 0; wp < NP; ++wp)
-          if (p + wp <= 2) acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv[c][wp], acc[c], 0, 0, 0);
-    }
+      for (int wp = 0; wp < NP; ++wp) {
+        if (p + wp > 2) continue;
+        floatx4 &to = p + wp == 0 ? acc[c] : low[c];
+        to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv[c][wp], to, 0, 0, 0);
+      }
   };
-  floatx4 acc[CG], part[CG];
+  floatx4 acc[CG], part[CG], low[CG];
   int buf = 0;
   const int last = max(it, it_end - 1);
 #pragma unroll
@@ -2214,6 +2235,7 @@ __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
         for (int c = 0; c < CG; ++c)
 #pragma unroll
           for (int i = 0; i < 4; ++i) acc[c][i] = 0.0f;
+        if constexpr (SUMS && NP > 1) zero_row(low);
       }
       if constexpr (SUMS) zero_row(part);
       if constexpr (NP == 1) {
@@ -2228,8 +2250,17 @@ __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
           }
         load_x(min(u + D, last), xf[d], xin[d]);
         load_w(min(u + D, last), wr[d]);
+        if constexpr (SUMS) {
 #pragma unroll
-        for (int q = 0; q < 2; ++q) mfma_step(SUMS ? part : acc, buf, q, bv[q]);
+          for (int p = 2; p >= 0; --p)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) mfma_part(part, part, buf, q, p, bv[q]);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int p = 0; p < 3; ++p) mfma_part(acc, acc, buf, q, p, bv[q]);
+        }
       } else {
         load_x(min(u + D, last), xf[d], xin[d]);
 #pragma unroll
@@ -2237,7 +2268,8 @@ __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
           bf16x8 bv[CG][NP];
 #pragma unroll
           for (int c = 0; c < CG; ++c) bf3_weights<BK>(wr[d][c], q, t3, zp, bv[c]);
-          mfma_step(SUMS ? part : acc, buf, q, bv);
+#pragma unroll
+          for (int p = 0; p < 3; ++p) mfma_part(SUMS ? part : acc, SUMS ? low : acc, buf, q, p, bv);
         }
         load_w(min(u + D, last), wr[d]);
       }
@@ -2246,6 +2278,7 @@ __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
       lds_barrier();  // the next units' loads stay in flight
       buf ^= 1;
       if (st == a.nst - 1 || u + 1 == it_end) {
+        if constexpr (SUMS && NP > 1) add_row(acc, low);
         // rows 4 g .. 4 g + 3 of the tile; a group wholly past M is never read
         float *dst = a.ws + ((int64_t)blockIdx.x * a.maxspan + (t - first_tile)) * (BM * BN);
         if (4 * g < a.M - unit_m0(u)) {
@@ -3118,23 +3151,29 @@ SkPlan plan_fwd_gemm(int f, int bk, int M, int K, int N, int share = 1) {
     // batch 32 and, up to it, those of the 4-bit kinds (FP8 / Int8 measured
     // slower there)
     const bool groups = bn == 256 && stages % 2 == 0 && (bm == 64 || (bm == 32 && (M > 32 || four_bit)));
-    // Shares of at least a sixteenth of K (a tile then has at most 17 partial
-    // tiles): past that the reduction's serial sum costs more than the shorter
-    // shares save (FP8 32 x 128 tiles, 4096 -> 512 b48 19.2 -> 11.7 us, 8192 ->
-    // 300 b24 28.0 -> 15.0, 1024^2 b100 11.9 -> 9.5; 16 x 128 tiles 4096 -> 512
-    // b13 17.0 -> 10.3; an eighth and a quarter lose at K >= 4096, shorter
-    // shares at K <= 4096).  Only with stage sums, which keep the longer
-    // shares' error: without them it triples (Float32 11008 -> 128 b17 1.5e-7
-    // -> 5.0e-7 from 64 bits, on the fp32 MFMA, where it is also slower:
-    // Int16 11008 -> 1024 b64 35.1 -> 45.0).  Not for NF4's two-group tiles,
-    // whose units take longest (11008 -> 1024 b17 19.7 -> 24.4).
-    const bool can_sum = bm <= 32 && (bk < BK_B16 || bk == BK_I4);
+    // Tiles of up to 32 rows: shares of at least a sixteenth of K, or of four
+    // units where that is less (three of NF4's two-group tiles, which take
+    // longest): past it the reduction's serial sum costs more than the shorter
+    // shares save (FP8 32 x 128 tiles, 4096 -> 512 b48 19.2 -> 11.7 us, 1024^2
+    // b100 11.9 -> 9.5; 16 x 128 tiles 4096 -> 512 b13 17.0 -> 10.3; NF4 4096 ->
+    // 512 b33 16.9 -> 12.4), and longer ones idle the CUs and lose precision
+    // (a sixteenth at K = 11008: NF4 11008 -> 1024 b17 19.7 -> 24.4 us, FP4
+    // 11008 -> 128 b8 9.2e-8 -> 1.0e-7 from 64 bits).  Only with stage sums:
+    // without them the error of longer shares triples (Float16 11008 -> 128
+    // b33 1.5e-7 -> 3.9e-7).
     const int units_k = groups ? stages / 2 : stages;
-    const int least = can_sum && !(groups && bk == BK_NF4) ? (units_k + 15) / 16 : 1;
+    const int least = bm <= 32 ? std::min((units_k + 15) / 16, groups && bk == BK_NF4 ? 3 : 4) : 1;
     SkPlan p = groups ? plan_sk(M, K, N, bm, bn, 1, 2, share, least)
                       : plan_sk(M, K, N, bm, bn, occ, 1, share, least);
     p.bf3 = true;
-    if (can_sum && share > 1) p.sums = true;  // a pair's shares are longer too
+    // Stage sums also in a pair launch (twice the shares of a single one) and
+    // in the 32-row tiles that took the place of 64-row ones or of the fp32
+    // MFMA, whose shares were shorter or rounded less: FP8 1024^2 b512 9.7e-8
+    // from 64 bits on 64 x 256 tiles, 1.6e-7 on these without sums, 7.4e-8
+    // with; Float16 4096^2 b64 fp32 MFMA 2.9e-7, 3.2e-7 / 8.4e-8; 1% of the
+    // time.  BFloat16 and Int4 stay below the fp32 MFMA's without them.
+    const bool took_over = bk != BK_B16 && bk != BK_I4 && M > (bk < BK_B16 ? 32 : 16);
+    if (bm <= 32 && (share > 1 || took_over)) p.sums = true;
     if (bk == BK_U8) p.ws_bytes += rowsum_bytes(M);
     return p;
   }
@@ -3321,10 +3360,20 @@ hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
   } else WH_GP32(BK)
 #define WH_GP32(BK)                                                                           \
   if (p.kg == 2) gemm_bf3k_kernel<BK, 1, 2, 2, true><<<grid, 512, 0, s>>>(a);              \
+  else WH_GP32N(BK)
+#define WH_GP32N(BK)  /* kinds whose 32-row tiles are never on two groups (plan_fwd_gemm) */   \
+  if (p.kg == 2) return hipErrorInvalidValue;                                               \
   else if (p.bn == 128) gemm_bf3_kernel<BK, 1, 1, 1, true><<<grid, 256, 0, s>>>(a);        \
   else gemm_bf3_kernel<BK, 1, 1, 2, true><<<grid, 256, 0, s>>>(a);
     switch (bk) {
-    case BK_I4: WH_GP32(BK_I4) break;  // batches above 16 only
+    case BK_I4: WH_GP32(BK_I4) break;  // batches above 16 only, as the next four
+    case BK_U8: WH_GP32(BK_U8) break;
+    case BK_B16: WH_GP32N(BK_B16) break;
+    case BK_H16: WH_GP32N(BK_H16) break;
+    case BK_F32:  // 32 x 128 tiles only
+      if (p.bn != 128) return hipErrorInvalidValue;
+      gemm_bf3_kernel<BK_F32, 1, 1, 1, true><<<grid, 256, 0, s>>>(a);
+      break;
     case BK_E4: WH_GP(BK_E4) break;
     case BK_I8: WH_GP(BK_I8) break;
     case BK_FP4: WH_GP(BK_FP4) break;
@@ -3334,6 +3383,7 @@ hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
     }
 #undef WH_GP
 #undef WH_GP32
+#undef WH_GP32N
     return hipGetLastError();
   }
 #define WH_GB(BK)                                                                     \

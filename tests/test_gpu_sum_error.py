@@ -59,3 +59,18 @@ def test_stage_sums(oracle, dtype, inn, out, batch):
     Wd = oracle_weights(oracle, dtype, W)
     stages = -(-(-(-batch // 32) * -(-out // 128) * (inn // 64)) // 512)  # a share of 512 blocks' equal ones
     assert error(pre, x.astype(np.float64) @ Wd.T) <= 2.0 ** -24 * np.sqrt((4 + stages + 1) / 2)
+
+
+@pytest.mark.parametrize("lo,hi", [(-3.0, 0.05), (-0.05, 3.0), (0.5, 0.75), (-0.05, 0.05)])
+def test_uint8_decoded_values(oracle, lo, hi):
+    """Uint8 multiplies the decoded values fl32(fl32(q scale) + min): with a
+    range far to one side of most weights their rounding is 1e-6 of them, and
+    products of unrounded q scale + min are that far off.  Six products a
+    weight, 24 roundings a stage, three stages a share."""
+    rng = np.random.default_rng(17)
+    W = np.clip(rng.normal(0, 0.01, (2065, 2032)).astype(np.float32) + np.float32(max(lo, 0)), lo, hi)
+    W[0, 0], W[-1, -1] = lo, hi
+    x = rng.normal(0, 1, (70, 2032)).astype(np.float32)
+    pre, _ = pywelvet.forward(W, x, dtype=13)
+    Wd = oracle_weights(oracle, 13, W)
+    assert error(pre, x.astype(np.float64) @ Wd.T) <= chain_bound(72)

@@ -786,15 +786,6 @@ struct GemmArgs {
   int64_t ws2 = 0;
 };
 
-// Split-x kinds from BK_B16 on: the kind for the reduction's recomputation of
-// NaN sums (-1: none), and for Uint8 the weights' common offset and the row
-// sums of A it multiplies (null: no such term).
-struct SplitFix {
-  int kind = -1;
-  double offset = 0.0;
-  const double *rowsum = nullptr;
-};
-
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int kBM = 64, kBN = 64, kBK = 64, kPad = 1;
@@ -1504,26 +1495,21 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // The kinds from BK_B16 on serve batches above 16: BFloat16 codes as they
 // are, Float16 as two exact parts (8 + 3 significand bits), Float32 as three
 // (split like x), Int4 codes as integers (times 16: the nibbles stay in the
-// high half of a byte) and Uint8 codes as integers q - zp around the code zp
-// nearest to the value 0, the rest of the offset, min + zp * scale, times the
-// row sum of x added by the reduction (SplitFix).
+// high half of a byte) and Uint8 like Float32 from its decoded values.  (Its
+// codes as integers around the one nearest to 0, with the rest of the offset
+// times the row sums of x, are half the products, but leave out the rounding
+// of fl32(fl32(q scale) + min), which its values have: where the range lies
+// far to one side of most weights an output was 1e-6 off.)
 enum Bf3Kind {
   BK_E4 = 0, BK_I8 = 1, BK_FP4 = 2, BK_NF4 = 3, BK_E5 = 4, BK_B16 = 5, BK_H16 = 6, BK_F32 = 7, BK_I4 = 8, BK_U8 = 9
 };
-
-// Uint8's centre code, the one whose value is nearest to 0 (weights of both
-// signs then keep small integers: no cancellation against the offset).
-__host__ __device__ inline float u8_centre(float scale, float minv) {
-  const float c = scale > 0.0f ? -minv / scale : 0.0f;
-  return c >= 255.0f ? 255.0f : c > 0.0f ? floorf(c + 0.5f) : 0.0f;
-}
 
 template <int BK>
 struct B3 {
   static constexpr int kBits = BK == BK_F32 ? 32 : (BK == BK_B16 || BK == BK_H16) ? 16
                              : (BK == BK_FP4 || BK == BK_NF4 || BK == BK_I4) ? 4 : 8;
   static constexpr int kWords = kBits;  // words of a lane's 32 weights per stage
-  static constexpr int kParts = (BK == BK_NF4 || BK == BK_F32) ? 3 : BK == BK_H16 ? 2 : 1;
+  static constexpr int kParts = (BK == BK_NF4 || BK == BK_F32 || BK == BK_U8) ? 3 : BK == BK_H16 ? 2 : 1;
 };
 
 typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
@@ -1540,10 +1526,11 @@ inline __device__ bf16x8 bf16x8_of(const uint32_t (&u)[4]) {
 }
 
 // 8 consecutive weights (the words of MFMA step q) as B operands: parts[0..P).
-// NF4 reads the split table t3[code] = {hi | mid << 16, lo}.
+// NF4 reads the split table t3[code] = {hi | mid << 16, lo}; Uint8 decodes
+// with scale and minv.
 template <int BK>
-__device__ inline void bf3_weights(const uint32_t *w, int q, const uint2 *t3, float zp,
-                                   bf16x8 (&parts)[B3<BK>::kParts]) {
+__device__ inline void bf3_weights(const uint32_t *w, int q, const uint2 *t3, bf16x8 (&parts)[B3<BK>::kParts],
+                                   float scale = 1.0f, float minv = 0.0f) {
   if constexpr (BK == BK_E4) {
     const uint32_t w0 = w[2 * q], w1 = w[2 * q + 1];
     const uint32_t u[4] = {
@@ -1581,7 +1568,7 @@ __device__ inline void bf3_weights(const uint32_t *w, int q, const uint2 *t3, fl
   } else if constexpr (BK == BK_B16) {
     const uint32_t u[4] = {w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]};
     parts[0] = bf16x8_of(u);
-  } else if constexpr (BK == BK_H16 || BK == BK_F32) {
+  } else if constexpr (BK == BK_H16 || BK == BK_F32 || BK == BK_U8) {
     uint32_t part[3][4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -1590,6 +1577,10 @@ __device__ inline void bf3_weights(const uint32_t *w, int q, const uint2 *t3, fl
         const uint32_t wd = w[4 * q + i];
         v[0] = (float)__builtin_bit_cast(_Float16, (uint16_t)wd);
         v[1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(wd >> 16));
+      } else if constexpr (BK == BK_U8) {
+        const uint32_t wd = w[2 * q + (i >> 1)] >> ((i & 1) * 16);
+        v[0] = (float)(wd & 0xffu) * scale + minv;
+        v[1] = (float)((wd >> 8) & 0xffu) * scale + minv;
       } else {
         v[0] = u2f(w[8 * q + 2 * i]);
         v[1] = u2f(w[8 * q + 2 * i + 1]);
@@ -1614,14 +1605,6 @@ __device__ inline void bf3_weights(const uint32_t *w, int q, const uint2 *t3, fl
     for (int i = 0; i < 4; ++i)
       u[i] = __builtin_amdgcn_perm(f2u((float)(int8_t)(uint8_t)(hi >> (8 * i))),
                                    f2u((float)(int8_t)(uint8_t)(lo >> (8 * i))), 0x07060302u);
-    parts[0] = bf16x8_of(u);
-  } else if constexpr (BK == BK_U8) {
-    uint32_t u[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t wd = w[2 * q + (i >> 1)] >> ((i & 1) * 16);
-      u[i] = __builtin_amdgcn_perm(f2u((float)((wd >> 8) & 0xffu) - zp), f2u((float)(wd & 0xffu) - zp), 0x07060302u);
-    }
     parts[0] = bf16x8_of(u);
   } else {  // NF4
     const uint32_t wd = w[q];
@@ -1674,7 +1657,6 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
   constexpr int XT = kBK / XE;        // threads per x row
   __shared__ uint16_t Xs[2][3][BM][kBf3Row];
   __shared__ uint2 t3[16];
-  const float zp = BK == BK_U8 ? u8_centre(a.scale, a.minv) : 0.0f;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int j = lane & 31, h = lane >> 5;
   if constexpr (BK == BK_NF4) {
@@ -1818,7 +1800,7 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
 #pragma unroll
           for (int c = 0; c < NC; ++c) {
             bf16x8 pp[1];
-            bf3_weights<BK>(wr[d][c], q, t3, zp, pp);
+            bf3_weights<BK>(wr[d][c], q, t3, pp);
             bv[q][c][0] = pp[0];
           }
         load_w(min(u + D, last), wr[d]);
@@ -1841,7 +1823,7 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
         for (int q = 0; q < 4; ++q) {
           bf16x8 bv[NC][NP];
 #pragma unroll
-          for (int c = 0; c < NC; ++c) bf3_weights<BK>(wr[d][c], q, t3, zp, bv[c]);
+          for (int c = 0; c < NC; ++c) bf3_weights<BK>(wr[d][c], q, t3, bv[c], a.scale, a.minv);
 #pragma unroll
           for (int p = 0; p < 3; ++p) mfma_part(SUMS ? part : acc, SUMS ? low : acc, buf, q, p, bv);
         }
@@ -1892,7 +1874,6 @@ __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
   __shared__ uint16_t Xs[2][2][3][BM][kBf3Row];  // [buffer][group][part][m][k]
   static_assert(sizeof(Xs) >= (size_t)P * 16 * 256 * sizeof(float), "the exchange fits the x buffers");
   __shared__ uint2 t3[16];
-  const float zp = BK == BK_U8 ? u8_centre(a.scale, a.minv) : 0.0f;
   const int tid = threadIdx.x, grp = tid >> 8, gt = tid & 255, lane = tid & 63, wave = gt >> 6;
   const int j = lane & 31, h = lane >> 5;
   if constexpr (BK == BK_NF4) {
@@ -2034,7 +2015,7 @@ __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
 #pragma unroll
           for (int c = 0; c < NC; ++c) {
             bf16x8 pp[1];
-            bf3_weights<BK>(wr[d][c], q, t3, zp, pp);
+            bf3_weights<BK>(wr[d][c], q, t3, pp);
             bv[q][c][0] = pp[0];
           }
         load_x(min(u + D, last), xf[d], xin[d]);  // first: the early x store waits for it alone
@@ -2056,7 +2037,7 @@ __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
         for (int q = 0; q < 4; ++q) {
           bf16x8 bv[NC][NP];
 #pragma unroll
-          for (int c = 0; c < NC; ++c) bf3_weights<BK>(wr[d][c], q, t3, zp, bv[c]);
+          for (int c = 0; c < NC; ++c) bf3_weights<BK>(wr[d][c], q, t3, bv[c]);
 #pragma unroll
           for (int p = 0; p < 3; ++p) mfma_part(SUMS ? part : acc, SUMS ? low : acc, buf, q, p, bv);
         }
@@ -2135,7 +2116,6 @@ __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
   static_assert(XE == 4 && (NW == 2 || NW == 4), "16-row split-x layout");
   __shared__ uint16_t Xs[2][3][BM][kBf3Row];
   __shared__ uint2 t3[16];
-  const float zp = BK == BK_U8 ? u8_centre(a.scale, a.minv) : 0.0f;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int j = lane & 15, g = lane >> 4;
   if constexpr (BK == BK_NF4) {
@@ -2245,7 +2225,7 @@ __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
 #pragma unroll
           for (int c = 0; c < CG; ++c) {
             bf16x8 pp[1];
-            bf3_weights<BK>(wr[d][c], q, t3, zp, pp);
+            bf3_weights<BK>(wr[d][c], q, t3, pp);
             bv[q][c][0] = pp[0];
           }
         load_x(min(u + D, last), xf[d], xin[d]);
@@ -2267,7 +2247,7 @@ __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
         for (int q = 0; q < 2; ++q) {
           bf16x8 bv[CG][NP];
 #pragma unroll
-          for (int c = 0; c < CG; ++c) bf3_weights<BK>(wr[d][c], q, t3, zp, bv[c]);
+          for (int c = 0; c < CG; ++c) bf3_weights<BK>(wr[d][c], q, t3, bv[c]);
 #pragma unroll
           for (int p = 0; p < 3; ++p) mfma_part(SUMS ? part : acc, SUMS ? low : acc, buf, q, p, bv);
         }
@@ -2317,7 +2297,6 @@ __global__ void __launch_bounds__(64 * KG * CW) gemm_bf3r_kernel(GemmArgs a, con
   __shared__ uint16_t Xs[NB][KG][3][BM][kBf3Row];
   __shared__ float ex[KG - 1][CW][4][64];
   __shared__ uint2 t3[16];
-  const float zp = BK == BK_U8 ? u8_centre(a.scale, a.minv) : 0.0f;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int grp = wv / CW, cw = wv % CW, gt = tid & (64 * CW - 1);
   const int j = lane & 15, g = lane >> 4;
@@ -2412,7 +2391,7 @@ __global__ void __launch_bounds__(64 * KG * CW) gemm_bf3r_kernel(GemmArgs a, con
       if (r >= rounds) goto done;
       bf16x8 bv[2][NP];
 #pragma unroll
-      for (int q = 0; q < 2; ++q) bf3_weights<BK>(wr[d], q, t3, zp, bv[q]);
+      for (int q = 0; q < 2; ++q) bf3_weights<BK>(wr[d], q, t3, bv[q]);
       load_x(min(r + D, last), xf[d], xin[d]);
       load_w(min(r + D, last), wr[d]);
 #pragma unroll
@@ -2473,13 +2452,13 @@ __device__ inline double split_nan_fix(const GemmArgs &a, int kind, int m, int n
 // a volume training step the pre of the layer below, act its piecewise
 // activation: the derivative act_deriv_kernel would apply, the same
 // expression as gemm_regt_kernel's NEXT epilogue).
-// FIX: the split-x kinds with a row-sum term or a NaN recomputation
-// (SplitFix); an instantiation of its own, since that code costs
-// the plain reduction 3%.
+// FIX: the split-x kinds from BK_B16 on whose NaN sums are recomputed
+// (fix_kind); an instantiation of its own, since that code costs the plain
+// reduction 3%.
 template <bool FWD, bool FIX = false>
 __global__ void __launch_bounds__(256) sk_reduce_kernel(GemmArgs a, const double *bias, int bias_len,
                                                         int act, float *out, float *post,
-                                                        const float *next_pre, SplitFix fx) {
+                                                        const float *next_pre, int fix_kind) {
   const int t = blockIdx.x;
   const int b0 = (int)((int64_t)t * a.nst / a.per_block);
   const int b1 = (int)(((int64_t)(t + 1) * a.nst - 1) / a.per_block);
@@ -2519,8 +2498,7 @@ __global__ void __launch_bounds__(256) sk_reduce_kernel(GemmArgs a, const double
   for (int i = 0; i < 4; ++i) {
     if (a.post != 1.0f) sum[i] *= (double)a.post;
     if constexpr (FIX) {
-      if (fx.rowsum != nullptr) sum[i] += fx.offset * fx.rowsum[m];
-      if (i < nv && isnan(sum[i])) sum[i] = split_nan_fix(a, fx.kind, m, n + i);
+      if (i < nv && isnan(sum[i])) sum[i] = split_nan_fix(a, fix_kind, m, n + i);
     }
     float p = (float)sum[i];
     if constexpr (FWD) {
@@ -2599,17 +2577,6 @@ __global__ void __launch_bounds__(256) sk_reduce_pair_kernel(GemmArgs a, float p
       h[idx + i] = hv[i];
     }
   }
-}
-
-// out[m] = sum over k of A [m][k], f64.
-__global__ void __launch_bounds__(256) rowsum_kernel(const float *__restrict__ A, int K, double *out) {
-  __shared__ double red[4];
-  double s = 0.0;
-  for (int k = threadIdx.x; k < K; k += 256) s += (double)A[(int64_t)blockIdx.x * K + k];
-  s = wave_sum(s);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) out[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
 __global__ void __launch_bounds__(256) reduce_plain_kernel(const float *ws, int slices, int64_t total,
@@ -3017,17 +2984,16 @@ int bf3_kind(const DevStore &w) {
 int bf3_fwd_kind(const DevStore &w, int batch) {
   const int bk = bf3_kind(w);
   if (bk >= 0 || knob(kTuneBf3) == 0 || batch <= 16 || w.cols % 16 != 0) return bk;
-  const int64_t units = (int64_t)((batch + 31) / 32) * ((w.rows + 127) / 128) * ((w.cols + kBK - 1) / kBK);
   switch (w.dtype) {
   case kBFloat16: return BK_B16;
   case kFloat16: return BK_H16;
   // six products: fewer outputs than 512 lose to the fp32 MFMA's narrower
-  // tiles (768 -> 300 b256 12.8 us against 11.1, 512^2 10.1 against 10.3)
+  // tiles (Float32 768 -> 300 b256 12.8 us against 11.1, 512^2 10.1 against
+  // 10.3; Uint8 from 512 on: 16 -> 512 b64 9.0 -> 6.9, 1024^2 b512 26.8 ->
+  // 22.7, 4096 -> 11008 b256 236 -> 171)
   case kFloat32: return w.rows >= 512 ? BK_F32 : -1;
+  case kUint8: return w.rows >= 512 ? BK_U8 : -1;
   case kInt4: return BK_I4;
-  // its row sums are a launch of their own (1024^2 b100, 512 units: 14.8 us
-  // against 14.0 on the fp32 MFMA; 2048^2 b48, 1024 units: 17.5 / 19.3)
-  case kUint8: return units >= 1024 ? BK_U8 : -1;
   }
   return -1;
 }
@@ -3090,11 +3056,8 @@ bool reg_gemm_ok(int f) { return f >= 0 && fmt_chunk_elems(f) >= 8; }  // format
 
 // The factor the reduction applies for a kind whose codes carry no scale.
 float bf3_post(const DevStore &w, int bk) {
-  return (bk == BK_I8 || bk == BK_NF4 || bk == BK_U8) ? w.scale : bk == BK_I4 ? w.scale * 0.0625f : 1.0f;
+  return (bk == BK_I8 || bk == BK_NF4) ? w.scale : bk == BK_I4 ? w.scale * 0.0625f : 1.0f;
 }
-
-// Row sums of x for Uint8 on the split-x GEMM, at the end of the workspace.
-size_t rowsum_bytes(int M) { return ((size_t)M * sizeof(double) + 15) / 16 * 16; }
 
 // Forward GEMM plan: the split-x bf16 kernel for the formats it takes, the
 // register-B kernel for other <= 16-bit formats, else the LDS-staged kernel.
@@ -3111,12 +3074,13 @@ SkPlan plan_fwd_gemm(int f, int bk, int M, int K, int N, int share = 1) {
     // 11008 b128 50.6 / 47.3) and up to 4096 for NF4 (2048 -> 8192 b64 22.5 /
     // 23.5, b256 60.8 / 56.5).  The 16-bit kinds gain nothing from the groups
     // there (twice the weight registers): 32 x 128 up to 4096 units (4096^2
-    // b64 18.3 / 21.9, b100 27.0 / 24.6), Float32 64 x 128 tiles beyond 1024
+    // b64 18.3 / 21.9, b100 27.0 / 24.6), Float32 and Uint8 64 x 128 tiles beyond 1024
     // (4096^2 b64 26.5 us, 32 x 128 28.7, 64 x 256 29.7; 4096 -> 11008 b512
     // 329 / - / 339).
     const int64_t units = (int64_t)((M + 31) / 32) * ((N + 127) / 128) * stages;
-    const bool wide_codes = bk == BK_B16 || bk == BK_H16 || bk == BK_F32;
-    const bool small = units <= (bk == BK_F32 ? 1024 : wide_codes ? 4096 : 2048);
+    const bool six = bk == BK_F32 || bk == BK_U8;  // products per weight
+    const bool wide_codes = bk == BK_B16 || bk == BK_H16 || six;
+    const bool small = units <= (six ? 1024 : wide_codes ? 4096 : 2048);
     const bool mid = !wide_codes && stages % 2 == 0 && units <= (bk == BK_NF4 ? 4096 : 8192);
     const int bm = M <= 16 ? 16 : (M <= 32 || small || mid) ? 32 : 64;
     // tile width: 128 output columns where outputs are few (N <= 8192) for
@@ -3127,7 +3091,7 @@ SkPlan plan_fwd_gemm(int f, int bk, int M, int K, int N, int share = 1) {
     // -> 11008 b8 FP8 19.6 against 20.1; the 4-bit kinds' 32-row tile keeps
     // the two-group workgroups, which need 256)
     const bool four_bit = bk == BK_NF4 || bk == BK_FP4 || bk == BK_I4;
-    const bool narrow = bk == BK_F32 || (M <= 16 ? N <= 8192 : M <= 32 ? N <= 8192 && !four_bit : small);
+    const bool narrow = six || (M <= 16 ? N <= 8192 : M <= 32 ? N <= 8192 && !four_bit : small);
     const int bn = narrow ? 128 : 256;
     // no k split for K <= 2048 (measured at batch 5-16: 1024^2 6.6 against
     // 10.3 us, 2048 -> 4096 9.4 against 14.3; at K = 4096 about even, at
@@ -3174,7 +3138,6 @@ SkPlan plan_fwd_gemm(int f, int bk, int M, int K, int N, int share = 1) {
     // time.  BFloat16 and Int4 stay below the fp32 MFMA's without them.
     const bool took_over = bk != BK_B16 && bk != BK_I4 && M > (bk < BK_B16 ? 32 : 16);
     if (bm <= 32 && (share > 1 || took_over)) p.sums = true;
-    if (bk == BK_U8) p.ws_bytes += rowsum_bytes(M);
     return p;
   }
   // batch <= 16 without a k split (gemm_regr_kernel): K <= 2048 as for the
@@ -3366,13 +3329,13 @@ hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
   else if (p.bn == 128) gemm_bf3_kernel<BK, 1, 1, 1, true><<<grid, 256, 0, s>>>(a);        \
   else gemm_bf3_kernel<BK, 1, 1, 2, true><<<grid, 256, 0, s>>>(a);
     switch (bk) {
-    case BK_I4: WH_GP32(BK_I4) break;  // batches above 16 only, as the next four
-    case BK_U8: WH_GP32(BK_U8) break;
+    case BK_I4: WH_GP32(BK_I4) break;  // batches above 16 only, as the next four kinds
     case BK_B16: WH_GP32N(BK_B16) break;
     case BK_H16: WH_GP32N(BK_H16) break;
-    case BK_F32:  // 32 x 128 tiles only
+    case BK_F32: case BK_U8:  // 128-column tiles only
       if (p.bn != 128) return hipErrorInvalidValue;
-      gemm_bf3_kernel<BK_F32, 1, 1, 1, true><<<grid, 256, 0, s>>>(a);
+      if (bk == BK_F32) gemm_bf3_kernel<BK_F32, 1, 1, 1, true><<<grid, 256, 0, s>>>(a);
+      else gemm_bf3_kernel<BK_U8, 1, 1, 1, true><<<grid, 256, 0, s>>>(a);
       break;
     case BK_E4: WH_GP(BK_E4) break;
     case BK_I8: WH_GP(BK_I8) break;
@@ -3406,7 +3369,6 @@ hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
     case BK_B16: WH_GK(BK_B16) break;
     case BK_H16: WH_GK(BK_H16) break;
     case BK_I4: WH_GK(BK_I4) break;
-    case BK_U8: WH_GK(BK_U8) break;
     case BK_E4: WH_GK(BK_E4) break;
     case BK_I8: WH_GK(BK_I8) break;
     case BK_FP4: WH_GK(BK_FP4) break;
@@ -3428,13 +3390,13 @@ hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
   switch (bk) {
   case BK_B16: WH_GB32(BK_B16) break;
   case BK_H16: WH_GB32(BK_H16) break;
-  case BK_F32:  // 128-column tiles only (plan_fwd_gemm)
-    if (p.bn != 128) return hipErrorInvalidValue;
-    if (p.bm == 32) gemm_bf3_kernel<BK_F32, 1, 1, 1><<<grid, 256, 0, s>>>(a);
-    else gemm_bf3_kernel<BK_F32, 2, 1, 1><<<grid, 256, 0, s>>>(a);
+  // 128-column tiles, of 32 rows with stage sums only (plan_fwd_gemm)
+  case BK_F32: case BK_U8:
+    if (p.bn != 128 || p.bm != 64) return hipErrorInvalidValue;
+    if (bk == BK_F32) gemm_bf3_kernel<BK_F32, 2, 1, 1><<<grid, 256, 0, s>>>(a);
+    else gemm_bf3_kernel<BK_U8, 2, 1, 1><<<grid, 256, 0, s>>>(a);
     break;
   case BK_I4: WH_GB32(BK_I4) break;
-  case BK_U8: WH_GB32(BK_U8) break;
   case BK_E4: WH_GB(BK_E4) break;
   case BK_I8: WH_GB(BK_I8) break;
   case BK_FP4: WH_GB(BK_FP4) break;
@@ -3679,17 +3641,11 @@ hipError_t launch_forward(const DevStore &w, int batch, const float *x, const do
   if (ws_bytes < p.ws_bytes) return hipErrorInvalidValue;
   GemmArgs a{kernel_body(w, f), w.lut, w.scale, w.minv, x, batch, w.cols, w.rows, row_bytes_of(w),
              p.gx, p.gy, p.nst, p.per_block, p.maxspan, (float *)ws, p.bm, p.bn};
-  SplitFix fx;
+  int fix_kind = -1;
   if (p.bf3) {
     a.post = bf3_post(w, bk);
     if (bk == BK_E4 || bk == BK_E5) a.body = w.kbody;
-    if (bk == BK_B16 || bk == BK_H16 || bk == BK_F32 || bk == BK_U8) fx.kind = bk;
-    if (bk == BK_U8) {
-      fx.offset = (double)w.minv + (double)u8_centre(w.scale, w.minv) * (double)w.scale;
-      double *rs = (double *)((char *)ws + p.ws_bytes - rowsum_bytes(batch));
-      rowsum_kernel<<<batch, 256, 0, s>>>(x, w.cols, rs);
-      fx.rowsum = rs;
-    }
+    if (bk == BK_B16 || bk == BK_H16 || bk == BK_F32 || bk == BK_U8) fix_kind = bk;
     if (p.rows) return launch_bf3r<true>(p, bk, a, bias, bias_len, act, pre, post, s);
     const hipError_t e = launch_bf3(p, bk, a, s);
     if (e != hipSuccess) return e;
@@ -3720,10 +3676,11 @@ hipError_t launch_forward(const DevStore &w, int batch, const float *x, const do
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  if (fx.kind >= 0)
-    sk_reduce_kernel<true, true><<<sk_reduce_grid(p), 256, 0, s>>>(a, bias, bias_len, act, pre, post, nullptr, fx);
+  if (fix_kind >= 0)
+    sk_reduce_kernel<true, true><<<sk_reduce_grid(p), 256, 0, s>>>(a, bias, bias_len, act, pre, post, nullptr,
+                                                                   fix_kind);
   else
-    sk_reduce_kernel<true><<<sk_reduce_grid(p), 256, 0, s>>>(a, bias, bias_len, act, pre, post, nullptr, fx);
+    sk_reduce_kernel<true><<<sk_reduce_grid(p), 256, 0, s>>>(a, bias, bias_len, act, pre, post, nullptr, -1);
   return hipGetLastError();
 }
 
@@ -3952,7 +3909,7 @@ hipError_t launch_backward(const DevStore &w, int batch, const float *x, const f
       e = launch_bf3(p, bk, a, s);
       if (e != hipSuccess) return e;
       sk_reduce_kernel<false><<<sk_reduce_grid(p), 256, 0, s>>>(a, nullptr, 0, chain.dx_next_act, dX, nullptr,
-                                                                chain.dx_next_pre, SplitFix{});
+                                                                chain.dx_next_pre, -1);
     }
   } else if (dx_rows(w, batch)) {
     const int st = dx_rows_stage(f);
@@ -3984,7 +3941,7 @@ hipError_t launch_backward(const DevStore &w, int batch, const float *x, const f
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     sk_reduce_kernel<false><<<sk_reduce_grid(p), 256, 0, s>>>(a, nullptr, 0, chain.dx_next_act, dX, nullptr,
-                                                              chain.dx_next_pre, SplitFix{});
+                                                              chain.dx_next_pre, -1);
   }
   e = hipGetLastError();
   if (e != hipSuccess) return e;

@@ -74,3 +74,15 @@ def test_uint8_decoded_values(oracle, lo, hi):
     pre, _ = pywelvet.forward(W, x, dtype=13)
     Wd = oracle_weights(oracle, 13, W)
     assert error(pre, x.astype(np.float64) @ Wd.T) <= chain_bound(72)
+
+
+@pytest.mark.parametrize("dtype", [1, 13])
+def test_short_k_many_outputs(oracle, dtype):
+    """Six-product kinds at K = 16 and more tiles than 64-row ones start at: two
+    steps of 16 products, the low parts' sum and the output's rounding."""
+    rng = np.random.default_rng(dtype)
+    W = rng.normal(0, 0.1, (8200, 16)).astype(np.float32)
+    x = rng.normal(0, 1, (1100, 16)).astype(np.float32)
+    pre, _ = pywelvet.forward(W, x, dtype=dtype)
+    Wd = oracle_weights(oracle, dtype, W)
+    assert error(pre, x.astype(np.float64) @ Wd.T) <= 2.0 ** -24 * np.sqrt((2 + 1 + 1) / 2)

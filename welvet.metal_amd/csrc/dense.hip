@@ -1740,8 +1740,10 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
         *(uint4 *)&Xs[buf][p][xm][xk + 8 * q] =
             make_uint4(wp[p][4 * q], wp[p][4 * q + 1], wp[p][4 * q + 2], wp[p][4 * q + 3]);
   };
-  // One MFMA step: products of x part p with weight part wp for p + wp <= 2
-  // (the dropped NF4 terms are below 2^-23 of each product).
+  // One MFMA step: products of x part p with weight part wp for p + wp <= 2.
+  // The parts are truncations, so the dropped terms have their product's sign:
+  // up to 3.9 2^-23 of it for three-part weights, 1.7 2^-23 for Float16's two
+  // (6e-8 and 3e-8 of a random sum).
   auto mfma_part = [&](floatx16 (&acc)[MT][NC], floatx16 (&low)[MT][NC], int buf, int q, int p,
                        const bf16x8 (&bv)[NC][NP]) {
 #pragma unroll
@@ -3074,13 +3076,16 @@ SkPlan plan_fwd_gemm(int f, int bk, int M, int K, int N, int share = 1) {
     // 11008 b128 50.6 / 47.3) and up to 4096 for NF4 (2048 -> 8192 b64 22.5 /
     // 23.5, b256 60.8 / 56.5).  The 16-bit kinds gain nothing from the groups
     // there (twice the weight registers): 32 x 128 up to 4096 units (4096^2
-    // b64 18.3 / 21.9, b100 27.0 / 24.6), Float32 and Uint8 64 x 128 tiles beyond 1024
-    // (4096^2 b64 26.5 us, 32 x 128 28.7, 64 x 256 29.7; 4096 -> 11008 b512
-    // 329 / - / 339).
+    // b64 18.3 / 21.9, b100 27.0 / 24.6).  Float32 and Uint8, six products a
+    // weight: 64 x 128 tiles beyond 2048 (4096^2 b64 26.5 us, 32 x 128 28.7, 64
+    // x 256 29.7; at 2048 1024^2 b512 22.4 against 22.7, Uint8 21.9 / 19.5, and
+    // 1.9e-7 from 64 bits against 9.1e-8), but one-stage rows stay on 32 x 128
+    // at any size: without stage sums they are further off than the fp32 MFMA
+    // (K = 16 9.5e-8 against 7.4e-8 and 6.8e-8 with).
     const int64_t units = (int64_t)((M + 31) / 32) * ((N + 127) / 128) * stages;
     const bool six = bk == BK_F32 || bk == BK_U8;  // products per weight
     const bool wide_codes = bk == BK_B16 || bk == BK_H16 || six;
-    const bool small = units <= (six ? 1024 : wide_codes ? 4096 : 2048);
+    const bool small = units <= (wide_codes && !six ? 4096 : 2048) || (six && stages == 1);
     const bool mid = !wide_codes && stages % 2 == 0 && units <= (bk == BK_NF4 ? 4096 : 8192);
     const int bm = M <= 16 ? 16 : (M <= 32 || small || mid) ? 32 : 64;
     // tile width: 128 output columns where outputs are few (N <= 8192) for

@@ -88,3 +88,44 @@ def test_noalloc_keeps_the_batches_it_took(oracle):
         got, _ = run(s, 3584, x, True)
     ref = x.astype(np.float64) @ W.astype(np.float64).T
     assert np.all(np.abs(got - ref) <= elementwise_bound(W.astype(np.float64), x, 1e-5))
+
+
+@pytest.mark.parametrize("dtype", [3, 1], ids=[DTYPE_NAMES[d] for d in (3, 1)])
+def test_nan_redo_is_bounded(dtype):
+    """The recomputation of NaN sums costs a small multiple of the product: a
+    NaN at the end of every row of x next to nothing (such rows need no walk
+    over K), one in every row of W a wave-wide walk per output.  The limits
+    leave a factor of three over what is measured; a serial walk per output
+    takes hundreds of times the product."""
+    import time
+
+    from devmem import DeviceArray, hip
+    n, batch = 2048, 512
+    rng = np.random.default_rng(5)
+    W = rng.normal(0, 0.1, (n, n)).astype(np.float32)
+    x = rng.normal(0, 1, (batch, n)).astype(np.float32)
+    d_x, d_pre, d_post = DeviceArray((batch, n)), DeviceArray((batch, n)), DeviceArray((batch, n))
+
+    def best(W, x):
+        d_x.upload(x)
+        with pywelvet.Session(W, batch=batch, act=-1, dtype=dtype) as s:
+            t = []
+            for _ in range(6):
+                hip().hipDeviceSynchronize()
+                t0 = time.perf_counter()
+                s.forward_device(d_x.ptr, d_pre.ptr, d_post.ptr)
+                hip().hipDeviceSynchronize()
+                t.append(time.perf_counter() - t0)
+        return min(t), d_pre.download()
+
+    xn, Wn = x.copy(), W.copy()
+    xn[:, -1] = np.nan
+    Wn[:, -1] = np.nan
+    plain, _ = best(W, x)
+    in_x, got = best(W, xn)
+    assert np.isnan(got).all()
+    in_w, got = best(Wn, x)
+    assert np.isnan(got).all()
+    print(f"plain {plain * 1e6:.0f} us, NaN in x {in_x * 1e6:.0f}, in W {in_w * 1e6:.0f}", flush=True)
+    assert in_x < 4 * plain
+    assert in_w < 60 * plain

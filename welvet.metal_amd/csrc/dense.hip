@@ -2428,23 +2428,70 @@ done:
   }
 }
 
-// A NaN sum of a split product, redone on the whole operands: a part of x or
+// Weights k .. k + 3 of a row (k a multiple of 4), as the store decodes them.
+__device__ inline void row_values(const uint8_t *row, int kind, int k, float scale, float minv, float (&w)[4]) {
+  if (kind == BK_F32) {
+    const float4 v = *(const float4 *)(row + 4 * (int64_t)k);
+    w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+  } else if (kind == BK_U8) {
+    const uint32_t v = *(const uint32_t *)(row + k);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = (float)((v >> (8 * e)) & 0xffu) * scale + minv;
+  } else {  // BK_B16, BK_H16
+    const uint2 v = *(const uint2 *)(row + 2 * (int64_t)k);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t c = ((e < 2 ? v.x : v.y) >> (16 * (e & 1))) & 0xffffu;
+      w[e] = kind == BK_B16 ? u2f(c << 16) : (float)__builtin_bit_cast(_Float16, (uint16_t)c);
+    }
+  }
+}
+
+// NaN sums of a split product, redone on the whole operands: a part of x or
 // w that is zero times an infinite other operand is NaN, where the product of
 // the whole values is an infinity, and an infinite weight of the next row
-// inside the last k stage meets the zeros that pad x.  The walk ends at the
-// first NaN, so tensors full of them cost little.
-__device__ inline double split_nan_fix(const GemmArgs &a, int kind, int m, int n) {
-  const uint8_t *row = a.body + (int64_t)n * a.row_bytes;
-  double s = 0.0;
-  for (int k = 0; k < a.K && !isnan(s); ++k) {
-    float w;
-    if (kind == BK_B16) w = u2f((uint32_t)((const uint16_t *)row)[k] << 16);
-    else if (kind == BK_H16) w = (float)((const _Float16 *)row)[k];
-    else if (kind == BK_F32) w = ((const float *)row)[k];
-    else w = (float)row[k] * a.scale + a.minv;  // BK_U8
-    s += (double)a.A[(int64_t)m * a.K + k] * (double)w;
+// inside the last k stage meets the zeros that pad x.  A lane holds row m,
+// columns n .. n + 3 (valid where `live`); the wave takes its NaN sums one by
+// one, its lanes along K.  A row of x that holds a NaN needs no walk: 2048^2
+// b512 BFloat16, a call with its wait, 44 us; with a NaN at the end of every
+// row of x 67, and with one in every row of W, whose sums are all walked, 1.1
+// ms (a thread walking for each of its outputs: 3.9 ms either way).
+__device__ inline void split_nan_fix(const GemmArgs &a, int kind, int m, int n, bool live, double (&sum)[4]) {
+  const int lane = threadIdx.x & 63;
+  int row = -1;  // the row of x looked at last, and whether it holds a NaN
+  bool row_nan = false;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint64_t todo = __ballot(live && n + i < a.N && isnan(sum[i]));
+    while (todo != 0) {
+      const int src = __builtin_ctzll(todo);
+      todo &= todo - 1;
+      const int mm = __builtin_amdgcn_readlane(m, src), nn = __builtin_amdgcn_readlane(n, src) + i;
+      const float *x = a.A + (int64_t)mm * a.K;
+      if (mm != row) {
+        bool bad = false;
+        for (int k = 4 * lane; k < a.K; k += 256) {
+          const float4 v = *(const float4 *)(x + k);
+          bad |= isnan(v.x) || isnan(v.y) || isnan(v.z) || isnan(v.w);
+        }
+        row = mm;
+        row_nan = __any(bad);
+      }
+      if (row_nan) continue;  // a NaN already
+      const uint8_t *wr = a.body + (int64_t)nn * a.row_bytes;
+      double s = 0.0;
+#pragma unroll 4
+      for (int k = 4 * lane; k < a.K; k += 256) {
+        const float4 v = *(const float4 *)(x + k);
+        float w[4];
+        row_values(wr, kind, k, a.scale, a.minv, w);
+        s += (double)v.x * (double)w[0] + (double)v.y * (double)w[1] + (double)v.z * (double)w[2] +
+             (double)v.w * (double)w[3];
+      }
+      s = wave_sum(s);
+      if (lane == src) sum[i] = s;
+    }
   }
-  return s;
 }
 
 // Sum of a tile's stream-K partials in workgroup order (f64).  Grid: x =
@@ -2463,12 +2510,18 @@ __global__ void __launch_bounds__(256) sk_reduce_kernel(GemmArgs a, const double
                                                         const float *next_pre, int fix_kind) {
   const int t = blockIdx.x;
   const int b0 = (int)((int64_t)t * a.nst / a.per_block);
-  const int b1 = (int)(((int64_t)(t + 1) * a.nst - 1) / a.per_block);
+  int b1 = (int)(((int64_t)(t + 1) * a.nst - 1) / a.per_block);
   const int tile = a.bm * a.bn;
   const int off = (blockIdx.y * 256 + threadIdx.x) * 4;
-  if (off >= tile) return;
+  if (off >= tile) return;  // whole blocks: tiles are multiples of 1024
   const int m = (t / a.gx) * a.bm + off / a.bn, n = (t % a.gx) * a.bn + off % a.bn;
-  if (m >= a.M) return;
+  const bool live = m < a.M;
+  if constexpr (FIX) {  // a wave stays whole for split_nan_fix
+    if (!__any(live)) return;
+    if (!live) b1 = b0 - 1;
+  } else {
+    if (!live) return;
+  }
   double sum[4] = {0, 0, 0, 0};
   // all loads of a group of 8 partials are issued before the first add
   for (int g = b0; g <= b1; g += 8) {
@@ -2496,12 +2549,13 @@ __global__ void __launch_bounds__(256) sk_reduce_kernel(GemmArgs a, const double
   float pv[4], qv[4];
   const int nv = min(4, a.N - n);
   const int64_t idx = (int64_t)m * a.N + n;
+  if constexpr (FIX) {  // these kinds' weights carry their scale (post is 1)
+    split_nan_fix(a, fix_kind, m, n, live, sum);
+    if (!live) return;
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     if (a.post != 1.0f) sum[i] *= (double)a.post;
-    if constexpr (FIX) {
-      if (i < nv && isnan(sum[i])) sum[i] = split_nan_fix(a, fix_kind, m, n + i);
-    }
     float p = (float)sum[i];
     if constexpr (FWD) {
       if (bias != nullptr && n + i < bias_len) p = (float)((double)p + bias[n + i]);

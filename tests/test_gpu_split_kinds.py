@@ -129,3 +129,47 @@ def test_nan_redo_is_bounded(dtype):
     print(f"plain {plain * 1e6:.0f} us, NaN in x {in_x * 1e6:.0f}, in W {in_w * 1e6:.0f}", flush=True)
     assert in_x < 4 * plain
     assert in_w < 60 * plain
+
+
+@pytest.mark.parametrize("scale,big", [(0.01, 1e37), (1.0, 1e37), (1e38, 1e-3), (1e-44, 1e30), (-0.5, 3e37)])
+def test_int4_extremes(oracle, scale, big):
+    """Int4 stores at both ends of the float range, mounted from native bytes:
+    sums of 16 code x pass the largest float where those of the decoded
+    weights do not, a sixteenth of a small scale is no float, and codes whose
+    value is infinite."""
+    rng = np.random.default_rng(3)
+    raw, _ = oracle.pack(14, rng.normal(0, 1, (70, 128)).astype(np.float32))
+    x = rng.normal(0, 1, (40, 128)).astype(np.float32)
+    if scale == 1e38:  # fp32 sums of its finite values (up to 3e38 |x|, 128 of them) stay below 3.4e38
+        x *= np.float32(1e-3)
+    x[:, 9] = big * rng.choice([-1.0, 0.5, 1.0], 40)
+    Wd = oracle.decode_f64(14, raw, scale, 70 * 128).reshape(70, 128)
+    with pywelvet.Session((70, 128), batch=40, dtype=14, native=(raw, scale)) as s:
+        pre, _ = s.execute(x)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = np.array([[np.sum(x[m].astype(np.float64) * Wd[n]) for n in range(70)] for m in range(40)])
+        ref32 = ref.astype(np.float32)
+        assert np.array_equal(np.isnan(pre), np.isnan(ref32))
+        assert np.array_equal(pre[np.isinf(ref32)], ref32[np.isinf(ref32)])
+        ok = np.isfinite(ref32)
+        bound = elementwise_bound(np.where(np.isfinite(Wd), Wd, 0), x, 1e-5)
+    assert np.all(np.abs(pre[ok] - ref[ok]) <= bound[ok] + 1.5e-45)
+
+
+def test_int4_pair_extremes(oracle):
+    """SwiGLU's Gate and Up in one launch with sums of 16 code x past the
+    largest float: g and u are small, h their product."""
+    rng = np.random.default_rng(4)
+    G, U = (rng.normal(0, 1e-36, (70, 128)).astype(np.float32) for _ in range(2))
+    D = rng.normal(0, 0.1, (128, 70)).astype(np.float32)
+    x = np.zeros((40, 128), np.float32)
+    x[:, 5], x[:, 77] = 2e37, -1e37
+    pre, _ = pywelvet.swiglu_forward(G, U, D, x, dtype=14)
+
+    def decoded(W):
+        raw, s = oracle.pack(14, W)
+        return oracle.decode_f64(14, raw, s, W.size).reshape(W.shape)
+
+    g, u = (x.astype(np.float64) @ decoded(W).T for W in (G, U))
+    ref = g / (1 + np.exp(-g)) * u
+    assert np.all(np.abs(pre - ref) <= 1e-5 * (np.abs(ref) + np.abs(u) + np.abs(g) + 1))

@@ -35,6 +35,7 @@
 // contract.  Float64 storage accumulates in f64 on the GEMV path.
 #include <algorithm>
 #include <atomic>
+#include <cfloat>
 #include <type_traits>
 
 #include "codec.hpp"
@@ -778,8 +779,9 @@ struct GemmArgs {
   float *ws;          // [blocks][maxspan][bm][bn] partial tiles
   int bm, bn;         // tile shape
   // the reduction multiplies sums by post (a per-tensor scale the split-x
-  // GEMM factors out of the weights)
-  float post = 1.0f;
+  // GEMM factors out of the weights; double: a sixteenth of a small scale is
+  // no f32)
+  double post = 1.0;
   // a second store's product with the same x in the same launch (grid y = 1):
   // its body, and its partial tiles this many floats into ws
   const uint8_t *body2 = nullptr;
@@ -1127,7 +1129,7 @@ __global__ void __launch_bounds__(64 * KG) gemm_regr_kernel(GemmArgs a, const do
     double sum = (double)acc[r];
 #pragma unroll
     for (int q = 0; q < KG - 1; ++q) sum += (double)ex[q][r][lane];
-    if (a.post != 1.0f) sum *= (double)a.post;
+    if (a.post != 1.0) sum *= a.post;
     if (m < a.M && n < a.N) bias_act_store(sum, n, bias, bias_len, act, pre, post, (int64_t)m * a.N + n);
   }
 }
@@ -1247,7 +1249,7 @@ __global__ void __launch_bounds__(64 * KG) gemm_regx_kernel(GemmArgs a, const do
     double sum = (double)acc[r];
 #pragma unroll
     for (int q = 0; q < KG - 1; ++q) sum += (double)ex[q][r][lane];
-    if (a.post != 1.0f) sum *= (double)a.post;
+    if (a.post != 1.0) sum *= a.post;
     if (m < a.M && n < a.N) bias_act_store(sum, n, bias, bias_len, act, pre, post, (int64_t)m * a.N + n);
   }
 }
@@ -1460,7 +1462,7 @@ __global__ void __launch_bounds__(64 * KG) gemm_regt_kernel(GemmArgs a, float *o
     double sum = (double)acc[r];
 #pragma unroll
     for (int q = 0; q < KG - 1; ++q) sum += (double)ex[q][r][lane];
-    if (a.post != 1.0f) sum *= (double)a.post;
+    if (a.post != 1.0) sum *= a.post;
     float v = (float)sum;
     if constexpr (NEXT) v = v * act_prime_piecewise(np[r], next_act);
     if (m < a.M && n < a.N) out[(int64_t)m * a.N + n] = v;
@@ -2420,7 +2422,7 @@ done:
       double sum = (double)acc[i];
 #pragma unroll
       for (int q = 0; q < KG - 1; ++q) sum += (double)ex[q][cw][i][lane];
-      if (a.post != 1.0f) sum *= (double)a.post;
+      if (a.post != 1.0) sum *= a.post;
       const int64_t idx = (int64_t)m * a.N + col;
       if constexpr (FWD) bias_act_store(sum, col, bias, bias_len, act, out, post, idx);
       else out[idx] = (float)sum;
@@ -2437,6 +2439,10 @@ __device__ inline void row_values(const uint8_t *row, int kind, int k, float sca
     const uint32_t v = *(const uint32_t *)(row + k);
 #pragma unroll
     for (int e = 0; e < 4; ++e) w[e] = (float)((v >> (8 * e)) & 0xffu) * scale + minv;
+  } else if (kind == BK_I4) {
+    const uint32_t v = *(const uint16_t *)(row + (k >> 1));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = (float)((int32_t)(v << (28 - 4 * e)) >> 28) * scale;
   } else {  // BK_B16, BK_H16
     const uint2 v = *(const uint2 *)(row + 2 * (int64_t)k);
 #pragma unroll
@@ -2450,19 +2456,21 @@ __device__ inline void row_values(const uint8_t *row, int kind, int k, float sca
 // NaN sums of a split product, redone on the whole operands: a part of x or
 // w that is zero times an infinite other operand is NaN, where the product of
 // the whole values is an infinity, and an infinite weight of the next row
-// inside the last k stage meets the zeros that pad x.  A lane holds row m,
-// columns n .. n + 3 (valid where `live`); the wave takes its NaN sums one by
+// inside the last k stage meets the zeros that pad x.  Int4's infinities are
+// redone too: its sums are 16 code x before the scale, and pass the largest
+// float where the products of the decoded weights need not.  A lane holds row
+// m, columns n .. n + 3 (valid where `live`); the wave takes its sums one by
 // one, its lanes along K.  A row of x that holds a NaN needs no walk: 2048^2
 // b512 BFloat16, a call with its wait, 44 us; with a NaN at the end of every
 // row of x 67, and with one in every row of W, whose sums are all walked, 1.1
 // ms (a thread walking for each of its outputs: 3.9 ms either way).
-__device__ inline void split_nan_fix(const GemmArgs &a, int kind, int m, int n, bool live, double (&sum)[4]) {
+__device__ inline void split_redo(const GemmArgs &a, int kind, int m, int n, uint32_t mine, double (&sum)[4]) {
   const int lane = threadIdx.x & 63;
   int row = -1;  // the row of x looked at last, and whether it holds a NaN
   bool row_nan = false;
-#pragma unroll
+#pragma unroll 1
   for (int i = 0; i < 4; ++i) {
-    uint64_t todo = __ballot(live && n + i < a.N && isnan(sum[i]));
+    uint64_t todo = __ballot((mine >> i & 1) != 0);
     while (todo != 0) {
       const int src = __builtin_ctzll(todo);
       todo &= todo - 1;
@@ -2480,7 +2488,6 @@ __device__ inline void split_nan_fix(const GemmArgs &a, int kind, int m, int n, 
       if (row_nan) continue;  // a NaN already
       const uint8_t *wr = a.body + (int64_t)nn * a.row_bytes;
       double s = 0.0;
-#pragma unroll 4
       for (int k = 4 * lane; k < a.K; k += 256) {
         const float4 v = *(const float4 *)(x + k);
         float w[4];
@@ -2489,9 +2496,18 @@ __device__ inline void split_nan_fix(const GemmArgs &a, int kind, int m, int n, 
              (double)v.w * (double)w[3];
       }
       s = wave_sum(s);
-      if (lane == src) sum[i] = s;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (lane == src && e == i) sum[e] = s;
     }
   }
+}
+__device__ inline void split_nan_fix(const GemmArgs &a, int kind, int m, int n, bool live, double (&sum)[4]) {
+  uint32_t mine = 0;  // bit i: sum i is to be redone
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (live && n + i < a.N && (kind == BK_I4 ? !isfinite(sum[i]) : isnan(sum[i]))) mine |= 1u << i;
+  if (__builtin_expect(__any(mine != 0), 0)) split_redo(a, kind, m, n, mine, sum);
 }
 
 // Sum of a tile's stream-K partials in workgroup order (f64).  Grid: x =
@@ -2501,7 +2517,7 @@ __device__ inline void split_nan_fix(const GemmArgs &a, int kind, int m, int n, 
 // a volume training step the pre of the layer below, act its piecewise
 // activation: the derivative act_deriv_kernel would apply, the same
 // expression as gemm_regt_kernel's NEXT epilogue).
-// FIX: the split-x kinds from BK_B16 on whose NaN sums are recomputed
+// FIX: the split-x kinds from BK_B16 on, whose sums split_nan_fix looks at
 // (fix_kind); an instantiation of its own, since that code costs the plain
 // reduction 3%.
 template <bool FWD, bool FIX = false>
@@ -2510,18 +2526,15 @@ __global__ void __launch_bounds__(256) sk_reduce_kernel(GemmArgs a, const double
                                                         const float *next_pre, int fix_kind) {
   const int t = blockIdx.x;
   const int b0 = (int)((int64_t)t * a.nst / a.per_block);
-  int b1 = (int)(((int64_t)(t + 1) * a.nst - 1) / a.per_block);
+  const int b1 = (int)(((int64_t)(t + 1) * a.nst - 1) / a.per_block);
   const int tile = a.bm * a.bn;
   const int off = (blockIdx.y * 256 + threadIdx.x) * 4;
   if (off >= tile) return;  // whole blocks: tiles are multiples of 1024
   const int m = (t / a.gx) * a.bm + off / a.bn, n = (t % a.gx) * a.bn + off % a.bn;
   const bool live = m < a.M;
-  if constexpr (FIX) {  // a wave stays whole for split_nan_fix
-    if (!__any(live)) return;
-    if (!live) b1 = b0 - 1;
-  } else {
-    if (!live) return;
-  }
+  // FIX: a wave stays whole for split_nan_fix; lanes past M add what their part
+  // of the tile's memory holds
+  if (FIX ? !__any(live) : !live) return;
   double sum[4] = {0, 0, 0, 0};
   // all loads of a group of 8 partials are issued before the first add
   for (int g = b0; g <= b1; g += 8) {
@@ -2549,13 +2562,15 @@ __global__ void __launch_bounds__(256) sk_reduce_kernel(GemmArgs a, const double
   float pv[4], qv[4];
   const int nv = min(4, a.N - n);
   const int64_t idx = (int64_t)m * a.N + n;
-  if constexpr (FIX) {  // these kinds' weights carry their scale (post is 1)
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (a.post != 1.0) sum[i] *= a.post;
+  if constexpr (FIX) {
     split_nan_fix(a, fix_kind, m, n, live, sum);
     if (!live) return;
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    if (a.post != 1.0f) sum[i] *= (double)a.post;
     float p = (float)sum[i];
     if constexpr (FWD) {
       if (bias != nullptr && n + i < bias_len) p = (float)((double)p + bias[n + i]);
@@ -2578,8 +2593,10 @@ __global__ void __launch_bounds__(256) sk_reduce_kernel(GemmArgs a, const double
 
 // The reduction of a pair launch: g and u are the two stores' products (each
 // as sk_reduce_kernel sums one), h = fl32(silu(g)) * u, op_swiglu's product.
-__global__ void __launch_bounds__(256) sk_reduce_pair_kernel(GemmArgs a, float post2, float *g_pre, float *u_pre,
-                                                             float *h) {
+// FIX: Int4, as there (scale2: the second store's).
+template <bool FIX>
+__global__ void __launch_bounds__(256) sk_reduce_pair_kernel(GemmArgs a, double post2, float scale2, float *g_pre,
+                                                             float *u_pre, float *h) {
   const int t = blockIdx.x;
   const int b0 = (int)((int64_t)t * a.nst / a.per_block);
   const int b1 = (int)(((int64_t)(t + 1) * a.nst - 1) / a.per_block);
@@ -2587,7 +2604,10 @@ __global__ void __launch_bounds__(256) sk_reduce_pair_kernel(GemmArgs a, float p
   const int off = (blockIdx.y * 256 + threadIdx.x) * 4;
   if (off >= tile) return;
   const int m = (t / a.gx) * a.bm + off / a.bn, n = (t % a.gx) * a.bn + off % a.bn;
-  if (m >= a.M) return;
+  const bool live = m < a.M;
+  // FIX: a wave stays whole for split_nan_fix; lanes past M add what their part
+  // of the tile's memory holds
+  if (FIX ? !__any(live) : !live) return;
   double sum[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
   for (int g = b0; g <= b1; g += 4) {
     float4 v[2][4];
@@ -2613,13 +2633,26 @@ __global__ void __launch_bounds__(256) sk_reduce_pair_kernel(GemmArgs a, float p
         }
       }
   }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    sum[0][i] *= a.post;
+    sum[1][i] *= post2;
+  }
+  if constexpr (FIX) {
+    split_nan_fix(a, BK_I4, m, n, live, sum[0]);
+    GemmArgs b = a;
+    b.body = a.body2;
+    b.scale = scale2;
+    split_nan_fix(b, BK_I4, m, n, live, sum[1]);
+    if (!live) return;
+  }
   float gv[4], uv[4], hv[4];
   const int nv = min(4, a.N - n);
   const int64_t idx = (int64_t)m * a.N + n;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    gv[i] = (float)(sum[0][i] * (double)a.post);
-    uv[i] = (float)(sum[1][i] * (double)post2);
+    gv[i] = (float)sum[0][i];
+    uv[i] = (float)sum[1][i];
     hv[i] = i < nv ? act_value(gv[i], kSilu) * uv[i] : 0.0f;
   }
   if (nv == 4 && (a.N & 3) == 0) {
@@ -3049,7 +3082,8 @@ int bf3_fwd_kind(const DevStore &w, int batch) {
   // 22.7, 4096 -> 11008 b256 236 -> 171)
   case kFloat32: return w.rows >= 512 ? BK_F32 : -1;
   case kUint8: return w.rows >= 512 ? BK_U8 : -1;
-  case kInt4: return BK_I4;
+  // its codes must decode to finite values
+  case kInt4: return fabsf(w.scale) <= FLT_MAX / 8 ? BK_I4 : -1;
   }
   return -1;
 }
@@ -3111,8 +3145,8 @@ bool reg_gemm_ok(int f) { return f >= 0 && fmt_chunk_elems(f) >= 8; }  // format
 
 
 // The factor the reduction applies for a kind whose codes carry no scale.
-float bf3_post(const DevStore &w, int bk) {
-  return (bk == BK_I8 || bk == BK_NF4) ? w.scale : bk == BK_I4 ? w.scale * 0.0625f : 1.0f;
+double bf3_post(const DevStore &w, int bk) {
+  return (bk == BK_I8 || bk == BK_NF4) ? w.scale : bk == BK_I4 ? w.scale * 0.0625 : 1.0;
 }
 
 // Forward GEMM plan: the split-x bf16 kernel for the formats it takes, the
@@ -3704,7 +3738,7 @@ hipError_t launch_forward(const DevStore &w, int batch, const float *x, const do
   if (p.bf3) {
     a.post = bf3_post(w, bk);
     if (bk == BK_E4 || bk == BK_E5) a.body = w.kbody;
-    if (bk == BK_B16 || bk == BK_H16 || bk == BK_F32 || bk == BK_U8) fix_kind = bk;
+    if (bk >= BK_B16) fix_kind = bk;
     if (p.rows) return launch_bf3r<true>(p, bk, a, bias, bias_len, act, pre, post, s);
     const hipError_t e = launch_bf3(p, bk, a, s);
     if (e != hipSuccess) return e;
@@ -3781,7 +3815,10 @@ hipError_t launch_forward_pair_gemm(const DevStore &g, const DevStore &u, int ba
   if (a.body == nullptr || a.body2 == nullptr) return hipErrorInvalidValue;
   const hipError_t e = launch_bf3(p, bk, a, s);
   if (e != hipSuccess) return e;
-  sk_reduce_pair_kernel<<<sk_reduce_grid(p), 256, 0, s>>>(a, bf3_post(u, bk), g_pre, u_pre, h);
+  if (bk == BK_I4)
+    sk_reduce_pair_kernel<true><<<sk_reduce_grid(p), 256, 0, s>>>(a, bf3_post(u, bk), u.scale, g_pre, u_pre, h);
+  else
+    sk_reduce_pair_kernel<false><<<sk_reduce_grid(p), 256, 0, s>>>(a, bf3_post(u, bk), u.scale, g_pre, u_pre, h);
   return hipGetLastError();
 }
 
@@ -3961,7 +3998,7 @@ hipError_t launch_backward(const DevStore &w, int batch, const float *x, const f
     const SkPlan p = plan_fwd_gemm(f, bk, batch, w.rows, w.cols);
     GemmArgs a{w.tbody, w.lut, w.scale, w.minv, dpre, batch, w.rows, w.cols, (int64_t)w.rows,
                p.gx, p.gy, p.nst, p.per_block, p.maxspan, (float *)ws, p.bm, p.bn};
-    a.post = bk == BK_I8 ? w.scale : 1.0f;
+    a.post = bk == BK_I8 ? w.scale : 1.0;
     if (p.rows) {
       e = launch_bf3r<false>(p, bk, a, nullptr, 0, -1, dX, nullptr, s);
     } else {

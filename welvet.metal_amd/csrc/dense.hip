@@ -3209,17 +3209,20 @@ SkPlan plan_fwd_gemm(int f, int bk, int M, int K, int N, int share = 1) {
     // slower there)
     const bool groups = bn == 256 && stages % 2 == 0 && (bm == 64 || (bm == 32 && (M > 32 || four_bit)));
     // Tiles of up to 32 rows: shares of at least a sixteenth of K, or of four
-    // units where that is less (three of NF4's two-group tiles, which take
-    // longest): past it the reduction's serial sum costs more than the shorter
-    // shares save (FP8 32 x 128 tiles, 4096 -> 512 b48 19.2 -> 11.7 us, 1024^2
-    // b100 11.9 -> 9.5; 16 x 128 tiles 4096 -> 512 b13 17.0 -> 10.3; NF4 4096 ->
-    // 512 b33 16.9 -> 12.4), and longer ones idle the CUs and lose precision
-    // (a sixteenth at K = 11008: NF4 11008 -> 1024 b17 19.7 -> 24.4 us, FP4
-    // 11008 -> 128 b8 9.2e-8 -> 1.0e-7 from 64 bits).  Only with stage sums:
-    // without them the error of longer shares triples (Float16 11008 -> 128
-    // b33 1.5e-7 -> 3.9e-7).
+    // units where that is less (six where shares of that many still give every
+    // CU one; three of NF4's two-group tiles, which take longest): past it the
+    // reduction's serial sum costs more than the shorter shares save (FP8 32 x
+    // 128 tiles, 4096 -> 512 b48 19.2 -> 11.7 us, 1024^2 b100 11.9 -> 9.5; 16 x
+    // 128 tiles 4096 -> 512 b13 17.0 -> 10.3; NF4 4096 -> 512 b33 16.9 -> 12.4;
+    // 8192 -> 300 b100 17.3 at four, 15.0 at six), and longer ones idle the CUs
+    // and lose precision (a sixteenth at K = 11008: NF4 11008 -> 1024 b17 19.7
+    // -> 24.4 us, FP4 11008 -> 128 b8 9.2e-8 -> 1.0e-7 from 64 bits).  Only with
+    // stage sums: without them the error of longer shares triples (Float16
+    // 11008 -> 128 b33 1.5e-7 -> 3.9e-7).
     const int units_k = groups ? stages / 2 : stages;
-    const int least = bm <= 32 ? std::min((units_k + 15) / 16, groups && bk == BK_NF4 ? 3 : 4) : 1;
+    const int64_t per_cu = ((int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * units_k + num_cus() - 1) / num_cus();
+    const int most = groups && bk == BK_NF4 ? 3 : (int)std::min<int64_t>(6, std::max<int64_t>(4, per_cu));
+    const int least = bm <= 32 ? std::min((units_k + 15) / 16, most) : 1;
     SkPlan p = groups ? plan_sk(M, K, N, bm, bn, 1, 2, share, least)
                       : plan_sk(M, K, N, bm, bn, occ, 1, share, least);
     p.bf3 = true;

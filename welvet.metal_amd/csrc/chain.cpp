@@ -51,7 +51,7 @@ struct Chain {
   }
   template <class T>
   welvet_status alloc(T **p, int64_t elems) {
-    WH_HIP(hipMalloc((void **)p, (size_t)std::max<int64_t>(elems, 1) * sizeof(T)));
+    WH_HIP(dev_malloc(p, (size_t)std::max<int64_t>(elems, 1) * sizeof(T)));
     bufs.push_back(*p);
     return ok();
   }
@@ -96,7 +96,7 @@ welvet_status make(Chain *L, bool residual, int rows, int dim, int depth, int ac
   size_t need = mse_workspace_bytes(n);
   for (const Store &w : L->child)
     need = std::max({need, forward_workspace_bytes(w.dev(), rows), backward_workspace_bytes(w.dev(), rows)});
-  WH_HIP(hipMalloc(&L->ws, need));
+  WH_HIP(dev_malloc(&L->ws, need));
   L->ws_bytes = need;
   return ok();
 }

@@ -16,8 +16,9 @@
 // Device memory.  A call's hipMalloc and hipFree (which waits for the whole
 // device) are a tenth of a one-shot call: 1024^2 Float16 b32 NormalBP 1308 ->
 // 1145 us, forward 425 -> 359 with DevBuf's pool of freed blocks (at most 256
-// MB in all, larger blocks are not kept, everything is given back when an
-// allocation fails).  A block returns to the pool only after its stream has
+// MB in all, larger blocks are not kept; every device allocation of the
+// library goes through dev_malloc, which gives all idle blocks back and tries
+// again where memory runs out).  A block returns to the pool only after its stream has
 // drained.  A resident store's mount allocates and frees its staging buffers
 // outside the pool: a grid whose mounts kept them there paid for it in its
 // first training step (32 layers of 1024^2: 1.5-2.0 ms -> 1.6-6.3), where the
@@ -213,6 +214,16 @@ DevPool &pool() {
 
 }  // namespace
 
+hipError_t dev_malloc_bytes(void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();  // must not read as a failed launch
+    dev_trim();
+    e = hipMalloc(p, bytes);
+  }
+  return e;
+}
+
 hipError_t dev_alloc(void **p, size_t bytes) try {
   DevPool &d = pool();
   bytes = (std::max<size_t>(bytes, 1) + 4095) / 4096 * 4096;
@@ -237,12 +248,7 @@ hipError_t dev_alloc(void **p, size_t bytes) try {
       return hipSuccess;
     }
   }
-  e = hipMalloc(p, bytes);
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();
-    dev_trim();
-    e = hipMalloc(p, bytes);
-  }
+  e = dev_malloc(p, bytes);
   if (e != hipSuccess) return e;
   try {
     std::lock_guard<std::mutex> lk(d.mu);

@@ -333,7 +333,7 @@ struct StackPass {
   float *alloc(Verdict &v, size_t elems) {
     void *p = nullptr;
     if (!v.ok()) return nullptr;
-    if (!v.hip(hipMalloc(&p, std::max<size_t>(elems, 1) * sizeof(float)))) return nullptr;
+    if (!v.hip(dev_malloc(&p, std::max<size_t>(elems, 1) * sizeof(float)))) return nullptr;
     bufs.push_back(p);
     return static_cast<float *>(p);
   }

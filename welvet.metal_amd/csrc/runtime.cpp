@@ -99,7 +99,7 @@ const char *device_identity() {
 // ------------------------------------------------------- resident store
 template <typename T>
 static hipError_t store_alloc(const Store &w, T **p, size_t bytes) {
-  return w.pooled ? dev_alloc((void **)p, bytes) : hipMalloc((void **)p, bytes);
+  return w.pooled ? dev_alloc((void **)p, bytes) : dev_malloc(p, bytes);
 }
 static void store_free(const Store &w, void *p) {
   if (w.pooled) dev_free(p);
@@ -358,7 +358,7 @@ namespace {
 
 template <typename T>
 hipError_t session_alloc(welvet_dense_session *s, T **p, size_t bytes) {
-  return s->pooled ? dev_alloc((void **)p, bytes) : hipMalloc((void **)p, bytes);
+  return s->pooled ? dev_alloc((void **)p, bytes) : dev_malloc(p, bytes);
 }
 
 void session_free(welvet_dense_session *s) {
@@ -399,6 +399,7 @@ welvet_status ensure_ws(welvet_dense_session *s, size_t bytes) {
     if (s->ws) WH_HIP(hipFree(s->ws));
   }
   s->ws = nullptr;
+  s->ws_bytes = 0;
   WH_HIP(session_alloc(s, &s->ws, bytes));
   s->ws_bytes = bytes;
   return ok();
@@ -799,11 +800,11 @@ welvet_status welvet_hip_mse_f32(const float *pred, const float *target, size_t 
   double *dl = nullptr;
   void *ws = nullptr;
   auto run = [&]() -> welvet_status {
-    WH_HIP(hipMalloc(&dp, n * 4));
-    WH_HIP(hipMalloc(&dt, n * 4));
-    WH_HIP(hipMalloc(&dg, n * 4));
-    WH_HIP(hipMalloc(&dl, 8));
-    WH_HIP(hipMalloc(&ws, mse_workspace_bytes((int64_t)n)));
+    WH_HIP(dev_malloc(&dp, n * 4));
+    WH_HIP(dev_malloc(&dt, n * 4));
+    WH_HIP(dev_malloc(&dg, n * 4));
+    WH_HIP(dev_malloc(&dl, 8));
+    WH_HIP(dev_malloc(&ws, mse_workspace_bytes((int64_t)n)));
     WH_HIP(hipMemcpy(dp, pred, n * 4, hipMemcpyHostToDevice));
     WH_HIP(hipMemcpy(dt, target, n * 4, hipMemcpyHostToDevice));
     WH_HIP(launch_mse(dp, dt, (int64_t)n, loss ? dl : nullptr, grad ? dg : nullptr, ws,

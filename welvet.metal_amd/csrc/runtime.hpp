@@ -35,13 +35,18 @@ const char *device_identity();
 // with hipMemcpyAsync, a host destination holds the data once `s` is synchronised.
 hipError_t copy_to_device(void *dst, const void *src, size_t bytes, hipStream_t s);
 hipError_t copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t s);
+// hipMalloc for everything the library keeps: where memory runs out, again
+// after the pool below has given its idle blocks back.
+hipError_t dev_malloc_bytes(void **p, size_t bytes);
+template <typename T>
+hipError_t dev_malloc(T **p, size_t bytes) { return dev_malloc_bytes((void **)p, bytes); }
 // Device memory for one call's buffers, from a bounded pool of freed blocks.
 // dev_free: no work on the block may be in flight.
 hipError_t dev_alloc(void **p, size_t bytes);
 void dev_free(void *p);
 void dev_trim();  // gives every idle block back
 // A call's buffer, freed when `stream` has drained; pooled: from dev_alloc,
-// else from hipMalloc.
+// else from dev_malloc.
 struct DevBuf {
   void *p = nullptr;
   hipStream_t stream;
@@ -50,7 +55,7 @@ struct DevBuf {
   ~DevBuf();
   DevBuf(const DevBuf &) = delete;
   DevBuf &operator=(const DevBuf &) = delete;
-  hipError_t alloc(size_t bytes) { return pooled ? dev_alloc(&p, bytes) : hipMalloc(&p, bytes); }
+  hipError_t alloc(size_t bytes) { return pooled ? dev_alloc(&p, bytes) : dev_malloc(&p, bytes); }
   template <typename T>
   T *as() const { return (T *)p; }
 };
@@ -70,7 +75,7 @@ struct Store {
   // cleared by an SGD step of a format that can produce them
   bool finite = true;
   // the allocations come from dev_alloc (a store of one call, whose stream
-  // drains before free_store), else from hipMalloc
+  // drains before free_store), else from dev_malloc
   bool pooled = false;
   // transposed codes for dX on the split-x GEMM (tbody_ok: current with body)
   uint8_t *tbody = nullptr;

@@ -50,7 +50,7 @@ struct Swiglu {
   }
   template <class T>
   welvet_status alloc(T **p, int64_t elems) {
-    WH_HIP(hipMalloc((void **)p, (size_t)std::max<int64_t>(elems, 1) * sizeof(T)));
+    WH_HIP(dev_malloc(p, (size_t)std::max<int64_t>(elems, 1) * sizeof(T)));
     bufs.push_back(*p);
     return ok();
   }
@@ -60,7 +60,7 @@ struct Swiglu {
     if (ws) WH_HIP(hipFree(ws));
     ws = nullptr;
     ws_bytes = 0;
-    WH_HIP(hipMalloc(&ws, bytes));
+    WH_HIP(dev_malloc(&ws, bytes));
     ws_bytes = bytes;
     return ok();
   }

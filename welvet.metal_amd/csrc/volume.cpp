@@ -110,7 +110,7 @@ welvet_status grow(float **p, int64_t *have, int64_t elems) {
   if (*p) WH_HIP(hipFree(*p));
   *p = nullptr;
   *have = 0;
-  WH_HIP(hipMalloc(p, (size_t)elems * sizeof(float)));
+  WH_HIP(dev_malloc(p, (size_t)elems * sizeof(float)));
   *have = elems;
   return ok();
 }
@@ -121,7 +121,7 @@ welvet_status grow_ws(Grid *g, size_t bytes) {
   if (g->ws) WH_HIP(hipFree(g->ws));
   g->ws = nullptr;
   g->ws_bytes = 0;
-  WH_HIP(hipMalloc(&g->ws, bytes));
+  WH_HIP(dev_malloc(&g->ws, bytes));
   g->ws_bytes = bytes;
   return ok();
 }
@@ -353,8 +353,8 @@ welvet_status prepare_step(Grid *g, int out_width) {
     Grid::Cell &c = g->cells[idx];
     max_in = std::max<int64_t>(max_in, c.in);
     max_out = std::max<int64_t>(max_out, c.out);
-    if (!c.dW) WH_HIP(hipMalloc(&c.dW, (size_t)c.W.n() * sizeof(float)));
-    if (!c.grad) WH_HIP(hipMalloc(&c.grad, (size_t)g->batch * c.out * sizeof(float)));
+    if (!c.dW) WH_HIP(dev_malloc(&c.dW, (size_t)c.W.n() * sizeof(float)));
+    if (!c.grad) WH_HIP(dev_malloc(&c.grad, (size_t)g->batch * c.out * sizeof(float)));
     welvet_status st = grow_ws(g, backward_workspace_bytes(c.W.dev(), g->batch));
     if (st.code) return st;
   }
@@ -366,7 +366,7 @@ welvet_status prepare_step(Grid *g, int out_width) {
       p = nullptr;
     }
     g->gx_elems = 0;
-    for (float *&p : g->gx) WH_HIP(hipMalloc(&p, (size_t)ng * sizeof(float)));
+    for (float *&p : g->gx) WH_HIP(dev_malloc(&p, (size_t)ng * sizeof(float)));
     g->gx_elems = ng;
   }
   welvet_status st = grow(&g->d_gy, &g->gy_elems, (int64_t)g->batch * out_width);
@@ -401,8 +401,8 @@ welvet_status bind_cell(Grid *g, int z, int y, int x, int l, int in, int out, in
   }
   if (st.code == 0) {
     const size_t yb = (size_t)g->batch * out * sizeof(float);
-    hipError_t e = hipMalloc(&c.pre, yb);
-    if (e == hipSuccess) e = hipMalloc(&c.post, yb);
+    hipError_t e = dev_malloc(&c.pre, yb);
+    if (e == hipSuccess) e = dev_malloc(&c.post, yb);
     if (e == hipSuccess) e = hipStreamSynchronize(g->stream);
     if (e != hipSuccess) st = make_status(kInternal, "hip: %s", hipGetErrorString(e));
   }
@@ -458,7 +458,7 @@ welvet_status welvet_hip_grid_new(int32_t depth, int32_t rows, int32_t cols, int
     return make_status(kInternal, "hip: %s", hipGetErrorString(e));
   };
   const size_t status_bytes = sizeof(double) + (2 + 2 * (size_t)n) * sizeof(int);
-  hipError_t e = hipMalloc(&g->d_status, status_bytes);
+  hipError_t e = dev_malloc(&g->d_status, status_bytes);
   if (e == hipSuccess) e = hipMemset(g->d_status, 0, status_bytes);
   if (e == hipSuccess) e = hipHostMalloc(&g->h_status, status_bytes, hipHostMallocDefault);
   if (e != hipSuccess) return fail(e);
@@ -541,7 +541,7 @@ welvet_status grid_set_batch(welvet_hip_grid *g, int batch) {
     for (float **p : {&c.pre, &c.post}) {
       if (*p) WH_HIP(hipFree(*p));
       *p = nullptr;
-      WH_HIP(hipMalloc(p, (size_t)batch * c.out * sizeof(float)));
+      WH_HIP(dev_malloc(p, (size_t)batch * c.out * sizeof(float)));
     }
     // the training gradient is [batch][out] too: the next step allocates it
     // at the new batch (prepare_step)
@@ -688,7 +688,7 @@ welvet_status welvet_hip_grid_export_f32(welvet_hip_grid *g, int32_t z, int32_t 
   welvet_status st = cell_at(g, z, y, x, l, &c);
   if (st.code) return st;
   float *d = nullptr;
-  WH_HIP(hipMalloc(&d, (size_t)c->W.n() * sizeof(float)));
+  WH_HIP(dev_malloc(&d, (size_t)c->W.n() * sizeof(float)));
   st = store_export(c->W, d, g->stream);
   hipError_t e = hipSuccess;
   if (st.code == 0) e = copy_to_host(W_out, d, (size_t)c->W.n() * sizeof(float), g->stream);

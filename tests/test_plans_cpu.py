@@ -1,0 +1,33 @@
+"""The split-x GEMM's plans and the kernels that serve them, on the CPU:
+tests/native/plans_check.cpp, built host-only."""
+import glob
+import os
+import re
+import subprocess
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "welvet.metal_amd", "csrc")
+OUT = os.path.join(ROOT, "welvet.metal_amd", "_build", "plans")
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+
+def _run(cmd, **kw):
+    r = subprocess.run(cmd, capture_output=True, text=True, **kw)
+    assert r.returncode == 0, f"{' '.join(cmd)}\n{r.stdout[-4000:]}\n{r.stderr[-4000:]}"
+    return r
+
+
+def test_every_plan_has_its_kernel_and_every_kernel_a_plan():
+    src = os.path.join(ROOT, "tests", "native", "plans_check.cpp")
+    exe = os.path.join(OUT, "plans_check")
+    obj = exe + ".o"
+    deps = [src, os.path.join(CSRC, "dense.hip")] + glob.glob(os.path.join(CSRC, "*.hpp"))
+    if not (os.path.exists(exe) and os.path.getmtime(exe) > max(os.path.getmtime(d) for d in deps)):
+        os.makedirs(OUT, exist_ok=True)
+        _run([HIPCC, "-x", "hip", "--offload-host-only", "-fgpu-rdc", "-std=c++17", "-O1", "-ffp-contract=off",
+              "-I", CSRC, "-c", src, "-o", obj])
+        _run([HIPCC, "-fgpu-rdc", "--offload-arch=gfx950", obj, "-o", exe])
+    symbols = _run(["nm", obj]).stdout
+    kernels = set(re.findall(r"__device_stub__gemm_bf3[sk]?_kernel\w*", symbols))
+    r = subprocess.run([exe, str(len(kernels))], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and "plans_check: ok" in r.stdout, r.stdout[-2000:]

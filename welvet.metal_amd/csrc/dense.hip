@@ -3408,101 +3408,73 @@ hipError_t launch_bf3r(const SkPlan &p, int bk, const GemmArgs &a, const double 
   return hipGetLastError();
 }
 
-// The split-x GEMM of plan p for weight kind bk (a.body, a.post set).
-hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
+// The split-x GEMM of plan p for weight kind BK (a.body, a.post set).  Only the
+// kernels that plan_fwd_gemm can ask for exist; any other plan is an error.
+template <int BK>
+hipError_t launch_bf3_kind(const SkPlan &p, GemmArgs &a, hipStream_t s) {
+  constexpr bool small_batch = BK < BK_B16;                 // also batches of 5 to 16
+  constexpr bool six = BK == BK_F32 || BK == BK_U8;         // 128-column tiles
+  constexpr bool tables = BK == BK_FP4 || BK == BK_NF4;
+  constexpr bool four_bit = tables || BK == BK_I4;          // two groups up to batch 32 too
   const dim3 grid(p.blocks, a.body2 != nullptr ? 2 : 1);
-  if (p.sums) {
-#define WH_GP(BK)                                                                             \
-  if (p.bm == 16) {                                                                           \
-    if (p.bn == 128) gemm_bf3s_kernel<BK, 1, 1, true><<<grid, 256, 0, s>>>(a);             \
-    else gemm_bf3s_kernel<BK, 1, 2, true><<<grid, 256, 0, s>>>(a);                         \
-  } else WH_GP32(BK)
-#define WH_GP32(BK)                                                                           \
-  if (p.kg == 2) gemm_bf3k_kernel<BK, 1, 2, 2, true><<<grid, 512, 0, s>>>(a);              \
-  else WH_GP32N(BK)
-#define WH_GP32N(BK)  /* kinds whose 32-row tiles are never on two groups (plan_fwd_gemm) */   \
-  if (p.kg == 2) return hipErrorInvalidValue;                                               \
-  else if (p.bn == 128) gemm_bf3_kernel<BK, 1, 1, 1, true><<<grid, 256, 0, s>>>(a);        \
-  else gemm_bf3_kernel<BK, 1, 1, 2, true><<<grid, 256, 0, s>>>(a);
-    switch (bk) {
-    case BK_I4: WH_GP32(BK_I4) break;  // batches above 16 only, as the next four kinds
-    case BK_B16: WH_GP32N(BK_B16) break;
-    case BK_H16: WH_GP32N(BK_H16) break;
-    case BK_F32: case BK_U8:  // 128-column tiles only
-      if (p.bn != 128) return hipErrorInvalidValue;
-      if (bk == BK_F32) gemm_bf3_kernel<BK_F32, 1, 1, 1, true><<<grid, 256, 0, s>>>(a);
-      else gemm_bf3_kernel<BK_U8, 1, 1, 1, true><<<grid, 256, 0, s>>>(a);
-      break;
-    case BK_E4: WH_GP(BK_E4) break;
-    case BK_I8: WH_GP(BK_I8) break;
-    case BK_FP4: WH_GP(BK_FP4) break;
-    case BK_NF4: WH_GP(BK_NF4) break;
-    case BK_E5: WH_GP(BK_E5) break;
-    default: return hipErrorInvalidValue;
-    }
-#undef WH_GP
-#undef WH_GP32
-#undef WH_GP32N
-    return hipGetLastError();
-  }
-#define WH_GB(BK)                                                                     \
-  if (p.bm == 16) {                                                                   \
-    if (p.bn == 128) gemm_bf3s_kernel<BK, 1, 1><<<grid, 256, 0, s>>>(a);           \
-    else gemm_bf3s_kernel<BK, 1, 2><<<grid, 256, 0, s>>>(a);                       \
-  } else if (p.bm == 32) {                                                            \
-    if (p.bn == 128) gemm_bf3_kernel<BK, 1, 1, 1><<<grid, 256, 0, s>>>(a);         \
-    else gemm_bf3_kernel<BK, 1, 1, 2><<<grid, 256, 0, s>>>(a);                     \
-  } else {                                                                            \
-    if (p.bn == 128) gemm_bf3_kernel<BK, 2, 1, 1><<<grid, 256, 0, s>>>(a);         \
-    else gemm_bf3_kernel<BK, 2, 1, 2><<<grid, 256, 0, s>>>(a);                     \
-  }
+  bool done = false;
+#define WH_B3(KERNEL, THREADS, ...)                  \
+  do {                                               \
+    KERNEL<__VA_ARGS__><<<grid, THREADS, 0, s>>>(a); \
+    done = true;                                     \
+  } while (0)
   if (p.rows) return hipErrorInvalidValue;  // launched with its epilogue by the caller
-  if (p.kg == 2) {  // two wave groups, a ring two units deep
-#define WH_GK(BK)                                                                             \
-  if (p.bm == 32) gemm_bf3k_kernel<BK, 1, 2, 2><<<grid, 512, 0, s>>>(a);                  \
-  else gemm_bf3k_kernel<BK, 2, 2, 2><<<grid, 512, 0, s>>>(a);
-    switch (bk) {
-    case BK_B16: WH_GK(BK_B16) break;
-    case BK_H16: WH_GK(BK_H16) break;
-    case BK_I4: WH_GK(BK_I4) break;
-    case BK_E4: WH_GK(BK_E4) break;
-    case BK_I8: WH_GK(BK_I8) break;
-    case BK_FP4: WH_GK(BK_FP4) break;
-    case BK_NF4: WH_GK(BK_NF4) break;
-    case BK_E5: WH_GK(BK_E5) break;
-    default: return hipErrorInvalidValue;
+  if (p.bm == 16) {
+    if constexpr (small_batch) {
+      if (p.bn == 128 && p.sums) WH_B3(gemm_bf3s_kernel, 256, BK, 1, 1, true);
+      else if (p.bn == 128) WH_B3(gemm_bf3s_kernel, 256, BK, 1, 1);
+      else if (p.sums) WH_B3(gemm_bf3s_kernel, 256, BK, 1, 2, true);
+      else WH_B3(gemm_bf3s_kernel, 256, BK, 1, 2);
     }
-#undef WH_GK
-    return hipGetLastError();
+  } else if (p.bm == 32 && p.kg == 2) {  // two wave groups, a ring two units deep
+    if (p.sums) {
+      if constexpr (small_batch || BK == BK_I4) WH_B3(gemm_bf3k_kernel, 512, BK, 1, 2, 2, true);
+    } else {
+      if constexpr (four_bit) WH_B3(gemm_bf3k_kernel, 512, BK, 1, 2, 2);
+    }
+  } else if (p.bm == 32 && p.bn == 128) {
+    if (p.sums) {
+      WH_B3(gemm_bf3_kernel, 256, BK, 1, 1, 1, true);
+    } else {
+      if constexpr (!six && !tables && BK != BK_H16) WH_B3(gemm_bf3_kernel, 256, BK, 1, 1, 1);
+    }
+  } else if (p.bm == 32) {
+    if (p.sums) {
+      if constexpr (!six && BK != BK_B16) WH_B3(gemm_bf3_kernel, 256, BK, 1, 1, 2, true);
+    } else {
+      if constexpr (!six && BK != BK_H16) WH_B3(gemm_bf3_kernel, 256, BK, 1, 1, 2);
+    }
+  } else if (!p.sums) {
+    if constexpr (six) {
+      if (p.bn == 128) WH_B3(gemm_bf3_kernel, 256, BK, 2, 1, 1);
+    } else if (p.bn == 256) {
+      if (p.kg == 2) WH_B3(gemm_bf3k_kernel, 512, BK, 2, 2, 2);
+      else WH_B3(gemm_bf3_kernel, 256, BK, 2, 1, 2);
+    }
   }
-#define WH_GB32(BK)  /* batches above 16 only */                                      \
-  if (p.bm == 32) {                                                                   \
-    if (p.bn == 128) gemm_bf3_kernel<BK, 1, 1, 1><<<grid, 256, 0, s>>>(a);         \
-    else gemm_bf3_kernel<BK, 1, 1, 2><<<grid, 256, 0, s>>>(a);                     \
-  } else {                                                                            \
-    if (p.bn == 128) gemm_bf3_kernel<BK, 2, 1, 1><<<grid, 256, 0, s>>>(a);         \
-    else gemm_bf3_kernel<BK, 2, 1, 2><<<grid, 256, 0, s>>>(a);                     \
-  }
+#undef WH_B3
+  return done ? hipGetLastError() : hipErrorInvalidValue;
+}
+
+hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
   switch (bk) {
-  case BK_B16: WH_GB32(BK_B16) break;
-  case BK_H16: WH_GB32(BK_H16) break;
-  // 128-column tiles, of 32 rows with stage sums only (plan_fwd_gemm)
-  case BK_F32: case BK_U8:
-    if (p.bn != 128 || p.bm != 64) return hipErrorInvalidValue;
-    if (bk == BK_F32) gemm_bf3_kernel<BK_F32, 2, 1, 1><<<grid, 256, 0, s>>>(a);
-    else gemm_bf3_kernel<BK_U8, 2, 1, 1><<<grid, 256, 0, s>>>(a);
-    break;
-  case BK_I4: WH_GB32(BK_I4) break;
-  case BK_E4: WH_GB(BK_E4) break;
-  case BK_I8: WH_GB(BK_I8) break;
-  case BK_FP4: WH_GB(BK_FP4) break;
-  case BK_NF4: WH_GB(BK_NF4) break;
-  case BK_E5: WH_GB(BK_E5) break;
+  case BK_E4: return launch_bf3_kind<BK_E4>(p, a, s);
+  case BK_I8: return launch_bf3_kind<BK_I8>(p, a, s);
+  case BK_FP4: return launch_bf3_kind<BK_FP4>(p, a, s);
+  case BK_NF4: return launch_bf3_kind<BK_NF4>(p, a, s);
+  case BK_E5: return launch_bf3_kind<BK_E5>(p, a, s);
+  case BK_B16: return launch_bf3_kind<BK_B16>(p, a, s);
+  case BK_H16: return launch_bf3_kind<BK_H16>(p, a, s);
+  case BK_F32: return launch_bf3_kind<BK_F32>(p, a, s);
+  case BK_I4: return launch_bf3_kind<BK_I4>(p, a, s);
+  case BK_U8: return launch_bf3_kind<BK_U8>(p, a, s);
   default: return hipErrorInvalidValue;
   }
-#undef WH_GB
-#undef WH_GB32
-  return hipGetLastError();
 }
 
 // gemv_loopb_kernel launch: R = 16 / (B * C) rows per group (16 sums per

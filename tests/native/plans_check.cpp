@@ -5,6 +5,7 @@
 //
 //   plans_check KERNELS    KERNELS: gemm_bf3 / bf3s / bf3k instantiations in the
 //                          object; prints "plans_check: ok" and the counts
+//   plans_check plan KIND M N K PAIR    the tile of one plan
 #include <cstdio>
 #include <cstdlib>
 #include <set>
@@ -31,6 +32,13 @@ hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) {
 
 int main(int argc, char **argv) {
   using namespace wh;
+  if (argc == 7) {
+    const int bk = std::atoi(argv[2]), M = std::atoi(argv[3]), N = std::atoi(argv[4]), K = std::atoi(argv[5]);
+    SkPlan p = plan_fwd_gemm(0, bk, M, K, N, std::atoi(argv[6]) ? 2 : 1);
+    if (p.bm == 64) p = plan_fwd_gemm(0, bk, M, K, N);  // pair_gemm_plan
+    std::printf("%dx%d%s%s\n", p.bm, p.bn, p.kg == 2 ? "x2" : "", p.sums ? "+" : "");
+    return 0;
+  }
   const int Ms[] = {5, 8, 13, 16, 17, 20, 32, 33, 48, 64, 65, 100, 128, 130, 256, 600, 2100};
   const int Ns[] = {1, 100, 300, 512, 777, 1024, 1368, 3000, 4096, 8192, 8200, 11008, 20000};
   const int Ks[] = {16, 64, 80, 128, 512, 1008, 1024, 2048, 2064, 2112, 3136, 4096, 8192, 11008, 11072};

@@ -97,12 +97,12 @@ def test_forward_kernel_variants(oracle, knobs):
 
 @pytest.mark.parametrize("dtype", [4, 5, 9, 16, 26])
 def test_split_x_two_group_workgroups(oracle, dtype):
-    """The split-x GEMM on 8-wave workgroups whose two wave groups take
+    """The split-x GEMM on 32-row tiles at batch 20-64 (two wave groups for the
+    4-bit kinds' batch 20), ragged batch included, K whose last stage runs past
+    it, shares crossing tile boundaries, and the dX of a forward through the
+    transposed codes (K = rows).  Two groups on larger tiles, which take
     alternate k stages and add their sums through LDS at each tile's end:
-    64-row tiles (batch 33-64, ragged batch included) and the 32-row tiles of
-    the 4-bit kinds, K whose last stage runs past it, shares crossing tile
-    boundaries, and the dX of a forward through the transposed codes (K =
-    rows)."""
+    test_gpu_split_tiles.py."""
     rng = np.random.default_rng(1500 + dtype)
     cases = ((300, 2016, 64), (257, 1024, 48), (128, 4096, 33), (1000, 512, 64), (300, 2016, 20))
     for out, inn, batch in cases:

@@ -55,3 +55,33 @@ def test_calls_from_several_threads():
     for t in team:
         t.join()
     assert not bad, bad[:4]
+
+
+def test_large_calls_from_several_threads():
+    """Three calls at once whose weights (38 MB) go up and whose gradient and
+    new weights come down in pieces on several threads each."""
+    rng = np.random.default_rng(6)
+    jobs = [(rng.normal(0, 0.1, (2304, 4096)).astype(np.float32), rng.normal(0, 1, (2, 4096)).astype(np.float32))
+            for _ in range(3)]
+
+    def call(k):
+        W, x = jobs[k]
+        r = pywelvet.normalbp(W, x, np.zeros((2, 2304), np.float32), 1, 0.1, act=-1, dtype=1)
+        return {n: np.array(v) for n, v in r.items()}
+
+    want = [call(k) for k in range(3)]
+    for k, (W, _) in enumerate(jobs):  # the Float32 step of the gradient that came down with it, within a rounding each
+        assert np.allclose(want[k]["W_after"], W - 0.1 * want[k]["dW"], rtol=3e-7, atol=1e-7)
+    bad = []
+
+    def work(k):
+        for _ in range(3):
+            got = call(k)
+            bad.extend((k, n) for n in got if not np.array_equal(got[n], want[k][n]))
+
+    team = [threading.Thread(target=work, args=(k,)) for k in range(3)]
+    for t in team:
+        t.start()
+    for t in team:
+        t.join()
+    assert not bad, bad[:4]

@@ -1,7 +1,7 @@
 """The split-x bf16 GEMM's kinds for batches above 16 (BFloat16, Float16,
-Float32, Int4, Uint8) against the oracle: edges of the row tiles (16, 32, 64),
-the k stage (64) and the column tiles, weights of one sign, and non-finite
-operands.  The products of BFloat16, Int4 and Float16's and Float32's higher
+Float32, Int4, Uint8) against the oracle: edges of the batch and of the k stage
+(64), weights of one sign, non-finite operands, and both ends of the float
+range (the tiles' edges: test_gpu_split_tiles.py).  The products of BFloat16, Int4 and Float16's and Float32's higher
 parts are exact; the dropped ones of the lower parts are at most 3.9 2^-23 of
 a product (Float16 1.7), and the sums are fp32, so an output is within 1e-5 of
 the sum of magnitudes, as for the other kinds."""
@@ -41,7 +41,9 @@ def test_split_kinds(oracle, dtype):
 
 @pytest.mark.parametrize("lo,hi", [(0.5, 0.75), (-0.75, -0.5), (-0.05, 3.0), (0.25, 0.25)])
 def test_uint8_offsets(oracle, lo, hi):
-    """Uint8 ranges without 0, with an outlier on one side, and of no width."""
+    """Uint8 ranges without 0, with an outlier on one side, and of no width (96
+    outputs: the fp32 MFMA; test_gpu_sum_error.py has such ranges on the
+    split-x GEMM)."""
     rng = np.random.default_rng(3)
     W = rng.normal(0, 0.01, (96, 256)).astype(np.float32) + np.float32((lo + hi) / 2 if lo * hi > 0 else 0)
     W = np.clip(W, lo, hi)
@@ -55,12 +57,14 @@ def test_uint8_offsets(oracle, lo, hi):
 
 @pytest.mark.parametrize("dtype", [3, 2, 1, 13])
 @pytest.mark.parametrize("batch", [20, 70])
-def test_split_kinds_nonfinite(oracle, dtype, batch):
+@pytest.mark.parametrize("out", [40, 520])
+def test_split_kinds_nonfinite(oracle, dtype, batch, out):
     """Infinities and NaN in x (all kinds) and W (the float ones): the class
     of every output is that of the whole operands' product.  K = 80 ends
-    inside a k stage, which then holds the next row's first weights."""
+    inside a k stage, which then holds the next row's first weights.  520
+    outputs: Float32 and Uint8, on the fp32 MFMA at 40, are split there too."""
     rng = np.random.default_rng(batch + dtype)
-    W = rng.choice(np.float32([-1.0, -0.5, 0.5, 1.0, 0.0]), (40, 80)).astype(np.float32)
+    W = rng.choice(np.float32([-1.0, -0.5, 0.5, 1.0, 0.0]), (out, 80)).astype(np.float32)
     W[0, 0], W[0, 1] = 1.0, -1.0
     x = rng.choice(np.float32([-2.0, -1.0, 1.0, 0.0, 0.37]), (batch, 80)).astype(np.float32)
     x[3, 5], x[4, 6], x[5, 7], x[6, 1], x[6, 2] = np.inf, -np.inf, np.nan, np.inf, -np.inf
@@ -69,7 +73,7 @@ def test_split_kinds_nonfinite(oracle, dtype, batch):
     pre, _ = pywelvet.forward(W, x, dtype=dtype)
     Wd = oracle_weights(oracle, dtype, W)
     with np.errstate(invalid="ignore"):
-        ref = np.array([[np.sum(x[m].astype(np.float64) * Wd[n]) for n in range(40)] for m in range(batch)])
+        ref = np.array([[np.sum(x[m].astype(np.float64) * Wd[n]) for n in range(out)] for m in range(batch)])
     assert np.array_equal(np.isnan(pre), np.isnan(ref))
     assert np.array_equal(pre[np.isinf(ref)], ref[np.isinf(ref)].astype(np.float32))
     ok = np.isfinite(ref)

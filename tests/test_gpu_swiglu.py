@@ -216,9 +216,9 @@ def test_resident_session_matches_one_shot():
 @pytest.mark.parametrize("dtype", [4, 5, 9, 14, 16, 26], ids=[pywelvet.DTYPE_NAMES[d] for d in (4, 5, 9, 14, 16, 26)])
 @pytest.mark.parametrize("rows,inn,inter", [(5, 4096, 300), (16, 2112, 257), (17, 96, 1000), (40, 640, 384), (70, 512, 1030)])
 def test_gate_and_up_in_one_launch(oracle, dtype, rows, inn, inter):
-    """Gate and Up as one split-x GEMM launch with one reduction (16-, 32- and
-    64-row tiles, ragged outputs): h and post against the f64 products of the
-    decoded weights.  g and u carry a product's 1e-5; h = silu(g) u at most
+    """Gate and Up as one split-x GEMM launch with one reduction (16- and 32-row
+    tiles, ragged outputs; 64-row ones: test_gpu_split_tiles.py): h and post
+    against the f64 products of the decoded weights.  g and u carry a product's 1e-5; h = silu(g) u at most
     their sum (|silu'| <= 1.1), post one product more."""
     rng = np.random.default_rng(rows + inn + dtype)
     scale = 2.0 if dtype == 16 else 0.5 / np.sqrt(inn)

@@ -17,7 +17,8 @@ def _run(cmd, **kw):
     return r
 
 
-def test_every_plan_has_its_kernel_and_every_kernel_a_plan():
+def _built():
+    """The check and its object."""
     src = os.path.join(ROOT, "tests", "native", "plans_check.cpp")
     exe = os.path.join(OUT, "plans_check")
     obj = exe + ".o"
@@ -27,7 +28,27 @@ def test_every_plan_has_its_kernel_and_every_kernel_a_plan():
         _run([HIPCC, "-x", "hip", "--offload-host-only", "-fgpu-rdc", "-std=c++17", "-O1", "-ffp-contract=off",
               "-I", CSRC, "-c", src, "-o", obj])
         _run([HIPCC, "-fgpu-rdc", "--offload-arch=gfx950", obj, "-o", exe])
+    return exe, obj
+
+
+def test_every_plan_has_its_kernel_and_every_kernel_a_plan():
+    exe, obj = _built()
     symbols = _run(["nm", obj]).stdout
     kernels = set(re.findall(r"__device_stub__gemm_bf3[sk]?_kernel\w*", symbols))
     r = subprocess.run([exe, str(len(kernels))], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and "plans_check: ok" in r.stdout, r.stdout[-2000:]
+
+
+def test_plans_of_the_edge_shapes():
+    """The shapes whose results test_gpu_split_tiles.py checks run the kernels
+    that the table says."""
+    import split_shapes as S
+    exe = _built()[0]
+    wrong = []
+    for out, inn, batch, single, pair in S.SHAPES:
+        for p, plans in ((0, single), (1, pair)):
+            for kind, want in plans.items():
+                got = _run([exe, "plan", str(kind), str(batch), str(out), str(inn), str(p)]).stdout.strip()
+                if got != want:
+                    wrong.append((out, inn, batch, p, kind, got, want))
+    assert not wrong, wrong

@@ -55,10 +55,9 @@ int main(int argc, char **argv) {
             if (pair && p.bm == 64) p = plan_fwd_gemm(0, bk, M, K, N);
             if (p.rows) continue;
             GemmArgs a{};
-            if (pair) a.body2 = (const uint8_t *)&a;
             ++plans;
             const int64_t units = (int64_t)p.gx * p.gy * p.nst;
-            if (launch_bf3(p, bk, a, nullptr) != hipSuccess || (int64_t)p.blocks * p.per_block < units ||
+            if (launch_bf3(p, bk, a, nullptr, pair != 0) != hipSuccess || (int64_t)p.blocks * p.per_block < units ||
                 (int64_t)(p.blocks - 1) * p.per_block >= units) {
               std::printf("plans_check: kind %d M %d N %d K %d pair %d\n", bk, M, N, K, pair);
               return 1;

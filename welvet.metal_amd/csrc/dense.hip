@@ -782,11 +782,9 @@ struct GemmArgs {
   // GEMM factors out of the weights; double: a sixteenth of a small scale is
   // no f32)
   double post = 1.0;
-  // a second store's product with the same x in the same launch (grid y = 1):
-  // its body, and its partial tiles this many floats into ws
-  const uint8_t *body2 = nullptr;
-  int64_t ws2 = 0;
 };
+// gemm_regt_kernel's other arguments are 20 bytes; past 128 a launch is slower (see take_pair)
+static_assert(sizeof(GemmArgs) + 20 <= 128, "GEMM arguments within 128 bytes");
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
@@ -1636,11 +1634,19 @@ __device__ inline void add_row(V (&to)[N], const V (&v)[N]) {
   for (int c = 0; c < N; ++c) to[c] += v[c];
 }
 
-// Blocks of grid row 1 work on the second store.
+// A pair launch multiplies two stores of one shape by the same x: grid row 1
+// works on the second one, whose body is in `lut` (which the split-x kinds do
+// not read) and whose partial tiles follow those of the first one's `bm`
+// blocks (a tile's size is a constant of these kernels).  No fields of their
+// own: with them the arguments of the other GEMMs pass 128 bytes, and each
+// launch takes 0.2 us more to start (FP8 1024^2 b16 dX 6.3 -> 6.5 us, 4096^2
+// b17 15.0 -> 15.3, Int8 1008 -> 3000 b17 11.2 -> 11.7).
+__device__ inline const uint8_t *pair_body(const GemmArgs &a) { return (const uint8_t *)a.lut; }
+template <int TILE>
 __device__ inline void take_pair(GemmArgs &a) {
   if (blockIdx.y != 0) {
-    a.body = a.body2;
-    a.ws += a.ws2;
+    a.body = pair_body(a);
+    a.ws += (int64_t)a.bm * a.maxspan * TILE;
   }
 }
 
@@ -1652,9 +1658,9 @@ __device__ inline void take_pair(GemmArgs &a) {
 // to 24.
 template <int BK, int MT, int D, int NC, bool SUMS = false>
 __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
-  take_pair(a);
   using K3 = B3<BK>;
   constexpr int BM = 32 * MT, BN = 128 * NC, NW = K3::kWords, NP = K3::kParts;
+  take_pair<BM * BN>(a);
   constexpr int XE = BM * kBK / 256;  // x values per thread per stage (8 or 16)
   constexpr int XT = kBK / XE;        // threads per x row
   __shared__ uint16_t Xs[2][3][BM][kBf3Row];
@@ -1868,9 +1874,9 @@ __global__ void __launch_bounds__(256) gemm_bf3_kernel(GemmArgs a) {
 // writes half the partial tiles.  GemmArgs::nst counts stage pairs here.
 template <int BK, int MT, int D, int NC, bool SUMS = false>
 __global__ void __launch_bounds__(512) gemm_bf3k_kernel(GemmArgs a) {
-  take_pair(a);
   using K3 = B3<BK>;
   constexpr int BM = 32 * MT, BN = 128 * NC, NW = K3::kWords, NP = K3::kParts;
+  take_pair<BM * BN>(a);
   constexpr int XE = BM * kBK / 256;  // x values per thread per stage (8 or 16)
   constexpr int XT = kBK / XE;        // threads per x row
   constexpr int P = MT * NC;          // 32 x 32 accumulator pieces per wave
@@ -2111,9 +2117,9 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // 4 g .. 4 g + 3.
 template <int BK, int D, int NC, bool SUMS = false>
 __global__ void __launch_bounds__(256) gemm_bf3s_kernel(GemmArgs a) {
-  take_pair(a);
   using K3 = B3<BK>;
   constexpr int BM = 16, BN = 128 * NC, NW = K3::kWords / 2, NP = K3::kParts;
+  take_pair<BM * BN>(a);
   constexpr int CG = 2 * NC;          // 16-column groups per wave
   constexpr int XE = BM * kBK / 256;  // 4 x values per thread per stage
   constexpr int XT = kBK / XE;        // 16 threads per x row
@@ -2595,8 +2601,8 @@ __global__ void __launch_bounds__(256) sk_reduce_kernel(GemmArgs a, const double
 // as sk_reduce_kernel sums one), h = fl32(silu(g)) * u, op_swiglu's product.
 // FIX: Int4, as there (scale2: the second store's).
 template <bool FIX>
-__global__ void __launch_bounds__(256) sk_reduce_pair_kernel(GemmArgs a, double post2, float scale2, float *g_pre,
-                                                             float *u_pre, float *h) {
+__global__ void __launch_bounds__(256) sk_reduce_pair_kernel(GemmArgs a, int64_t ws2, double post2, float scale2,
+                                                             float *g_pre, float *u_pre, float *h) {
   const int t = blockIdx.x;
   const int b0 = (int)((int64_t)t * a.nst / a.per_block);
   const int b1 = (int)(((int64_t)(t + 1) * a.nst - 1) / a.per_block);
@@ -2618,7 +2624,7 @@ __global__ void __launch_bounds__(256) sk_reduce_pair_kernel(GemmArgs a, double 
         const int slot = t - (int)((int64_t)b * a.per_block / a.nst);
         const float *src = a.ws + ((int64_t)b * a.maxspan + slot) * tile + off;
         v[0][i] = *(const float4 *)src;
-        v[1][i] = *(const float4 *)(src + a.ws2);
+        v[1][i] = *(const float4 *)(src + ws2);
       }
     }
 #pragma unroll
@@ -2641,7 +2647,7 @@ __global__ void __launch_bounds__(256) sk_reduce_pair_kernel(GemmArgs a, double 
   if constexpr (FIX) {
     split_nan_fix(a, BK_I4, m, n, live, sum[0]);
     GemmArgs b = a;
-    b.body = a.body2;
+    b.body = pair_body(a);
     b.scale = scale2;
     split_nan_fix(b, BK_I4, m, n, live, sum[1]);
     if (!live) return;
@@ -3411,12 +3417,13 @@ hipError_t launch_bf3r(const SkPlan &p, int bk, const GemmArgs &a, const double 
 // The split-x GEMM of plan p for weight kind BK (a.body, a.post set).  Only the
 // kernels that plan_fwd_gemm can ask for exist; any other plan is an error.
 template <int BK>
-hipError_t launch_bf3_kind(const SkPlan &p, GemmArgs &a, hipStream_t s) {
+hipError_t launch_bf3_kind(const SkPlan &p, GemmArgs a, bool pair, hipStream_t s) {
   constexpr bool small_batch = BK < BK_B16;                 // also batches of 5 to 16
   constexpr bool six = BK == BK_F32 || BK == BK_U8;         // 128-column tiles
   constexpr bool tables = BK == BK_FP4 || BK == BK_NF4;
   constexpr bool four_bit = tables || BK == BK_I4;          // two groups up to batch 32 too
-  const dim3 grid(p.blocks, a.body2 != nullptr ? 2 : 1);
+  const dim3 grid(p.blocks, pair ? 2 : 1);
+  if (pair) a.bm = p.blocks;  // take_pair
   bool done = false;
 #define WH_B3(KERNEL, THREADS, ...)                  \
   do {                                               \
@@ -3461,18 +3468,18 @@ hipError_t launch_bf3_kind(const SkPlan &p, GemmArgs &a, hipStream_t s) {
   return done ? hipGetLastError() : hipErrorInvalidValue;
 }
 
-hipError_t launch_bf3(const SkPlan &p, int bk, GemmArgs &a, hipStream_t s) {
+hipError_t launch_bf3(const SkPlan &p, int bk, const GemmArgs &a, hipStream_t s, bool pair = false) {
   switch (bk) {
-  case BK_E4: return launch_bf3_kind<BK_E4>(p, a, s);
-  case BK_I8: return launch_bf3_kind<BK_I8>(p, a, s);
-  case BK_FP4: return launch_bf3_kind<BK_FP4>(p, a, s);
-  case BK_NF4: return launch_bf3_kind<BK_NF4>(p, a, s);
-  case BK_E5: return launch_bf3_kind<BK_E5>(p, a, s);
-  case BK_B16: return launch_bf3_kind<BK_B16>(p, a, s);
-  case BK_H16: return launch_bf3_kind<BK_H16>(p, a, s);
-  case BK_F32: return launch_bf3_kind<BK_F32>(p, a, s);
-  case BK_I4: return launch_bf3_kind<BK_I4>(p, a, s);
-  case BK_U8: return launch_bf3_kind<BK_U8>(p, a, s);
+  case BK_E4: return launch_bf3_kind<BK_E4>(p, a, pair, s);
+  case BK_I8: return launch_bf3_kind<BK_I8>(p, a, pair, s);
+  case BK_FP4: return launch_bf3_kind<BK_FP4>(p, a, pair, s);
+  case BK_NF4: return launch_bf3_kind<BK_NF4>(p, a, pair, s);
+  case BK_E5: return launch_bf3_kind<BK_E5>(p, a, pair, s);
+  case BK_B16: return launch_bf3_kind<BK_B16>(p, a, pair, s);
+  case BK_H16: return launch_bf3_kind<BK_H16>(p, a, pair, s);
+  case BK_F32: return launch_bf3_kind<BK_F32>(p, a, pair, s);
+  case BK_I4: return launch_bf3_kind<BK_I4>(p, a, pair, s);
+  case BK_U8: return launch_bf3_kind<BK_U8>(p, a, pair, s);
   default: return hipErrorInvalidValue;
   }
 }
@@ -3782,18 +3789,18 @@ hipError_t launch_forward_pair_gemm(const DevStore &g, const DevStore &u, int ba
   SkPlan p;
   if (!pair_gemm_plan(g, u, batch, bk, p) || ws_bytes < 2 * p.ws_bytes) return hipErrorInvalidValue;
   const bool ready = bk == BK_E4 || bk == BK_E5;
-  GemmArgs a{ready ? g.kbody : g.body, g.lut, g.scale, g.minv, x, batch, g.cols, g.rows, row_bytes_of(g),
+  const uint8_t *body = ready ? g.kbody : g.body, *body2 = ready ? u.kbody : u.body;
+  if (body == nullptr || body2 == nullptr) return hipErrorInvalidValue;
+  GemmArgs a{body, (const float *)body2, g.scale, g.minv, x, batch, g.cols, g.rows, row_bytes_of(g),
              p.gx, p.gy, p.nst, p.per_block, p.maxspan, (float *)ws, p.bm, p.bn};
   a.post = bf3_post(g, bk);
-  a.body2 = ready ? u.kbody : u.body;
-  a.ws2 = (int64_t)(p.ws_bytes / sizeof(float));
-  if (a.body == nullptr || a.body2 == nullptr) return hipErrorInvalidValue;
-  const hipError_t e = launch_bf3(p, bk, a, s);
+  const int64_t ws2 = (int64_t)(p.ws_bytes / sizeof(float));
+  const hipError_t e = launch_bf3(p, bk, a, s, true);
   if (e != hipSuccess) return e;
   if (bk == BK_I4)
-    sk_reduce_pair_kernel<true><<<sk_reduce_grid(p), 256, 0, s>>>(a, bf3_post(u, bk), u.scale, g_pre, u_pre, h);
+    sk_reduce_pair_kernel<true><<<sk_reduce_grid(p), 256, 0, s>>>(a, ws2, bf3_post(u, bk), u.scale, g_pre, u_pre, h);
   else
-    sk_reduce_pair_kernel<false><<<sk_reduce_grid(p), 256, 0, s>>>(a, bf3_post(u, bk), u.scale, g_pre, u_pre, h);
+    sk_reduce_pair_kernel<false><<<sk_reduce_grid(p), 256, 0, s>>>(a, ws2, bf3_post(u, bk), u.scale, g_pre, u_pre, h);
   return hipGetLastError();
 }
 

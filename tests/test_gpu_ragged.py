@@ -94,3 +94,37 @@ def test_ragged_nonfinite_weights_stay_in_their_columns(oracle):
         assert np.isfinite(pre[:, good]).all() and not np.isfinite(pre[:, [3, 9, 12]]).any()
         good = [i for i in range(37) if i not in (0, 5, 36)]
         assert np.isfinite(dX[:, good]).all() and not np.isfinite(dX[:, [0, 5, 36]]).any()
+
+
+@pytest.mark.parametrize("dtype", range(34), ids=DTYPE_NAMES)
+@pytest.mark.parametrize("batch", [5, 6, 7, 8])
+def test_ragged_long_rows_small_batch(oracle, dtype, batch):
+    """Batch 5 to 8 of long rows as row products in two halves (an odd batch's
+    halves share a row); 515 columns for Complex64, which takes them there."""
+    for out, inn in ((5, 3075), (9, 515)):
+        if inn % chunk(dtype):
+            check(oracle, dtype, out, inn, batch)
+
+
+def test_ragged_batch_5_costs_little_more_than_batch_4():
+    """One MFMA chain per 16 x 16 outputs took three times batch 4's row
+    products at 4095 -> 100; two halves of them take 1.2 times."""
+    import time
+
+    from devmem import DeviceArray, hip
+    W = np.random.default_rng(1).normal(0, 1, (100, 4095)).astype(np.float32)
+    best = {}
+    for batch in (4, 5):
+        d_x, d_pre, d_post = (DeviceArray((batch, n), 0.5) for n in (4095, 100, 100))
+        with pywelvet.Session(W, batch=batch, act=-1, dtype=1) as s:
+            t = []
+            for _ in range(8):
+                hip().hipDeviceSynchronize()
+                t0 = time.perf_counter()
+                for _ in range(100):
+                    s.forward_device(d_x.ptr, d_pre.ptr, d_post.ptr)
+                hip().hipDeviceSynchronize()
+                t.append((time.perf_counter() - t0) / 100)
+        best[batch] = min(t)
+    print({b: "%.1f us" % (t * 1e6) for b, t in best.items()}, flush=True)
+    assert best[5] < 2 * best[4]

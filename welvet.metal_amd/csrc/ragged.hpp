@@ -88,15 +88,17 @@ __device__ inline void load_row(const float *__restrict__ row, int k, int K, boo
   }
 }
 
-// Row products, B = M rows of x: a block holds 4 / S output rows, S waves share one, its
-// pieces of P codes dealt to their lanes in turn.  One row: up to four codes
-// per lane (a whole chunk leaves most lanes of a short row idle).  More rows,
-// of which most start off a 16-byte boundary: one code per lane, so each
-// row's loads are whole cache lines (four dwords per lane of a 16-byte-strided
-// row take 39 cycles each: 4095^2 b2 32 us).
+// Row products, B rows of x (grid row 1: the last B of M): a block holds 4 / S
+// output rows, S waves share one, its pieces of P codes dealt to their lanes in
+// turn.  One row: up to four codes per lane (a whole chunk leaves most lanes of
+// a short row idle), but one of Complex64, whose imaginary halves are not
+// loaded: two strided dwords per lane take longer than one (4095 -> 1000 b1 9.0
+// us, with one 6.9).  More rows, of which most start off a 16-byte boundary: one code
+// per lane, so each row's loads are whole cache lines (four dwords per lane of
+// a 16-byte-strided row take 39 cycles each: 4095^2 b2 32 us).
 template <int F, int B>
 constexpr int ragged_piece() {
-  return B > 1 ? 1 : FI<F>::kE < 4 ? FI<F>::kE : 4;
+  return B > 1 || F == FC64 ? 1 : FI<F>::kE < 4 ? FI<F>::kE : 4;
 }
 template <int F, int B>
 __global__ void __launch_bounds__(256) ragged_gemv_kernel(RaggedArgs a, int S, const double *bias, int bias_len,
@@ -117,8 +119,9 @@ __global__ void __launch_bounds__(256) ragged_gemv_kernel(RaggedArgs a, int S, c
   double acc[B];
 #pragma unroll
   for (int b = 0; b < B; ++b) acc[b] = 0.0;
-  const int npieces = (a.K + P - 1) / P;
+  const int npieces = (a.K + P - 1) / P, m0 = blockIdx.y == 0 ? 0 : a.M - B;
   const int64_t base = (int64_t)row * a.cols;
+  const float *x = a.A + (int64_t)m0 * a.K;
   for (int c = part * 64 + lane; c < npieces; c += 64 * S) {
     const int k = c * P;
     uint32_t w[W];
@@ -129,10 +132,10 @@ __global__ void __launch_bounds__(256) ragged_gemv_kernel(RaggedArgs a, int S, c
     for (int b = 0; b < B; ++b) {
       const int64_t off = (int64_t)b * a.K;
       if (B == 1 && whole) {
-        load_x<P>(a.A + k, xv[b]);
+        load_x<P>(x + k, xv[b]);
       } else {
 #pragma unroll
-        for (int e = 0; e < P; ++e) xv[b][e] = a.A[off + min(k + e, a.K - 1)];
+        for (int e = 0; e < P; ++e) xv[b][e] = x[off + min(k + e, a.K - 1)];
       }
     }
 #pragma unroll
@@ -153,7 +156,7 @@ __global__ void __launch_bounds__(256) ragged_gemv_kernel(RaggedArgs a, int S, c
     const int r = tid / B, b = tid % B, o = blockIdx.x * (4 / S) + r;
     double t = 0.0;
     for (int i = 0; i < S; ++i) t += red[r * S + i][b];
-    if (o < a.N) bias_act_store(t, o, bias, bias_len, act, pre, post, (int64_t)b * a.N + o);
+    if (o < a.N) bias_act_store(t, o, bias, bias_len, act, pre, post, (int64_t)(m0 + b) * a.N + o);
   }
 }
 
@@ -349,15 +352,21 @@ template <int F>
 hipError_t ragged_forward(RaggedArgs a, const double *bias, int bias_len, int act, float *pre, float *post,
                           hipStream_t s) {
   // up to 4 rows as row products; from 8 M weights on the MFMA reads them at
-  // least as fast (4095^2 Int8 b2 / b4 17.3 / 17.5 us against 18.1 / 22.7)
-  if (a.M == 1 || (a.M <= 4 && (int64_t)a.K * a.N <= ((int64_t)8 << 20))) {
+  // least as fast (4095^2 Int8 b2 / b4 17.3 / 17.5 us against 18.1 / 22.7).  5
+  // to 8 rows as two halves where K is long: the MFMA's one chain per 16 x 16
+  // outputs is then the time (Float32 4095 -> 100 b5 17.3 us against 5.1, 4095
+  // -> 1000 b8 18.4 / 11.5; 2047^2 b8 stays on it, 11.2 us), from 512 on for
+  // Complex64, whose loads there are strided (1001 -> 777 b5 9.7 / 6.1).
+  const bool few = (int64_t)a.K * a.N <= ((int64_t)8 << 20);
+  if (a.M == 1 || (a.M <= 4 && few) || (a.M <= 8 && few && a.K >= (F == FC64 ? 512 : 3072))) {
     const int P = a.M == 1 ? ragged_piece<F, 1>() : 1;
     const int npieces = (a.K + P - 1) / P;
     const int S = npieces > 128 ? 4 : npieces > 64 ? 2 : 1;
-    const int blocks = (a.N + 4 / S - 1) / (4 / S);
-    if (a.M == 1) ragged_gemv_kernel<F, 1><<<blocks, 256, 0, s>>>(a, S, bias, bias_len, act, pre, post);
-    else if (a.M == 2) ragged_gemv_kernel<F, 2><<<blocks, 256, 0, s>>>(a, S, bias, bias_len, act, pre, post);
-    else if (a.M == 3) ragged_gemv_kernel<F, 3><<<blocks, 256, 0, s>>>(a, S, bias, bias_len, act, pre, post);
+    const dim3 blocks((a.N + 4 / S - 1) / (4 / S), a.M <= 4 ? 1 : 2);
+    const int B = a.M <= 4 ? a.M : (a.M + 1) / 2;
+    if (B == 1) ragged_gemv_kernel<F, 1><<<blocks, 256, 0, s>>>(a, S, bias, bias_len, act, pre, post);
+    else if (B == 2) ragged_gemv_kernel<F, 2><<<blocks, 256, 0, s>>>(a, S, bias, bias_len, act, pre, post);
+    else if (B == 3) ragged_gemv_kernel<F, 3><<<blocks, 256, 0, s>>>(a, S, bias, bias_len, act, pre, post);
     else ragged_gemv_kernel<F, 4><<<blocks, 256, 0, s>>>(a, S, bias, bias_len, act, pre, post);
     return hipGetLastError();
   }

@@ -128,3 +128,12 @@ def test_ragged_batch_5_costs_little_more_than_batch_4():
         best[batch] = min(t)
     print({b: "%.1f us" % (t * 1e6) for b, t in best.items()}, flush=True)
     assert best[5] < 2 * best[4]
+
+
+@pytest.mark.parametrize("dtype", [1, 0, 14, 27])
+@pytest.mark.parametrize("out,inn,batch", [(16, 4095, 16), (16, 4097, 16), (17, 33, 31), (17, 41, 25), (777, 11, 8)])
+def test_ragged_dx_few(oracle, dtype, out, inn, batch):
+    """dX of few rows or few outputs, on both sides of where its kernels change
+    (16 rows and 65536 outputs, 1024 outputs)."""
+    if inn % chunk(dtype):
+        check(oracle, dtype, out, inn, batch)

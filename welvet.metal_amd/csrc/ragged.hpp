@@ -385,8 +385,51 @@ hipError_t ragged_forward(RaggedArgs a, const double *bias, int bias_len, int ac
   return hipGetLastError();
 }
 
+// dX of few terms or few outputs, bound by the launch and one load chain: L
+// lanes (1 or 64) per output walk the rows of W, one code each.
+template <int F, int L>
+__global__ void __launch_bounds__(256) ragged_dx_few_kernel(RaggedArgs a, float *out, const float *next_pre,
+                                                            int next_act) {
+  using I = FI<F>;
+  __shared__ __align__(16) float lut_s[I::kTable];
+  const int tid = threadIdx.x;
+  if constexpr (I::kLut) {
+    TabCopy<F> tab;
+    tab.load(a.lut, tid);
+    tab.store(lut_s, tid);
+    __syncthreads();
+  }
+  const int total = a.M * a.N, q = blockIdx.x * (256 / L) + tid / L, qc = min(q, total - 1);
+  const int m = qc / a.N, i = qc % a.N;
+  double s = 0.0;
+#pragma unroll 4
+  for (int o = tid % L; o < a.K; o += L) {
+    uint32_t w[I::kW];
+    load_chunk_at<F, 1>(a.body, (int64_t)o * a.cols + i, w);
+    s = fma((double)chunk_value<F>(w, 0, lut_s, a.scale, a.minv), (double)a.A[(int64_t)m * a.K + o], s);
+  }
+  if constexpr (L > 1) s = wave_sum(s);
+  if (q < total && tid % L == 0) {
+    float v = (float)s;
+    if (next_pre != nullptr) v = v * act_prime_piecewise(next_pre[q], next_act);
+    out[q] = v;
+  }
+}
+
 template <int F>
 hipError_t ragged_dx(RaggedArgs a, float *dX, const float *next_pre, int next_act, hipStream_t s) {
+  // up to 16 terms (a quarter of a stage) or 1024 outputs: the MFMA kernel's
+  // staging and exchange are most of its time (Float32 10 rows of 777 b8 4.0
+  // us, 3.2 here; 777 rows of 10 b8 5.4 / 4.5)
+  const int64_t total = (int64_t)a.M * a.N;
+  if (a.K <= 16 && total <= 65536) {
+    ragged_dx_few_kernel<F, 1><<<(int)((total + 255) / 256), 256, 0, s>>>(a, dX, next_pre, next_act);
+    return hipGetLastError();
+  }
+  if (total <= 1024) {
+    ragged_dx_few_kernel<F, 64><<<(int)((total + 3) / 4), 256, 0, s>>>(a, dX, next_pre, next_act);
+    return hipGetLastError();
+  }
   a.nst = (a.K + RaggedTShape<F>::ST - 1) / RaggedTShape<F>::ST;
   a.gx = (a.N + 15) / 16;
   const int gy32 = (a.M + 31) / 32;

@@ -329,8 +329,9 @@ WELVET_API void welvet_hip_set_forward_path(int32_t path);
  * are unknown):
  *   10 split-x bf16 MFMA GEMM (x split exactly into three bf16 parts) for
  *      FP8 E4M3 / E5M2, Int8, FP4 and NF4 weights at batch > 4 and for
- *      BFloat16, Float16, Float32, Int4 and Uint8 weights at batch > 16
- *      (rows of a multiple of 16), 0 = the fp32 MFMA GEMMs [1]
+ *      BFloat16, Float16 and Int4 weights, and Float32 and Uint8 ones of at
+ *      least 512 outputs, at batch > 16 (rows of a multiple of 16), 0 = the
+ *      fp32 MFMA GEMMs [1]
  *   16 batch <= 16 forward and dX without a k split across workgroups
  *      (epilogue in the kernel, no reduction launch; the split-x GEMM for
  *      its formats, the fp32 MFMA for the others): 0 off, 1 for a

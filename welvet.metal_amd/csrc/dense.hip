@@ -3235,7 +3235,7 @@ SkPlan plan_fwd_gemm(int f, int bk, int M, int K, int N, int share = 1) {
     // Stage sums also in a pair launch (twice the shares of a single one) and
     // in the 32-row tiles that took the place of 64-row ones or of the fp32
     // MFMA, whose shares were shorter or rounded less: FP8 1024^2 b512 9.7e-8
-    // from 64 bits on 64 x 256 tiles, 1.6e-7 on these without sums, 7.4e-8
+    // from 64 bits on 64 x 256 tiles, 1.6e-7 on these without sums, 6.2e-8
     // with; Float16 4096^2 b64 fp32 MFMA 2.9e-7, 3.2e-7 / 8.4e-8; 1% of the
     // time.  BFloat16 and Int4 stay below the fp32 MFMA's without them.
     const bool took_over = bk != BK_B16 && bk != BK_I4 && M > (bk < BK_B16 ? 32 : 16);

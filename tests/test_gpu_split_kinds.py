@@ -80,14 +80,15 @@ def test_split_kinds_nonfinite(oracle, dtype, batch, out):
     assert np.allclose(pre[ok], ref[ok], rtol=1e-5, atol=1e-4)
 
 
-def test_noalloc_keeps_the_batches_it_took(oracle):
+@pytest.mark.parametrize("inn", [64, 128])
+def test_noalloc_keeps_the_batches_it_took(oracle, inn):
     """A batch whose split-x plan needs more partial tiles than the fixed
-    64 MiB takes the fp32 MFMA plan there (Float32 64 -> 4096 b3584: 80 against
-    64 MiB)."""
+    64 MiB takes the fp32 MFMA plan there (Float32 128 -> 4096 b3584: 80
+    against 64 MiB; one k stage, on 32-row tiles, fits)."""
     from test_zz_no_alloc import run
     rng = np.random.default_rng(9)
-    W = rng.normal(0, 0.1, (4096, 64)).astype(np.float32)
-    x = rng.normal(0, 1, (3584, 64)).astype(np.float32)
+    W = rng.normal(0, 0.1, (4096, inn)).astype(np.float32)
+    x = rng.normal(0, 1, (3584, inn)).astype(np.float32)
     with pywelvet.Session(W, batch=1, act=-1, dtype=1) as s:
         got, _ = run(s, 3584, x, True)
     ref = x.astype(np.float64) @ W.astype(np.float64).T

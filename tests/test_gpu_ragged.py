@@ -137,3 +137,20 @@ def test_ragged_dx_few(oracle, dtype, out, inn, batch):
     (16 rows and 65536 outputs, 1024 outputs)."""
     if inn % chunk(dtype):
         check(oracle, dtype, out, inn, batch)
+
+
+@pytest.mark.parametrize("batch", [5, 6, 7, 8])
+def test_ragged_swiglu_halves(batch):
+    """SwiGLU's Up projection reads h and overwrites it: a row in both halves of
+    an odd batch is stored once.  g and u are f64 sums rounded once, so h is
+    within a few f32 roundings of silu(g) u."""
+    rng = np.random.default_rng(batch)
+    G, U = (rng.normal(0, 0.02, (37, 3075)).astype(np.float32) for _ in range(2))
+    D = rng.normal(0, 0.2, (3075, 37)).astype(np.float32)
+    x = rng.normal(0, 1, (batch, 3075)).astype(np.float32)
+    xd = x.astype(np.float64)
+    g, u = xd @ G.astype(np.float64).T, xd @ U.astype(np.float64).T
+    ref = g / (1 + np.exp(-g)) * u
+    for _ in range(5):
+        h, _ = pywelvet.swiglu_forward(G, U, D, x, dtype=1)
+        assert np.all(np.abs(h - ref) <= 1e-6 * (np.abs(ref) + np.abs(u) + np.abs(g)) + 1e-30)

@@ -156,7 +156,9 @@ __global__ void __launch_bounds__(256) ragged_gemv_kernel(RaggedArgs a, int S, c
     const int r = tid / B, b = tid % B, o = blockIdx.x * (4 / S) + r;
     double t = 0.0;
     for (int i = 0; i < S; ++i) t += red[r * S + i][b];
-    if (o < a.N) bias_act_store(t, o, bias, bias_len, act, pre, post, (int64_t)(m0 + b) * a.N + o);
+    // a row that both halves hold is the first one's: the epilogue may read
+    // what it overwrites (kSwiGated)
+    if (o < a.N && (blockIdx.y == 0 || m0 + b >= B)) bias_act_store(t, o, bias, bias_len, act, pre, post, (int64_t)(m0 + b) * a.N + o);
   }
 }
 

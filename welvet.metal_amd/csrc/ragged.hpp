@@ -6,8 +6,9 @@
 // A chunk of E codes may start at any bit of the packed body: a lane loads
 // the dwords that cover it (one more than a chunk has) and shifts them into
 // the aligned chunk the other kernels' decode takes.  Products and sums are
-// f64 (each f32 operand widened): on the VALU for one row of x and for up to
-// four where the weights are few, else on the f64 MFMA.
+// f64 (each f32 operand widened): on the VALU for one row of x, for up to four
+// where the weights are few (eight where rows are also long) and for dX of few
+// rows or outputs, else on the f64 MFMA.
 //
 // What bounds them: short rows, the launch and one load-compute-reduce chain
 // (4-6 us); large ones, the f64 matrix rate (half of fp32's) and the chunk
@@ -158,7 +159,8 @@ __global__ void __launch_bounds__(256) ragged_gemv_kernel(RaggedArgs a, int S, c
     for (int i = 0; i < S; ++i) t += red[r * S + i][b];
     // a row that both halves hold is the first one's: the epilogue may read
     // what it overwrites (kSwiGated)
-    if (o < a.N && (blockIdx.y == 0 || m0 + b >= B)) bias_act_store(t, o, bias, bias_len, act, pre, post, (int64_t)(m0 + b) * a.N + o);
+    if (o < a.N && (blockIdx.y == 0 || m0 + b >= B))
+      bias_act_store(t, o, bias, bias_len, act, pre, post, (int64_t)(m0 + b) * a.N + o);
   }
 }
 
